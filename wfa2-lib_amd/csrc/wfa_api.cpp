@@ -191,6 +191,8 @@ Engine::~Engine() {
     if (ev) (void)hipEventDestroy(ev);
   if (plain.exec) (void)hipGraphExecDestroy(plain.exec);
   if (plain.graph) (void)hipGraphDestroy(plain.graph);
+  for (auto& ev : tile.ev)
+    if (ev) (void)hipEventDestroy(ev);
 }
 
 Engine* engine_of(wavefront_aligner_t* wf) { return static_cast<Engine*>(wf->device); }
@@ -919,14 +921,22 @@ std::vector<PlanGroup> make_plan(const JobSet& js, const std::vector<int>& ids, 
   const bool heur_ok = js.heur.cut() <= 1;
   const bool lean_ok = lt.enabled && ncomp == 3 && js.bits == 2 && !js.cbeg && !js.cend && ef_fits && heur_ok &&
                        wfa::lean_supported(pen);
-  std::vector<int> lean_ids[2];
+  std::vector<int> lean_ids[2], tile_ids;
   int lean_lmax[2] = {0, 0};
+  // Pairs above 1,024 bases in tiles, where the kernels have an instance: on
+  // any number of pairs the device is filled by tiles, not by pairs.
+  const bool tile_ok = js.tiles && js.bits == 2 && !js.cbeg && !js.cend && !js.ef.on && js.heur.cut() == 0 &&
+                       wfa::tile_shape(pen) != 0;
   for (int i : ids) {
     const int L = std::max(js.h_plen[i], js.h_tlen[i]);
     if (lean_ok && L <= kLeanMaxLen) {
       const int c = L <= lt.short_len ? 0 : 1;
       lean_ids[c].push_back(i);
       lean_lmax[c] = std::max<int>(lean_lmax[c], L / spw + 3);
+      continue;
+    }
+    if (tile_ok && L > kLeanMaxLen && tile_fits(js.h_plen[i], js.h_tlen[i])) {
+      tile_ids.push_back(i);
       continue;
     }
     if (wcap_small >= 64 && L <= 1024) {
@@ -958,6 +968,12 @@ std::vector<PlanGroup> make_plan(const JobSet& js, const std::vector<int>& ids, 
     g.ids = std::move(small_ids);
     plan.push_back(std::move(g));
   }
+  if (!tile_ids.empty()) {
+    PlanGroup g;
+    g.family = wfa::kTile;
+    g.ids = std::move(tile_ids);
+    plan.push_back(std::move(g));
+  }
   for (auto& c : cls)
     if (!c.empty()) plan.push_back(make_large(nullptr, js, std::move(c)));
   return plan;
@@ -979,13 +995,16 @@ int run_jobs(wavefront_aligner_t* wf, Engine* e, const JobSet& js, std::vector<P
     double want = 0;
     for (PlanGroup& g : plan) {
       if (g.est_rec_bytes < 0) {
-        const double per_l2 = g.family == wfa::kLarge ? 1.0 / kLargeRecordShareOfL2 : 1.0 / 16;
+        const bool large = g.family == wfa::kLarge || g.family == wfa::kTile;
+        const double per_l2 = large ? kLargeRecordShareOfL2 : 1.0 / 16;
         double w = 0;
         for (int i : g.ids) {
           const double L = std::max(js.h_plen[i], js.h_tlen[i]);
           w += L * L * per_l2 + 8 * L;
         }
-        g.est_rec_bytes = w + (double)shape_of(e, g, js.bits, pen, js.heur.cut()).grid * wfa::kChunkUnits * 16;
+        g.est_rec_bytes = w;
+        if (g.family != wfa::kTile)  // and the record chunk of every workgroup
+          g.est_rec_bytes += (double)shape_of(e, g, js.bits, pen, js.heur.cut()).grid * wfa::kChunkUnits * 16;
       }
       want += g.est_rec_bytes;
     }
@@ -1005,7 +1024,8 @@ int run_jobs(wavefront_aligner_t* wf, Engine* e, const JobSet& js, std::vector<P
     if (round > 0 && !hip_ok(wfa::launch_reset_counters(counters_of(e), 1, st), "reset")) return WF_STATUS_OOM;
     bool fresh = true;
     for (PlanGroup& g : *pending) {
-      const int rc = enqueue_group(wf, e, js, g, pen, records, fresh);
+      const int rc = g.family == wfa::kTile ? run_tile_group(e, js, g, pen, records, tot)
+                                            : enqueue_group(wf, e, js, g, pen, records, fresh);
       if (rc != WF_STATUS_OK) return rc;
       if (!g.ids.empty()) fresh = false;
       ++tot->launches;
@@ -1163,6 +1183,7 @@ wfa_host::JobSet wfa_device_batch_t::jobs() const {
   js.end_rec = d_end_rec.as<int>();
   js.ef = ef;
   js.heur = heur;
+  js.tiles = tiles;
   return js;
 }
 
@@ -1597,6 +1618,11 @@ int run_trials(wavefront_aligner_t* wf, Engine* e, const JobSet& js, int records
 
 namespace {
 
+// Whether the aligner has no step limit (the default attributes' INT_MAX).
+bool unlimited_steps(const wavefront_aligner_t* wf) {
+  return wf->system.max_alignment_steps <= 0 || wf->system.max_alignment_steps == INT_MAX;
+}
+
 // Final per-pair statuses of a run with failures: internal codes the host
 // reports differently, and the first failing status.
 int settle_statuses(wavefront_aligner_t* wf, std::vector<int>& status) {
@@ -1631,6 +1657,7 @@ int batch_run(wavefront_aligner_t* wf, wfa_device_batch_t* b, Engine* e) {
   b->records = records;
   b->ef = ends_free_of(wf);
   b->heur = heuristic_of(wf);
+  b->tiles = !e->na && unlimited_steps(wf);
   b->stats = wfa_run_stats_t{};
   b->have_results = false;
   b->host_results = false;
@@ -1663,7 +1690,7 @@ int batch_run(wavefront_aligner_t* wf, wfa_device_batch_t* b, Engine* e) {
     if (rc != WF_STATUS_OK) return rc;
   } else {
     const std::vector<int> key = {pen.metric, pen.x, pen.o1, pen.e1, pen.o2, pen.e2, b->bits, b->ef.on,
-                                  b->heur.cut(), records};
+                                  b->heur.cut(), records, b->tiles};
     if (b->plan_key != key) {
       std::vector<PlanGroup> plan = make_plan(b->jobs(), b->sorted, pen);
       std::vector<TuneTrial> trials;
@@ -1957,6 +1984,7 @@ int plain_run(wavefront_aligner_t* wf, Engine* e, wfa_device_batch_t* b, const w
   b->heur = heuristic_of(wf);
   b->stats = wfa_run_stats_t{};
   b->bi_mode = false;
+  b->tiles = unlimited_steps(wf);
   b->first_fail = WF_STATUS_ALG_COMPLETED;
   hipStream_t st = e->stream;
   const JobSet js = b->jobs();
@@ -1966,7 +1994,7 @@ int plain_run(wavefront_aligner_t* wf, Engine* e, wfa_device_batch_t* b, const w
     return hip_ok(hipMemcpyAsync(b->words.p, b->h_words.p, upload, hipMemcpyHostToDevice, st), "upload")
                ? 1 : WF_STATUS_OOM;
   };
-  if (plan.size() != 1) return general();
+  if (plan.size() != 1 || plan[0].family == wfa::kTile) return general();
   PlanGroup& g = plan[0];
   if (g.family != wfa::kLarge) g.lmax_words = (int)(upload / 8);  // the bucket's words: a capacity, not a length
   if (!reserve_for(e, plan, js.bits, pen, js.heur.cut(), records)) return WF_STATUS_OOM;

@@ -170,8 +170,9 @@ struct BacktraceArgs {
 // Kernel families.  kSmall: one 64-lane wavefront per pair, wavefront ring
 // and both sequences in LDS.  kLarge: one workgroup per pair, ring in HBM.
 // kLean: like kSmall, gap-affine with 2-bit sequences, specialised on the
-// penalties' slot structure (wfa_lean.hip).
-enum Family : int { kSmall = 0, kLarge = 1, kLean = 2 };
+// penalties' slot structure (wfa_lean.hip).  kTile: long pairs in tiles of
+// diagonals, a block of steps per launch (wfa_tile.hip).
+enum Family : int { kSmall = 0, kLarge = 1, kLean = 2, kTile = 3 };
 
 struct LaunchShape {
   int family = 0;

@@ -9,6 +9,7 @@
 
 #include "wfa_device.h"
 #include "wfa_mi355x.h"
+#include "wfa_tile.h"
 
 namespace wfa_host {
 
@@ -140,6 +141,17 @@ struct Engine {
     DevBuf mail, hand;  // paired-workgroup searches: mailboxes and handover records
     hipEvent_t ev[2] = {nullptr, nullptr};
   } bi;
+  // Long pairs in tiles (wfa_tile_run.cpp): the range table of the penalties
+  // last used and the grow-only buffers of a run.
+  struct TileState {
+    int shape = 0;
+    std::vector<int> lo, hi;          // hull of the ranges up to each step
+    std::vector<int> m_range;         // untrimmed range of M at each step (lo, hi)
+    std::vector<long long> dsteps;
+    DevBuf d_range, d_dsteps, d_job_range, d_dev, d_ends, d_flags, d_dsum, d_step_state, d_step_off, d_step0, d_step_act, d_off, d_pitch, d_jobs, d_marks, d_act, d_info, d_tab;
+    HostBuf h_n;                      // jobs left, written by the device
+    hipEvent_t ev[5] = {nullptr, nullptr, nullptr, nullptr, nullptr};
+  } tile;
   // Set for the duration of a no-allocation run: plan groups take their
   // order arrays from `order`, and the HBM-ring family's grid is limited so
   // that its rings fit in ring_bytes (the engine's rec/ring/counters buffers
@@ -219,6 +231,7 @@ struct JobSet {
   int* end_rec = nullptr;      // z-drop: record byte of the end cell (0xFF: no source)
   EndsFree ef;
   wfa::HeurArgs heur{};        // wf-adaptive (none for BiWFA base jobs)
+  bool tiles = false;          // long jobs may run in tiles (no step limit, buffers may grow)
 };
 
 // The aligner's wf-adaptive parameters (none unless the strategy is wf-adaptive).
@@ -239,6 +252,12 @@ std::vector<PlanGroup> make_plan(const JobSet& js, const std::vector<int>& ids, 
 // for the host copy of the statuses.  Returns WF_STATUS_OK or WF_STATUS_OOM.
 int run_jobs(wavefront_aligner_t* wf, Engine* e, const JobSet& js, std::vector<PlanGroup>& plan,
              int records, RunTotals* tot, std::vector<int>& h_status);
+
+// Long pairs in tiles (wfa_tile_run.cpp).
+bool tile_table(Engine* e, int shape, int steps);
+bool tile_fits(int plen, int tlen);
+int run_tile_group(Engine* e, const JobSet& js, const PlanGroup& grp, const wfa::Penalties& pen, int records,
+                   RunTotals* tot);
 
 }  // namespace wfa_host
 
@@ -268,6 +287,7 @@ struct wfa_device_batch_t {
   std::vector<int> status, score, ops_begin, end_k, end_off;
   wfa_host::EndsFree ef;                   // form of the last run
   wfa::HeurArgs heur{};                    // heuristic of the last run
+  bool tiles = false;                      // whether the last run could take long pairs in tiles
   bool have_results = false;
   bool host_results = false;
   bool ops_on_device = false;

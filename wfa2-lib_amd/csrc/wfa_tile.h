@@ -1,0 +1,158 @@
+// Interface of the tile kernels (wfa_tile.hip): long pairs advanced a block
+// of score steps per launch, in tiles of diagonals.  Steps are counted in
+// slots: step i is score (i + 1) * g, and score 0 is step -1.
+#pragma once
+#include "wfa_device.h"
+
+namespace wfa {
+
+// State diagonals below the pattern's and above the text's length: a tile
+// reads its halo there, and the last tile reaches past the last diagonal.
+constexpr int kTilePadLow = 128, kTilePadHigh = 768;
+// Index of diagonal 0 in a job's state rows (a multiple of 4).
+__host__ __device__ inline int tile_kpad(int plen) { return (plen + kTilePadLow + 3) / 4 * 4; }
+__host__ __device__ inline int tile_pitch(int plen, int tlen) { return tile_kpad(plen) + (tlen + kTilePadHigh + 3) / 4 * 4; }
+
+// LDS for the two sequences of a job (2-bit sequences up to 130 kbp).
+constexpr size_t kTileSeqLdsBytes = 64 * 1024;
+
+struct TileBlockInfo {  // records of one block: first diagonal and bytes per step
+  int kb, pitch;
+};
+
+// The diagonals of a job in one block: rows written over [left, right), and
+// the lowest and highest diagonal a wavefront of the block reached.
+struct TileRange {
+  int left, right, min_lo, max_hi;
+};
+
+struct TileArgs {
+  const int* act;              // active jobs
+  const int* n_act;
+  const int* plen;
+  const int* tlen;
+  const uint64_t* words;
+  const int64_t* pat_pos;
+  const int64_t* txt_pos;
+  int* state;                  // rows of every job
+  const int64_t* st_off;       // first int of a job's state
+  const int* st_pitch;         // ints per row
+  int* done;                   // step at which the job reached its end (INT_MAX: not yet)
+  int* irr;                    // first step whose end left its tile (INT_MAX: none)
+  TileRange* range;            // per job, of the last four blocks
+  const int2* m_range;         // per step, the untrimmed range of M (lo > hi: none)
+  int* exact_lo;               // 1 + the block in which the job's low / high end was first
+  int* exact_hi;               // trimmed, or 0
+  long long* dev[2][2];        // by block parity and end: the limits minus the tabulated ones, summed
+                               // up to each step of the block (steps-per-block entries per job)
+  const long long* dsteps_upto;  // untrimmed diagonal-steps up to and including step i at [i + 1]
+  int* stepped;                // whether the job changed over to one step per launch
+  uint4* rec;                  // record arena
+  uint32_t* rec_tab;           // per job and block: first unit of its records
+  int tab_stride;
+  uint32_t rec_unit0;          // this block's records: job y at rec_unit0 + y * rec_job_units
+  uint32_t rec_job_units;
+  int rec_kb;                  // first diagonal of the records
+  int rec_pitch;               // bytes per step
+  int blk;
+  int tiles;                   // at most
+  int lmax_words;              // LDS words per sequence
+};
+
+constexpr int kTileStepEnds = 12, kTileStepFlags = 32;
+
+// Jobs whose ends jump, one step per launch (tile_step_kernel).
+struct StepArgs {
+  const int* act;
+  const int* n_act;
+  const int* plen;
+  const int* tlen;
+  const uint64_t* words;
+  const int64_t* pat_pos;
+  const int64_t* txt_pos;
+  int* state;
+  const int64_t* st_off;       // first int of a job's rows
+  const int* st_pitch;
+  int* done;
+  int* ends;                   // per job, ring of 4 steps: kTileStepEnds ends of the components
+  int* flags;                  // per job, ring of kTileStepFlags steps: which components have a valid cell
+  long long* dsum;             // diagonal-steps before the latest step
+  int* step0;                  // the job's first step
+  uint4* rec;
+  uint32_t* rec_tab;
+  int tab_stride;
+  uint32_t rec_unit0;          // this block's records: job y at rec_unit0 + y * rec_job_units
+  uint32_t rec_job_units;
+  const TileBlockInfo* blocks;
+};
+
+struct TileFinishArgs {
+  int n;
+  const int* jobs;             // null: 0..n-1
+  const int* plen;
+  const int* tlen;
+  const int* done;
+  const int* irr;
+  const long long* dsteps_upto;
+  const int* exact_lo;
+  const int* exact_hi;
+  const long long* dev[2][2];
+  const int* stepped;
+  const int* step_ends;        // StepArgs::ends
+  const int* flags;
+  const long long* dsum;
+  int steps;                   // per block
+  int g;
+  int* out_status;
+  int* out_score;
+  long long* out_dsteps;
+  uint32_t* out_last_block;
+  int* out_end_k;
+  int* out_end_off;
+  unsigned long long* dsteps_total;
+  unsigned int* retry_count;
+};
+
+struct TileTraceArgs {
+  const int* jobs;
+  const int* plen;
+  const int* tlen;
+  int* status;
+  const int* score;
+  const uint4* rec;
+  const uint32_t* rec_tab;
+  int tab_stride;
+  const TileBlockInfo* blocks;
+  const uint64_t* words;
+  const int64_t* pat_pos;
+  const int64_t* txt_pos;
+  char* ops;
+  const int64_t* ops_off;
+  int* ops_begin;
+  unsigned int* fail_count;
+  int g;
+  int lmax_words;
+};
+
+struct TileGeometry {
+  int steps;                   // per block
+  int useful;                  // diagonals per tile
+  int state_rows;
+  int step_rows;               // of the step kernels
+  int dx, do1, de1, do2, de2;  // distances in steps (do2 = 0: no second gap)
+};
+
+// 0: no instance for these penalties.
+int tile_shape(const Penalties& pen);
+TileGeometry tile_geometry(int shape);
+hipError_t launch_tile_fill(int* state, long long ints, hipStream_t st);
+hipError_t launch_tile_init(int shape, const TileArgs& a, int n, const int* jobs, int* act, int* n_act, hipStream_t st);
+hipError_t launch_tile_block(int shape, bool records, const TileArgs& a, int jobs, hipStream_t st);
+hipError_t launch_tile_step_init(int shape, const StepArgs& a, const TileArgs& t, int n, int max_pitch, hipStream_t st);
+hipError_t launch_tile_step(int shape, bool records, const StepArgs& a, int t, int jobs, int max_width, hipStream_t st);
+hipError_t launch_tile_compact(const int* act, const int* n_act, const int* done, const int* irr, int ib, int* act2,
+                               int* n_act2, int* host_n, hipStream_t st);
+hipError_t launch_tile_finish(int shape, const TileFinishArgs& a, hipStream_t st);
+hipError_t launch_tile_backtrace(int shape, const TileTraceArgs& a, int n, hipStream_t st);
+
+}  // namespace wfa

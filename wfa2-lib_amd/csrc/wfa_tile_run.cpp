@@ -1,0 +1,419 @@
+// Host side of the tile kernels (wfa_tile.hip): the table of wavefront
+// ranges, and the loop that advances a set of long pairs block by block.
+#include <algorithm>
+#include <climits>
+#include <cstdio>
+#include <cstring>
+
+#include "wfa_internal.h"
+
+namespace wfa_host {
+namespace {
+
+// State rows of the jobs that run at once.
+constexpr size_t kTileStateBytes = size_t(24) << 30;
+constexpr int kTileMaxJobs = 32768;  // grid y
+// Records a long pair is planned with: 1-20 kbp pairs of 1-15% error write
+// 0.25 L^2 bytes on average and up to 0.7 L^2.
+constexpr double kTileRecordShareOfL2 = 0.5;
+// Blocks between two looks at the number of jobs left.
+constexpr int kTileFirstChunk = 4, kTileChunk = 16;
+
+struct Range {
+  int lo = 1, hi = -1;
+  bool valid() const { return lo <= hi; }
+};
+
+}  // namespace
+
+// The ranges of every step from 0 to at least `steps`, which are the same for
+// all pairs until an end cell leaves the matrix
+// (wavefront_compute_limits_input, wavefront_compute.c:40-86, with every
+// range as wide as its sources make it).  Returns false on an allocation or
+// copy failure.
+bool tile_table(Engine* e, int shape, int steps) {
+  Engine::TileState& t = e->tile;
+  if (t.shape == shape && (int)t.lo.size() >= steps) return true;
+  const wfa::TileGeometry g = wfa::tile_geometry(shape);
+  steps = std::max(steps, 4096);
+  if (t.shape == shape) steps = std::max(steps, 2 * (int)t.lo.size());
+  t.shape = shape;
+  t.lo.assign(steps, 0);
+  t.hi.assign(steps, 0);
+  t.m_range.assign(2 * (size_t)steps, 0);
+  t.dsteps.assign((size_t)steps + 1, 0);
+  const bool two = g.do2 > 0;
+  // row r at index r + 1 (row -1: score 0, M = [0, 0])
+  std::vector<Range> M(steps + 1), I1(steps + 1), D1(steps + 1), I2(steps + 1), D2(steps + 1);
+  M[0] = Range{0, 0};
+  int hull_lo = 0, hull_hi = 0;
+  for (int i = 0; i < steps; ++i) {
+    auto at = [&](const std::vector<Range>& v, int back) {
+      const int r = i + 1 - back;
+      return r >= 0 ? v[r] : Range{};
+    };
+    const Range mx = at(M, g.dx), mo = at(M, g.do1), i1 = at(I1, g.de1), d1 = at(D1, g.de1);
+    const Range mo2 = two ? at(M, g.do2) : Range{}, i2 = two ? at(I2, g.de2) : Range{},
+                d2 = two ? at(D2, g.de2) : Range{};
+    Range m;
+    auto add = [](Range& r, const Range& s, int d) {
+      if (!s.valid()) return;
+      if (!r.valid()) { r = Range{s.lo + d, s.hi + d}; return; }
+      r.lo = std::min(r.lo, s.lo + d);
+      r.hi = std::max(r.hi, s.hi + d);
+    };
+    add(I1[i + 1], mo, 1); add(I1[i + 1], i1, 1);
+    add(D1[i + 1], mo, -1); add(D1[i + 1], d1, -1);
+    add(I2[i + 1], mo2, 1); add(I2[i + 1], i2, 1);
+    add(D2[i + 1], mo2, -1); add(D2[i + 1], d2, -1);
+    // limits: each source contributes its range shifted as its gap moves it;
+    // an opening contributes both ways
+    add(m, mx, 0); add(m, I1[i + 1], 0); add(m, D1[i + 1], 0); add(m, I2[i + 1], 0); add(m, D2[i + 1], 0);
+    M[i + 1] = m;
+    t.dsteps[i + 1] = t.dsteps[i] + (m.valid() ? m.hi - m.lo + 1 : 0);
+    if (m.valid()) {
+      hull_lo = std::min(hull_lo, m.lo);
+      hull_hi = std::max(hull_hi, m.hi);
+    }
+    t.lo[i] = hull_lo;
+    t.hi[i] = hull_hi;
+    t.m_range[2 * (size_t)i] = m.lo;
+    t.m_range[2 * (size_t)i + 1] = m.hi;
+  }
+  hipStream_t st = e->stream;
+  return t.d_range.ensure(t.m_range.size() * sizeof(int)) && t.d_dsteps.ensure(t.dsteps.size() * sizeof(long long)) &&
+         hip_ok(hipMemcpyAsync(t.d_range.p, t.m_range.data(), t.m_range.size() * sizeof(int), hipMemcpyHostToDevice, st),
+                "tile table") &&
+         hip_ok(hipMemcpyAsync(t.d_dsteps.p, t.dsteps.data(), t.dsteps.size() * sizeof(long long),
+                               hipMemcpyHostToDevice, st), "tile table") &&
+         hip_ok(hipStreamSynchronize(st), "tile table");
+}
+
+// Whether a job of these lengths can run in tiles: its sequences in LDS.
+bool tile_fits(int plen, int tlen) {
+  const int lw = std::max(plen, tlen) / 32 + 3;
+  return 2 * (size_t)lw * sizeof(uint64_t) <= wfa::kTileSeqLdsBytes;
+}
+
+// The jobs whose ends moved past their end tiles, one step per launch from
+// the start of the block that found it, all of them side by side.  `unit`:
+// record units taken so far.  Jobs left when the records run out stay
+// unfinished (they are re-run with the records free again).
+int run_steps(Engine* e, const JobSet& js, int shape, const wfa::TileGeometry& g, const wfa::TileArgs& a,
+              const int* ids, int n_pass, const std::vector<wfa::TileBlockInfo>& info, int records,
+              uint64_t rec_units, uint64_t* unit) {
+  Engine::TileState& t = e->tile;
+  hipStream_t st = e->stream;
+  const int T = g.steps;
+  std::vector<int> marks(2 * (size_t)js.n);
+  if (!hip_ok(hipMemcpyAsync(marks.data(), a.done, marks.size() * 4, hipMemcpyDeviceToHost, st), "tile marks") ||
+      !hip_ok(hipStreamSynchronize(st), "tile marks"))
+    return WF_STATUS_OOM;
+  const int* done = marks.data();
+  const int* irr = done + js.n;
+  std::vector<int> jobs;
+  for (int x = 0; x < n_pass; ++x)
+    if (irr[ids[x]] != INT_MAX && irr[ids[x]] < done[ids[x]]) jobs.push_back(ids[x]);
+  const bool ok = t.d_ends.ensure((size_t)js.n * 4 * wfa::kTileStepEnds * 4) &&
+                  t.d_flags.ensure((size_t)js.n * wfa::kTileStepFlags * 4) && t.d_dsum.ensure((size_t)js.n * 8);
+  if (!ok) return WF_STATUS_OOM;
+  // as many at once as their rows' memory allows
+  for (size_t first = 0; first < jobs.size();) {
+    std::vector<int64_t> off(js.n, 0);
+    int64_t ints = 0;
+    int n = 0, max_pitch = 0, max_width = 0;
+    while (first + n < jobs.size()) {
+      const int i = jobs[first + n], pitch = wfa::tile_pitch(js.h_plen[i], js.h_tlen[i]);
+      const int64_t need = (int64_t)pitch * g.step_rows;
+      if (n > 0 && (size_t)(ints + need) * 4 > kTileStateBytes) break;
+      off[i] = ints;
+      ints += need;
+      max_pitch = std::max(max_pitch, pitch);
+      max_width = std::max(max_width, js.h_plen[i] + js.h_tlen[i] + 4);
+      ++n;
+    }
+    const int* sel = jobs.data() + first;
+    if (!t.d_step_state.ensure((size_t)ints * 4) || !t.d_step_off.ensure((size_t)js.n * 8) ||
+        !t.d_step0.ensure((size_t)js.n * 4) || !t.d_step_act.ensure((size_t)2 * n * 4 + 64)) {
+      fprintf(stderr, "[WFA] cannot allocate %zu MB of wavefront rows\n", (size_t)ints >> 18);
+      return WF_STATUS_OOM;
+    }
+    int* n_act = t.d_step_act.as<int>();
+    int* act[2] = {n_act + 16, n_act + 16 + n};
+    wfa::StepArgs s{};
+    s.act = act[0];
+    s.n_act = n_act;
+    s.plen = js.plen;
+    s.tlen = js.tlen;
+    s.words = js.words;
+    s.pat_pos = js.ppos;
+    s.txt_pos = js.tpos;
+    s.state = t.d_step_state.as<int>();
+    s.st_off = t.d_step_off.as<int64_t>();
+    s.st_pitch = a.st_pitch;
+    s.done = a.done;
+    s.ends = t.d_ends.as<int>();
+    s.flags = t.d_flags.as<int>();
+    s.dsum = t.d_dsum.as<long long>();
+    s.step0 = t.d_step0.as<int>();
+    s.rec = a.rec;
+    s.rec_tab = a.rec_tab;
+    s.tab_stride = a.tab_stride;
+    s.blocks = t.d_info.as<wfa::TileBlockInfo>();
+    volatile int* h_n = t.h_n.as<int>() + 8;
+    if (!hip_ok(hipMemcpyAsync(t.d_step_off.p, off.data(), (size_t)js.n * 8, hipMemcpyHostToDevice, st), "steps") ||
+        !hip_ok(hipMemcpyAsync(act[0], sel, (size_t)n * 4, hipMemcpyHostToDevice, st), "steps") ||
+        !hip_ok(hipMemcpyAsync(n_act, &n, 4, hipMemcpyHostToDevice, st), "steps") ||
+        !hip_ok(wfa::launch_tile_step_init(shape, s, a, n, max_pitch, st), "step init"))
+      return WF_STATUS_OOM;
+    // blocks of T steps, every job at the same place of its block
+    int known = n, which = 0;
+    for (int b = 0; known > 0; ++b) {
+      uint32_t units = 0;
+      bool any = false;
+      for (int x = 0; x < n; ++x) {
+        const size_t blk = (size_t)irr[sel[x]] / T + b;
+        if (blk >= info.size()) continue;
+        any = true;
+        units = std::max(units, (uint32_t)((size_t)T * info[blk].pitch / 16));
+      }
+      if (!any) break;
+      if (records && *unit + (uint64_t)known * units > rec_units) break;
+      s.act = act[which];
+      s.n_act = n_act + which;
+      s.rec_unit0 = (uint32_t)*unit;
+      s.rec_job_units = units;
+      if (records) *unit += (uint64_t)known * units;
+      for (int x = 0; x < T; ++x)
+        if (!hip_ok(wfa::launch_tile_step(shape, records != 0, s, b * T + x, known, max_width, st), "step launch"))
+          return WF_STATUS_OOM;
+      const int slot = b & 1;
+      if (!hip_ok(wfa::launch_tile_compact(act[which], n_act + which, a.done, nullptr, INT_MAX, act[which ^ 1],
+                                           n_act + (which ^ 1), const_cast<int*>(h_n) + slot, st), "tile compact") ||
+          !hip_ok(hipEventRecord(t.ev[3 + slot], st), "tile event"))
+        return WF_STATUS_OOM;
+      which ^= 1;
+      if (b > 0) {
+        if (!hip_ok(hipEventSynchronize(t.ev[3 + (slot ^ 1)]), "steps")) return WF_STATUS_OOM;
+        known = h_n[slot ^ 1];
+      }
+    }
+    if (!hip_ok(hipStreamSynchronize(st), "steps")) return WF_STATUS_OOM;
+    first += n;
+  }
+  return WF_STATUS_OK;
+}
+
+// Aligns the jobs of a tile group; statuses, scores and CIGARs stay on the
+// device, and jobs to be re-run are counted in the run counters.
+int run_tile_group(Engine* e, const JobSet& js, const PlanGroup& grp, const wfa::Penalties& pen, int records,
+                   RunTotals* tot) {
+  Engine::TileState& t = e->tile;
+  const int shape = wfa::tile_shape(pen);
+  const wfa::TileGeometry g = wfa::tile_geometry(shape);
+  hipStream_t st = e->stream;
+  wfa::Counters* c = counters_of(e);
+  const int T = g.steps;
+  // no alignment costs more than deleting and inserting everything, or than
+  // mismatches along the shorter sequence
+  int max_steps = 0;
+  for (int i : grp.ids) {
+    const int64_t mn = std::min(js.h_plen[i], js.h_tlen[i]), mx = std::max(js.h_plen[i], js.h_tlen[i]);
+    max_steps = (int)std::max<int64_t>(max_steps, mn * g.dx + g.do1 + (mx - mn) * g.de1);
+  }
+  const int max_blocks = max_steps / T + 2;
+  if (!tile_table(e, shape, (max_blocks + 1) * T)) return WF_STATUS_OOM;
+  for (auto& ev : t.ev)
+    if (!ev && !hip_ok(hipEventCreate(&ev), "hipEventCreate")) return WF_STATUS_OOM;
+  if (!t.h_n.ensure(4096)) return WF_STATUS_OOM;
+  volatile int* h_n = t.h_n.as<int>();
+  // per block the tiles a job has at most, and its records' first diagonal
+  // and bytes per step (no range goes beyond the longest sequences)
+  int pmax = 0, tmax = 0;
+  for (int i : grp.ids) { pmax = std::max(pmax, js.h_plen[i]); tmax = std::max(tmax, js.h_tlen[i]); }
+  std::vector<wfa::TileBlockInfo> info(max_blocks);
+  std::vector<int> tiles(max_blocks);
+  for (int b = 0; b < max_blocks; ++b) {
+    const int lo = std::max(t.lo[(size_t)(b + 1) * T - 1], -pmax - 1), hi = std::min(t.hi[(size_t)(b + 1) * T - 1], tmax + 1);
+    const int kb = -((-lo + 15) / 16 * 16);
+    info[b] = wfa::TileBlockInfo{kb, (hi - kb + 16) / 16 * 16};
+    const int lo0 = b ? std::max(t.lo[(size_t)b * T - 1], -pmax - 1) : 0, hi0 = b ? std::min(t.hi[(size_t)b * T - 1], tmax + 1) : 0;
+    tiles[b] = (hi0 - lo0 + 1 + 2 * T + 8) / g.useful + 1;
+  }
+  const int n_all = (int)grp.ids.size();
+  std::vector<int64_t> st_off(js.n, 0);
+  std::vector<int> st_pitch(js.n, 0);
+  if (!t.d_off.ensure((size_t)js.n * 8) || !t.d_pitch.ensure((size_t)js.n * 4) || !t.d_jobs.ensure((size_t)n_all * 4) ||
+      !t.d_marks.ensure((size_t)js.n * 5 * 4) ||
+      !t.d_job_range.ensure((size_t)js.n * 4 * sizeof(wfa::TileRange)) || !t.d_dev.ensure((size_t)js.n * 4 * T * 8) || !t.d_act.ensure((size_t)2 * n_all * 4 + 64) ||
+      !t.d_info.ensure((size_t)max_blocks * sizeof(wfa::TileBlockInfo)) ||
+      (records && !t.d_tab.ensure((size_t)js.n * max_blocks * 4))) {
+    fprintf(stderr, "[WFA] cannot allocate the tile buffers of %d pairs\n", n_all);
+    return WF_STATUS_OOM;
+  }
+  if (!hip_ok(hipMemcpyAsync(t.d_info.p, info.data(), info.size() * sizeof(info[0]), hipMemcpyHostToDevice, st), "tiles"))
+    return WF_STATUS_OOM;
+  const uint64_t rec_units = records ? std::min<uint64_t>(e->rec.cap / 16, 0xFFFFFFF0ull) : 0;
+
+  for (int first = 0; first < n_all;) {
+    // the jobs of one pass: their state rows and planned records fit
+    int64_t ints = 0;
+    double rec_plan = 0;
+    int n = 0, lw = 0;
+    while (first + n < n_all && n < kTileMaxJobs) {
+      const int i = grp.ids[first + n];
+      const int pitch = wfa::tile_pitch(js.h_plen[i], js.h_tlen[i]);
+      const int64_t need = (int64_t)pitch * g.state_rows;
+      const double L = std::max(js.h_plen[i], js.h_tlen[i]);
+      if (n > 0 && ((size_t)(ints + need) * 4 > kTileStateBytes || grp.max_grid == n ||
+                    (records && rec_plan + L * L * kTileRecordShareOfL2 > (double)rec_units * 16)))
+        break;
+      st_off[i] = ints;
+      st_pitch[i] = pitch;
+      ints += need;
+      rec_plan += L * L * kTileRecordShareOfL2;
+      lw = std::max(lw, (int)L / 32 + 3);
+      ++n;
+    }
+    if (!e->ring.ensure((size_t)ints * 4)) {
+      fprintf(stderr, "[WFA] cannot allocate %zu MB of wavefront rows\n", (size_t)ints >> 18);
+      return WF_STATUS_OOM;
+    }
+    const int* ids = grp.ids.data() + first;
+    if (!hip_ok(hipMemcpyAsync(t.d_off.p, st_off.data(), (size_t)js.n * 8, hipMemcpyHostToDevice, st), "tiles") ||
+        !hip_ok(hipMemcpyAsync(t.d_pitch.p, st_pitch.data(), (size_t)js.n * 4, hipMemcpyHostToDevice, st), "tiles") ||
+        !hip_ok(hipMemcpyAsync(t.d_jobs.p, ids, (size_t)n * 4, hipMemcpyHostToDevice, st), "tiles"))
+      return WF_STATUS_OOM;
+    int* marks = t.d_marks.as<int>();
+    int* act[2] = {t.d_act.as<int>() + 16, t.d_act.as<int>() + 16 + n_all};
+    int* n_act = t.d_act.as<int>();  // counts of the two lists
+    wfa::TileArgs a{};
+    a.act = act[0];
+    a.n_act = n_act;
+    a.plen = js.plen;
+    a.tlen = js.tlen;
+    a.words = js.words;
+    a.pat_pos = js.ppos;
+    a.txt_pos = js.tpos;
+    a.state = e->ring.as<int>();
+    a.st_off = t.d_off.as<int64_t>();
+    a.st_pitch = t.d_pitch.as<int>();
+    a.done = marks;
+    a.irr = marks + js.n;
+    a.range = t.d_job_range.as<wfa::TileRange>();
+    a.m_range = t.d_range.as<int2>();
+    a.exact_lo = marks + 2 * (size_t)js.n;
+    a.exact_hi = marks + 3 * (size_t)js.n;
+    a.stepped = marks + 4 * (size_t)js.n;
+    for (int x = 0; x < 4; ++x) a.dev[x / 2][x % 2] = t.d_dev.as<long long>() + (size_t)js.n * T * x;
+    a.dsteps_upto = t.d_dsteps.as<long long>();
+    a.rec = e->rec.as<uint4>();
+    a.rec_tab = t.d_tab.as<uint32_t>();
+    a.tab_stride = max_blocks;
+    a.lmax_words = lw;
+    (void)hipEventRecord(t.ev[0], st);
+    if (!hip_ok(wfa::launch_tile_fill(a.state, ints, st), "tile fill") ||
+        !hip_ok(wfa::launch_tile_init(shape, a, n, t.d_jobs.as<int>(), act[0], n_act, st), "tile init"))
+      return WF_STATUS_OOM;
+    int known = n, which = 0, chunk = 0;
+    uint64_t unit = 0;
+    bool full = false;
+    for (int b = 0; b < max_blocks && known > 0 && !full;) {
+      const int to = std::min(max_blocks, b + (chunk < 4 ? kTileFirstChunk : kTileChunk));
+      for (; b < to; ++b) {
+        a.act = act[which];
+        a.n_act = n_act + which;
+        a.blk = b;
+        a.tiles = tiles[b];
+        a.rec_kb = info[b].kb;
+        a.rec_pitch = info[b].pitch;
+        a.rec_job_units = (uint32_t)((size_t)T * info[b].pitch / 16);
+        a.rec_unit0 = (uint32_t)unit;
+        if (records) {
+          if (unit + (uint64_t)known * a.rec_job_units > rec_units) { full = true; break; }
+          unit += (uint64_t)known * a.rec_job_units;
+        }
+        if (!hip_ok(wfa::launch_tile_block(shape, records != 0, a, known, st), "tile launch")) return WF_STATUS_OOM;
+      }
+      if (full) break;
+      // drop the finished jobs; the host looks at the count one chunk later,
+      // so that the device always has launches queued
+      const int slot = chunk & 1;
+      if (!hip_ok(wfa::launch_tile_compact(act[which], n_act + which, a.done, a.irr, b * T, act[which ^ 1],
+                                           n_act + (which ^ 1), const_cast<int*>(h_n) + slot, st), "tile compact") ||
+          !hip_ok(hipEventRecord(t.ev[3 + slot], st), "tile event"))
+        return WF_STATUS_OOM;
+      which ^= 1;
+      if (chunk > 0) {
+        if (!hip_ok(hipEventSynchronize(t.ev[3 + (slot ^ 1)]), "tiles")) return WF_STATUS_OOM;
+        known = h_n[slot ^ 1];
+      }
+      ++chunk;
+    }
+    if (!full) {
+      const int rc = run_steps(e, js, shape, g, a, ids, n, info, records, rec_units, &unit);
+      if (rc != WF_STATUS_OK) return rc;
+    }
+    wfa::TileFinishArgs f{};
+    f.n = n;
+    f.jobs = t.d_jobs.as<int>();
+    f.plen = js.plen;
+    f.tlen = js.tlen;
+    f.done = a.done;
+    f.irr = a.irr;
+    f.exact_lo = a.exact_lo;
+    f.exact_hi = a.exact_hi;
+    for (int x = 0; x < 4; ++x) f.dev[x / 2][x % 2] = a.dev[x / 2][x % 2];
+    f.stepped = a.stepped;
+    f.step_ends = t.d_ends.as<int>();
+    f.flags = t.d_flags.as<int>();
+    f.dsum = t.d_dsum.as<long long>();
+    f.steps = T;
+    f.dsteps_upto = t.d_dsteps.as<long long>();
+    f.g = pen.g;
+    f.out_status = js.status;
+    f.out_score = js.score;
+    f.out_dsteps = js.dsteps;
+    f.out_last_block = js.last;
+    f.out_end_k = js.end_k;
+    f.out_end_off = js.end_off;
+    f.dsteps_total = &c->dsteps;
+    f.retry_count = &c->retry;
+    if (!hip_ok(wfa::launch_tile_finish(shape, f, st), "tile finish")) return WF_STATUS_OOM;
+    (void)hipEventRecord(t.ev[1], st);
+    if (records) {
+      wfa::TileTraceArgs ta{};
+      ta.jobs = t.d_jobs.as<int>();
+      ta.plen = js.plen;
+      ta.tlen = js.tlen;
+      ta.status = js.status;
+      ta.score = js.score;
+      ta.rec = a.rec;
+      ta.rec_tab = a.rec_tab;
+      ta.tab_stride = a.tab_stride;
+      ta.blocks = t.d_info.as<wfa::TileBlockInfo>();
+      ta.words = js.words;
+      ta.pat_pos = js.ppos;
+      ta.txt_pos = js.tpos;
+      ta.ops = js.ops;
+      ta.ops_off = js.ops_off;
+      ta.ops_begin = js.ops_begin;
+      ta.fail_count = &c->fail;
+      ta.g = pen.g;
+      ta.lmax_words = lw;
+      if (!hip_ok(wfa::launch_tile_backtrace(shape, ta, n, st), "tile backtrace")) return WF_STATUS_OOM;
+    }
+    (void)hipEventRecord(t.ev[2], st);
+    if (!hip_ok(hipStreamSynchronize(st), "tiles")) return WF_STATUS_OOM;
+    float fms = 0, bms = 0;
+    (void)hipEventElapsedTime(&fms, t.ev[0], t.ev[1]);
+    (void)hipEventElapsedTime(&bms, t.ev[1], t.ev[2]);
+    tot->forward_ms += fms;
+    tot->backtrace_ms += bms;
+    if (first > 0) ++tot->launches;  // a further pass (the caller counts one)
+    first += n;
+  }
+  return WF_STATUS_OK;
+}
+
+}  // namespace wfa_host
