@@ -229,7 +229,7 @@ bool engine_init(Engine* e) {
   } else if (!hip_ok(hipStreamCreateWithFlags(&e->stream, hipStreamNonBlocking), "hipStreamCreate")) {
     return false;
   }
-  if (!e->counters.ensure(64)) return false;
+  if (!e->counters.ensure(sizeof(wfa::Counters))) return false;
   // Record arena: up to half of the free HBM (block indices address 64 GB),
   // or WFA_RECORD_ARENA_MB; each run sizes it from its pairs' lengths.
   size_t free_b = 0, total_b = 0;
@@ -782,7 +782,7 @@ void group_args(wavefront_aligner_t* wf, Engine* e, const JobSet& js, const Plan
   fa.rec_top = &c->rec_top;
   fa.ring_global = grp.family == wfa::kLarge ? e->ring.as<int>() : nullptr;
   fa.ring_stride = grp.family == wfa::kLarge ? (long long)wfa::ring_slots(pen) * grp.wcap : 0;
-  fa.queue = &c->queue;
+  fa.queue = c->queue;
   fa.dsteps_total = &c->dsteps;
   fa.retry_count = &c->retry;
   fa.fail_count = &c->fail;
@@ -836,9 +836,11 @@ void group_args(wavefront_aligner_t* wf, Engine* e, const JobSet& js, const Plan
 
 // Forward (and, with records, backtrace) launches of one group, with the
 // group's events around them when it has events.
-hipError_t launch_group(const PlanGroup& grp, const LaunchShape& shape, const ForwardArgs& fa,
+hipError_t launch_group(const PlanGroup& grp, const LaunchShape& shape, const ForwardArgs& args,
                         const BacktraceArgs& ba, int ncomp, int bits, int records, hipStream_t st) {
   if (grp.ev[0]) (void)hipEventRecord(grp.ev[0], st);
+  ForwardArgs fa = args;
+  fa.queues = shape.grid >= 64 * wfa::kMaxQueues ? wfa::kMaxQueues : 1;
   hipError_t err = grp.family == wfa::kLean ? wfa::launch_forward_lean(fa, shape, st)
                                             : wfa::launch_forward(fa, ncomp, bits, shape, st);
   if (err != hipSuccess) return err;
@@ -1030,7 +1032,7 @@ int run_jobs(wavefront_aligner_t* wf, Engine* e, const JobSet& js, std::vector<P
       if (!g.ids.empty()) fresh = false;
       ++tot->launches;
     }
-    if (!hip_ok(hipMemcpyAsync(&host_c, e->counters.p, sizeof(host_c), hipMemcpyDeviceToHost, st), "counters") ||
+    if (!hip_ok(hipMemcpyAsync(&host_c, e->counters.p, wfa::kCounterTotals, hipMemcpyDeviceToHost, st), "counters") ||
         !hip_ok(hipStreamSynchronize(st), "alignment"))
       return WF_STATUS_OOM;
     for (PlanGroup& g : *pending) {
@@ -1760,6 +1762,7 @@ namespace wfa_host {
 int device_batch_run_in(wavefront_aligner_t* wf, wfa_device_batch_t* b, char* scratch, size_t bytes) {
   constexpr size_t kRingShare = 64ull << 20;
   constexpr size_t kMinArena = 32ull << 20;
+  constexpr size_t kCounters = (sizeof(wfa::Counters) + 255) & ~(size_t)255;
   if (!b) return WF_STATUS_OOM;
   presets_check(wf, b->plen.data(), b->tlen.data(), b->n);
   const int sup = check_supported(wf);
@@ -1781,10 +1784,10 @@ int device_batch_run_in(wavefront_aligner_t* wf, wfa_device_batch_t* b, char* sc
     return WF_STATUS_OOM;
   }
   const size_t order_bytes = ((size_t)b->n * 8 + 4096 + 255) & ~(size_t)255;
-  if (256 + order_bytes + kRingShare + kMinArena > bytes) {
+  if (kCounters + order_bytes + kRingShare + kMinArena > bytes) {
     fprintf(stderr, "[WFA] wfa_device_batch_run_noalloc: %d pairs exceed the %zu MB scratch array "
             "(at most %zu pairs per call)\n", b->n, bytes >> 20,
-            (size_t)((bytes - 256 - kRingShare - kMinArena - 4096) / 8));
+            (size_t)((bytes - kCounters - kRingShare - kMinArena - 4096) / 8));
     return WF_STATUS_OOM;
   }
   const Penalties pen = make_penalties(wf->penalties);
@@ -1799,19 +1802,19 @@ int device_batch_run_in(wavefront_aligner_t* wf, wfa_device_batch_t* b, char* sc
   }
   // counters | order arrays | ring share | record arena
   Engine::NoAlloc na;
-  na.order.base = scratch + 256;
+  na.order.base = scratch + kCounters;
   na.order.bytes = order_bytes;
   na.ring_bytes = kRingShare;
   ScratchRegion fixed;  // binds the views below: they never allocate or free
   DevBuf counters, ring, rec;
   counters.p = scratch;
-  counters.cap = 256;
+  counters.cap = kCounters;
   counters.region = &fixed;
-  ring.p = scratch + 256 + order_bytes;
+  ring.p = scratch + kCounters + order_bytes;
   ring.cap = kRingShare;
   ring.region = &fixed;
-  rec.p = scratch + 256 + order_bytes + kRingShare;
-  rec.cap = (bytes - 256 - order_bytes - kRingShare) & ~(size_t)255;
+  rec.p = scratch + kCounters + order_bytes + kRingShare;
+  rec.cap = (bytes - kCounters - order_bytes - kRingShare) & ~(size_t)255;
   rec.region = &fixed;
   std::swap(e->counters, counters);
   std::swap(e->ring, ring);
@@ -2041,7 +2044,7 @@ int plain_run(wavefront_aligner_t* wf, Engine* e, wfa_device_batch_t* b, const w
               wfa::launch_reset_counters(counters_of(e), 2, st) == hipSuccess &&
               launch_group(g, shape, fa, ba, pen.ncomp, js.bits, records, st) == hipSuccess &&
               hipMemcpyAsync(out, b->d_res.p, 5 * sizeof(int), hipMemcpyDeviceToHost, st) == hipSuccess &&
-              hipMemcpyAsync(out + 64, e->counters.p, sizeof(wfa::Counters), hipMemcpyDeviceToHost, st) ==
+              hipMemcpyAsync(out + 64, e->counters.p, wfa::kCounterTotals, hipMemcpyDeviceToHost, st) ==
                   hipSuccess &&
               (!records || hipMemcpyAsync(out + 256, b->d_ops.p, ops_cap, hipMemcpyDeviceToHost, st) == hipSuccess);
     const hipError_t ec = hipStreamEndCapture(st, &graph);
@@ -2061,8 +2064,8 @@ int plain_run(wavefront_aligner_t* wf, Engine* e, wfa_device_batch_t* b, const w
   if (!hip_ok(hipGraphLaunch(pg.exec, st), "graph launch") || !hip_ok(hipStreamSynchronize(st), "graph"))
     return WF_STATUS_OOM;
   ++pg.replays;
-  wfa::Counters c;
-  memcpy(&c, out + 64, sizeof(c));
+  wfa::Counters c{};
+  memcpy(&c, out + 64, wfa::kCounterTotals);
   if (c.retry != 0) return 1;  // a ring or the arena overflowed: the general path retries (inputs are up)
   b->status.assign(1, 0);
   b->score.assign(1, 0);

@@ -208,7 +208,7 @@ bool run_breakpoints(wavefront_aligner_t* wf, Engine* e, wfa_device_batch_t* b, 
       a.ring = e->ring.as<int>();
       a.ring_stride = stride;
       a.wcap = wcap;
-      a.queue = &c->queue;
+      a.queue = c->queue;
       a.dsteps_total = &c->dsteps;
       a.max_steps = wf->system.max_alignment_steps > 0 ? wf->system.max_alignment_steps : INT_MAX;
       a.lmax_words = lw;
@@ -234,7 +234,7 @@ bool run_breakpoints(wavefront_aligner_t* wf, Engine* e, wfa_device_batch_t* b, 
       (void)hipEventRecord(e1, st);
       ok = ok && hip_ok(hipMemcpyAsync(res.data(), d_out.p, res.size() * sizeof(wfa::BiOutcome),
                                        hipMemcpyDeviceToHost, st), "bi download") &&
-           hip_ok(hipMemcpyAsync(&host_c, e->counters.p, sizeof(host_c), hipMemcpyDeviceToHost, st), "counters") &&
+           hip_ok(hipMemcpyAsync(&host_c, e->counters.p, wfa::kCounterTotals, hipMemcpyDeviceToHost, st), "counters") &&
            hip_ok(hipStreamSynchronize(st), "breakpoint");
       float ms = 0;
       (void)hipEventElapsedTime(&ms, e0, e1);

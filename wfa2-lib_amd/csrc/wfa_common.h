@@ -35,6 +35,22 @@ struct MetaRegs {
   CutRange<NC, CUT> cut;
 };
 
+// The work queue of the persistent kernels: `queues` counters in lines of
+// their own.  Workgroup b takes item b first, then the items of its counter
+// b % queues: those congruent to it modulo `queues`, in order (the pairs are
+// sorted by length, so every counter deals the same mix).  One counter for
+// all serves about 80 million pairs a second (atomics of every die on one
+// address): 150,000 short reads took 1.9 ms of forward kernel whatever the
+// metric, 0.9 ms (edit distance) and 1.5 ms (gap-affine scores) on 16.
+__device__ __forceinline__ unsigned int* work_queue(unsigned int* queue, int queues) {
+  return queue + ((int)blockIdx.x & (queues - 1)) * kQueueStride;
+}
+__device__ __forceinline__ int work_item(int queues, bool first, int taken) {
+  const int b = (int)blockIdx.x, g = (int)gridDim.x, id = b & (queues - 1);
+  // the counter's first items went to its (g - id + queues - 1) / queues workgroups
+  return first ? b : id + queues * (taken + (g - id + queues - 1) / queues);
+}
+
 constexpr int kFarDiagonal = 0x40000000;
 
 // A compute input.  lim_lo/lim_hi are the limits it contributes to the output

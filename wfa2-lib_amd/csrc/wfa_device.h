@@ -1,6 +1,7 @@
 // Internal interface between the C-ABI host layer (wfa_api.cpp) and the HIP
 // kernels (wfa_kernels.hip).  Not installed; no torch types anywhere.
 #pragma once
+#include <stddef.h>
 #include <stdint.h>
 #include <hip/hip_runtime.h>
 
@@ -94,6 +95,9 @@ struct HeurArgs {
   __host__ __device__ int cut() const { return (xdrop || zdrop) ? 2 : ((wfadaptive || banded) ? 1 : 0); }
 };
 
+// Work-queue counters of a launch, and their distance (a 128-byte line each).
+constexpr int kMaxQueues = 16, kQueueStride = 32;
+
 struct ForwardArgs {
   int n_pairs;
   const int* order;            // processing order (pair ids), longest first
@@ -113,7 +117,8 @@ struct ForwardArgs {
   unsigned long long* rec_top; // bump pointer into the arena, 16-byte units
   int* ring_global;            // per-workgroup ring scratch (global-ring kernels)
   long long ring_stride;       // ints per workgroup
-  unsigned int* queue;         // work-queue counter
+  unsigned int* queue;         // work-queue counters (kQueueStride apart)
+  int queues;                  // how many of them: a power of two, at most kMaxQueues and the grid
   unsigned long long* dsteps_total;  // sum of diagonal-steps over the launch
   unsigned int* retry_count;   // pairs that must be re-run (ring overflow / arena full)
   unsigned int* fail_count;    // pairs that finished with another non-completed status
@@ -185,17 +190,20 @@ struct LaunchShape {
 hipError_t launch_forward(const ForwardArgs& a, int ncomp, int bits,
                           const LaunchShape& shape, hipStream_t stream);
 hipError_t launch_backtrace(const BacktraceArgs& a, hipStream_t stream);
-// Device counters of one run (one 64-byte block).
+// Device counters of one run: the totals (64 bytes, copied to the host) and
+// the work queues of the current launch.
 struct Counters {
-  unsigned int queue;            // work queue of the current launch
+  unsigned int pad1;
   unsigned int retry;            // pairs to re-run (ring overflow / arena full)
   unsigned long long rec_top;    // record arena bump pointer (16-byte units)
   unsigned long long dsteps;     // diagonal-steps of the pairs that finished
   unsigned int fail;             // pairs that finished with a status other than completed
   unsigned int pad0;
-  unsigned long long pad[4];
+  unsigned long long pad[12];
+  unsigned int queue[kMaxQueues * kQueueStride];
 };
-static_assert(sizeof(Counters) == 64, "Counters layout");
+constexpr int kCounterTotals = 64;  // bytes of the totals
+static_assert(offsetof(Counters, queue) == 128, "Counters layout");
 // Zeroes the queue and the arena pointer; with all=1 also retry; with all=2
 // also the run totals (diagonal-steps, failures).
 hipError_t launch_reset_counters(Counters* c, int all, hipStream_t stream);

@@ -144,10 +144,15 @@ __global__ void __launch_bounds__(BLOCK, BLOCK == 1024 ? 4 : 1) wfa_forward_kern
   unsigned long long wg_dsteps = 0;                  // diagonal-steps of this workgroup
   MetaRegs<NC, HC> meta;
 
+  bool q_first = true;
   for (;;) {
     int qv = 0;
-    if (tid == 0) qv = (int)atomicAdd(a.queue, 1u);
-    const int qi = broadcast0(qv, 0);
+    if (!q_first) {
+      if (tid == 0) qv = (int)atomicAdd(work_queue(a.queue, a.queues), 1u);
+      qv = broadcast0(qv, 0);
+    }
+    const int qi = work_item(a.queues, q_first, qv);
+    q_first = false;
     if (qi >= a.n_pairs) break;
     const int p = a.order ? a.order[qi] : qi;
     const int plen = a.plen[p];
@@ -1005,8 +1010,8 @@ __global__ void __launch_bounds__(256) wfa_backtrace_kernel(BacktraceArgs a) {
 }
 
 __global__ void wfa_reset_kernel(Counters* c, int all) {
+  if (threadIdx.x < kMaxQueues) c->queue[threadIdx.x * kQueueStride] = 0u;
   if (threadIdx.x == 0) {
-    c->queue = 0u;
     c->rec_top = 0ull;
     if (all >= 1) c->retry = 0u;
     if (all >= 2) { c->dsteps = 0ull; c->fail = 0u; }

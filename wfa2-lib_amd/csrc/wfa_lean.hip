@@ -265,11 +265,14 @@ __global__ void __launch_bounds__(64) wfa_forward_lean_kernel(ForwardArgs a) {
   uint32_t chunk_cur = 0, chunk_end = 0;  // record chunk of this wave (16-byte units)
   unsigned long long wg_dsteps = 0;
 
+  // Pairs are dealt over a.queues counters (see work_item).
+  bool q_first = true;
   for (;;) {
-    int qv = 0;
     KernArgs A = args_now();
-    if (lane == 0) qv = (int)atomicAdd(A->queue, 1u);
-    const int qi = lane_of(qv, 0);
+    int qv = 0;
+    if (!q_first && lane == 0) qv = (int)atomicAdd(work_queue(A->queue, A->queues), 1u);
+    const int qi = work_item(A->queues, q_first, lane_of(qv, 0));
+    q_first = false;
     if (qi >= A->n_pairs) break;
     const int p = A->order ? A->order[qi] : qi;
     const int plen = A->plen[p];
