@@ -16,6 +16,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <array>
 #include <atomic>
 #include <climits>
 #include <cstdio>
@@ -100,6 +101,9 @@ PlanGroup& PlanGroup::operator=(PlanGroup&& o) noexcept {
   lmax_words = o.lmax_words;
   max_grid = o.max_grid;
   lclass = o.lclass;
+  wave = o.wave;
+  wave_rec = o.wave_rec;
+  wave_ef = o.wave_ef;
   ids = std::move(o.ids);
   d_ids = std::move(o.d_ids);
   ids_on_device = o.ids_on_device;
@@ -685,6 +689,7 @@ int small_wcap(const Penalties& pen, int ncomp) {
 // WFA_LEAN=0 turns the family off; WFA_LEAN_WCAP="short,long[,short_len]"
 // overrides the widths.
 constexpr int kLeanMaxLen = 1024;
+constexpr int kLeanMaxRing = 768;  // the widest instance
 struct LeanTuning {
   bool enabled = true;
   int wcap_short = 224;
@@ -733,7 +738,10 @@ LaunchShape shape_of(Engine* e, const PlanGroup& g, int bits, const Penalties& p
   shape.family = g.family;
   shape.block = g.block;
   int per_cu = 0;
-  if (g.family == wfa::kLean) {
+  if (g.family == wfa::kWave) {
+    shape.lds_bytes = wfa::wave_lds_bytes(g.lmax_words);
+    per_cu = wfa::wave_max_blocks_per_cu(wfa::wave_shape(pen), g.wcap, g.wave_rec, bits, g.wave_ef, shape.lds_bytes);
+  } else if (g.family == wfa::kLean) {
     shape.lds_bytes = wfa::lean_lds_bytes(pen, g.wcap, g.lmax_words);
     per_cu = wfa::lean_max_blocks_per_cu(pen, g.wcap, shape.lds_bytes);
   } else {
@@ -831,7 +839,22 @@ void group_args(wavefront_aligner_t* wf, Engine* e, const JobSet& js, const Plan
   ba.end_off = js.end_off;
   ba.end_rec = js.end_rec;
   ba.pen = pen;
+  if (grp.family == wfa::kWave) {
+    pfa->wave = grp.wave;
+    pfa->wave.lds_words = grp.lmax_words;
+    ba.wave = pen.ncomp;
+    for (int ph = 0; ph < wfa::kWavePhases; ++ph) ba.wave_last[ph] = grp.wave.last[ph];
+    ba.wave_center = grp.wave.center;
+  }
   *pba = ba;
+}
+
+// The kernel and phases of a wave group.
+void set_wave(const JobSet& js, PlanGroup& g, const Penalties& pen, int records) {
+  if (g.family != wfa::kWave) return;
+  g.wave_rec = records != 0;
+  g.wave_ef = js.ef.on != 0;
+  (void)wfa::wave_phases(wfa::wave_shape(pen), js.ef.on ? js.ef.pbf : 0, js.ef.on ? js.ef.tbf : 0, g.wcap, &g.wave);
 }
 
 // Forward (and, with records, backtrace) launches of one group, with the
@@ -841,8 +864,10 @@ hipError_t launch_group(const PlanGroup& grp, const LaunchShape& shape, const Fo
   if (grp.ev[0]) (void)hipEventRecord(grp.ev[0], st);
   ForwardArgs fa = args;
   fa.queues = shape.grid >= 64 * wfa::kMaxQueues ? wfa::kMaxQueues : 1;
-  hipError_t err = grp.family == wfa::kLean ? wfa::launch_forward_lean(fa, shape, st)
-                                            : wfa::launch_forward(fa, ncomp, bits, shape, st);
+  hipError_t err = grp.family == wfa::kWave
+                       ? wfa::launch_forward_wave(fa, wfa::wave_shape(fa.pen), grp.wcap, bits, shape, st)
+                   : grp.family == wfa::kLean ? wfa::launch_forward_lean(fa, shape, st)
+                                              : wfa::launch_forward(fa, ncomp, bits, shape, st);
   if (err != hipSuccess) return err;
   if (grp.ev[1]) (void)hipEventRecord(grp.ev[1], st);
   if (records) {
@@ -860,6 +885,7 @@ int enqueue_group(wavefront_aligner_t* wf, Engine* e, const JobSet& js, PlanGrou
   const int n = (int)grp.ids.size();
   if (n == 0) return WF_STATUS_OK;
   hipStream_t st = e->stream;
+  set_wave(js, grp, pen, records);
   const LaunchShape shape = shape_of(e, grp, js.bits, pen, js.heur.cut());
   bool ident = true;
   for (int i = 0; i < n && ident; ++i) ident = grp.ids[i] == i;
@@ -923,21 +949,35 @@ std::vector<PlanGroup> make_plan(const JobSet& js, const std::vector<int>& ids, 
   const bool heur_ok = js.heur.cut() <= 1;
   const bool lean_ok = lt.enabled && ncomp == 3 && js.bits == 2 && !js.cbeg && !js.cend && ef_fits && heur_ok &&
                        wfa::lean_supported(pen);
-  std::vector<int> lean_ids[2], tile_ids;
+  std::vector<int> lean_ids[2], wave_ids[2], tile_ids;
   int lean_lmax[2] = {0, 0};
   // Pairs above 1,024 bases in tiles, where the kernels have an instance: on
   // any number of pairs the device is filled by tiles, not by pairs.
   const bool tile_ok = js.tiles && js.bits == 2 && !js.cbeg && !js.cend && !js.ef.on && js.heur.cut() == 0 &&
                        wfa::tile_shape(pen) != 0;
+  // Pairs of at most 1,024 bases on the wave family where it has an instance:
+  // up to 4 diagonals per lane for the short class, 8 above.
+  wfa::WaveArgs wa;
+  const bool wave_ok = lt.enabled && js.unlimited && !js.cbeg && !js.cend && js.heur.cut() == 0 &&
+                       (js.bits == 2 || js.nibbles) && wfa::wave_shape(pen) != 0 &&
+                       wfa::wave_phases(wfa::wave_shape(pen), js.ef.on ? js.ef.pbf : 0, js.ef.on ? js.ef.tbf : 0, 4, &wa);
+  int wave_words[2] = {0, 0};
   for (int i : ids) {
     const int L = std::max(js.h_plen[i], js.h_tlen[i]);
+    // (with a second gap, pairs of the longer class outgrow a wave: tiles)
+    if (wave_ok && L <= (ncomp == 5 && tile_ok ? lt.short_len : kLeanMaxLen)) {
+      const int c = L <= lt.short_len ? 0 : 1;
+      wave_ids[c].push_back(i);
+      wave_words[c] = std::max(wave_words[c], js.bits == 2 ? 2 * (L / 32 + 3) : L / 8 + 3);
+      continue;
+    }
     if (lean_ok && L <= kLeanMaxLen) {
       const int c = L <= lt.short_len ? 0 : 1;
       lean_ids[c].push_back(i);
       lean_lmax[c] = std::max<int>(lean_lmax[c], L / spw + 3);
       continue;
     }
-    if (tile_ok && L > kLeanMaxLen && tile_fits(js.h_plen[i], js.h_tlen[i])) {
+    if (tile_ok && L > (ncomp == 5 ? lt.short_len : kLeanMaxLen) && tile_fits(js.h_plen[i], js.h_tlen[i])) {
       tile_ids.push_back(i);
       continue;
     }
@@ -950,6 +990,16 @@ std::vector<PlanGroup> make_plan(const JobSet& js, const std::vector<int>& ids, 
     }
   }
   std::vector<PlanGroup> plan;
+  for (int c = 0; c < 2; ++c) {
+    if (wave_ids[c].empty()) continue;
+    PlanGroup g;
+    g.family = wfa::kWave;
+    g.block = 64;
+    g.wcap = c == 0 ? 4 : 8;
+    g.lmax_words = wave_words[c];
+    g.ids = std::move(wave_ids[c]);
+    plan.push_back(std::move(g));
+  }
   for (int c = 0; c < 2; ++c) {
     if (lean_ids[c].empty()) continue;
     PlanGroup g;
@@ -1005,6 +1055,7 @@ int run_jobs(wavefront_aligner_t* wf, Engine* e, const JobSet& js, std::vector<P
           w += L * L * per_l2 + 8 * L;
         }
         g.est_rec_bytes = w;
+        set_wave(js, g, pen, records);
         if (g.family != wfa::kTile)  // and the record chunk of every workgroup
           g.est_rec_bytes += (double)shape_of(e, g, js.bits, pen, js.heur.cut()).grid * wfa::kChunkUnits * 16;
       }
@@ -1059,7 +1110,28 @@ int run_jobs(wavefront_aligner_t* wf, Engine* e, const JobSet& js, std::vector<P
         else if (h_status[i] == wfa::kDevArenaFull) arena_full.push_back(i);
       }
       if (!ring_over.empty()) {
-        if (g.family == wfa::kLean && wfa::lean_width(g.wcap + 1) > 0) {
+        if (g.family == wfa::kWave && g.wcap < 8) {
+          PlanGroup h = take_group(e);
+          h.family = wfa::kWave;
+          h.block = 64;
+          h.wcap = 8;
+          h.lmax_words = g.lmax_words;
+          h.ids = std::move(ring_over);
+          next.push_back(std::move(h));
+        } else if (g.family == wfa::kWave && pen.ncomp == 5 && js.tiles && js.bits == 2 && !js.ef.on) {
+          PlanGroup h = take_group(e);
+          h.family = wfa::kTile;
+          h.ids = std::move(ring_over);
+          next.push_back(std::move(h));
+        } else if (g.family == wfa::kWave && js.bits == 2 && wfa::lean_supported(pen)) {
+          PlanGroup h = take_group(e);
+          h.family = wfa::kLean;
+          h.block = 64;
+          h.wcap = wfa::lean_width(kLeanMaxRing);
+          h.lmax_words = (g.lmax_words + 1) / 2;
+          h.ids = std::move(ring_over);
+          next.push_back(std::move(h));
+        } else if (g.family == wfa::kLean && wfa::lean_width(g.wcap + 1) > 0) {
           PlanGroup h = take_group(e);
           h.family = wfa::kLean;
           h.block = 64;
@@ -1185,7 +1257,9 @@ wfa_host::JobSet wfa_device_batch_t::jobs() const {
   js.end_rec = d_end_rec.as<int>();
   js.ef = ef;
   js.heur = heur;
+  js.unlimited = unlimited;
   js.tiles = tiles;
+  js.nibbles = nibbles;
   return js;
 }
 
@@ -1298,10 +1372,20 @@ bool wfa_device_batch_t::load(Engine* e, const wfa_pair_t* pairs, int count, boo
   const int64_t per_thread = 1 << 16;  // symbols: small batches are packed inline
   const int nt = std::max(1, std::min<int>({16, (int)std::thread::hardware_concurrency(),
                                             (int)std::min<int64_t>(nw * (64 / bits) / per_thread + 1, 16)}));
+  // symbols present in an 8-bit batch, per thread
+  std::vector<std::array<bool, 256>> seen(bits == 8 ? nt : 0);
+  for (auto& s : seen) s.fill(false);
   auto pack = [&](int t) {
     for (int i = t; i < n; i += nt) {
       pack_seq(host_words + patw[i], pairs[i].pattern, plen[i], bits);
       pack_seq(host_words + txtw[i], pairs[i].text, tlen[i], bits);
+      if (bits == 8) {
+        bool* s = seen[t].data();
+        const unsigned char* p = reinterpret_cast<const unsigned char*>(pairs[i].pattern);
+        for (int j = 0; j < plen[i]; ++j) s[p[j]] = true;
+        const unsigned char* q = reinterpret_cast<const unsigned char*>(pairs[i].text);
+        for (int j = 0; j < tlen[i]; ++j) s[q[j]] = true;
+      }
     }
   };
   if (nt == 1) {
@@ -1310,6 +1394,15 @@ bool wfa_device_batch_t::load(Engine* e, const wfa_pair_t* pairs, int count, boo
     std::vector<std::thread> th;
     for (int t = 0; t < nt; ++t) th.emplace_back(pack, t);
     for (auto& x : th) x.join();
+  }
+  nibbles = bits == 8;
+  if (bits == 8) {
+    int of_nibble[16] = {};
+    for (int c = 0; c < 256; ++c) {
+      bool any = false;
+      for (const auto& s : seen) any = any || s[c];
+      if (any && of_nibble[c & 15]++) nibbles = false;
+    }
   }
   // Longest pairs first, ties in input order: a counting sort over
   // plen + tlen when the longest is within a few times the pair count, else
@@ -1659,7 +1752,8 @@ int batch_run(wavefront_aligner_t* wf, wfa_device_batch_t* b, Engine* e) {
   b->records = records;
   b->ef = ends_free_of(wf);
   b->heur = heuristic_of(wf);
-  b->tiles = !e->na && unlimited_steps(wf);
+  b->unlimited = unlimited_steps(wf);
+  b->tiles = b->unlimited && !e->na;
   b->stats = wfa_run_stats_t{};
   b->have_results = false;
   b->host_results = false;
@@ -1692,7 +1786,7 @@ int batch_run(wavefront_aligner_t* wf, wfa_device_batch_t* b, Engine* e) {
     if (rc != WF_STATUS_OK) return rc;
   } else {
     const std::vector<int> key = {pen.metric, pen.x, pen.o1, pen.e1, pen.o2, pen.e2, b->bits, b->ef.on,
-                                  b->heur.cut(), records, b->tiles};
+                                  b->heur.cut(), records, b->unlimited};
     if (b->plan_key != key) {
       std::vector<PlanGroup> plan = make_plan(b->jobs(), b->sorted, pen);
       std::vector<TuneTrial> trials;
@@ -1987,7 +2081,7 @@ int plain_run(wavefront_aligner_t* wf, Engine* e, wfa_device_batch_t* b, const w
   b->heur = heuristic_of(wf);
   b->stats = wfa_run_stats_t{};
   b->bi_mode = false;
-  b->tiles = unlimited_steps(wf);
+  b->unlimited = b->tiles = unlimited_steps(wf);
   b->first_fail = WF_STATUS_ALG_COMPLETED;
   hipStream_t st = e->stream;
   const JobSet js = b->jobs();
@@ -1999,13 +2093,16 @@ int plain_run(wavefront_aligner_t* wf, Engine* e, wfa_device_batch_t* b, const w
   };
   if (plan.size() != 1 || plan[0].family == wfa::kTile) return general();
   PlanGroup& g = plan[0];
-  if (g.family != wfa::kLarge) g.lmax_words = (int)(upload / 8);  // the bucket's words: a capacity, not a length
+  // the bucket's words: a capacity, not a length (32-bit LDS words for the wave family)
+  if (g.family == wfa::kWave) g.lmax_words = (int)(upload / 8) * (js.bits == 2 ? 2 : 1);
+  else if (g.family != wfa::kLarge) g.lmax_words = (int)(upload / 8);
+  set_wave(js, g, pen, records);
   if (!reserve_for(e, plan, js.bits, pen, js.heur.cut(), records)) return WF_STATUS_OOM;
   size_t ops_cap = 1024;
   while ((int64_t)ops_cap < b->total_ops) ops_cap *= 2;
   if ((records && !b->d_ops.ensure(ops_cap)) || !e->plain_out.ensure(256 + ops_cap)) return WF_STATUS_OOM;
   const LaunchShape shape = shape_of(e, g, js.bits, pen, js.heur.cut());
-  ForwardArgs fa;
+  ForwardArgs fa{};
   BacktraceArgs ba;
   group_args(wf, e, js, g, pen, records, true, &fa, &ba);
   char* out = e->plain_out.as<char>();

@@ -51,6 +51,21 @@ __device__ __forceinline__ int work_item(int queues, bool first, int taken) {
   return first ? b : id + queues * (taken + (g - id + queues - 1) / queues);
 }
 
+// The kernel arguments, reread from the kernel-argument segment where a
+// value is needed outside the step loop (the asm makes each pointer opaque,
+// so the compiler reloads instead of keeping every field in scalar
+// registers across the loop).
+using KernArgs = const __attribute__((address_space(4))) ForwardArgs*;
+__device__ __forceinline__ KernArgs args_now() {
+#if defined(__HIP_DEVICE_COMPILE__)
+  KernArgs p = (KernArgs)__builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(p));
+  return p;
+#else
+  return nullptr;  // host pass of the single-source compile: never executed
+#endif
+}
+
 constexpr int kFarDiagonal = 0x40000000;
 
 // A compute input.  lim_lo/lim_hi are the limits it contributes to the output

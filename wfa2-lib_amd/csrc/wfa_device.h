@@ -98,6 +98,15 @@ struct HeurArgs {
 // Work-queue counters of a launch, and their distance (a 128-byte line each).
 constexpr int kMaxQueues = 16, kQueueStride = 32;
 
+// Wave family: N = 1, 2, 4, 8 diagonals per lane in turn.
+constexpr int kWavePhases = 4;
+struct WaveArgs {
+  int last[kWavePhases];       // steps done when each phase ends (its wavefronts fit the wave)
+  int center;                  // diagonal of lane 32
+  int phase0;                  // phase that holds the score-0 wavefront
+  int lds_words;               // LDS words (32-bit) per sequence
+};
+
 struct ForwardArgs {
   int n_pairs;
   const int* order;            // processing order (pair ids), longest first
@@ -138,6 +147,7 @@ struct ForwardArgs {
   int* out_end_off;
   int* out_end_rec;            // z-drop: the end cell's record byte (0xFF: no source), or null
   HeurArgs heur;                // heuristic cut-off (none: the exact instances)
+  WaveArgs wave;                // wave family
   Penalties pen;
 };
 
@@ -169,6 +179,9 @@ struct BacktraceArgs {
   const int* end_k;
   const int* end_off;
   const int* end_rec;          // z-drop: the end cell's record byte (0xFF: no source)
+  int wave;                    // records of the wave family: its components (1, 3 or 5), else 0
+  int wave_last[kWavePhases];  // WaveArgs::last and center
+  int wave_center;
   Penalties pen;
 };
 
@@ -177,7 +190,9 @@ struct BacktraceArgs {
 // kLean: like kSmall, gap-affine with 2-bit sequences, specialised on the
 // penalties' slot structure (wfa_lean.hip).  kTile: long pairs in tiles of
 // diagonals, a block of steps per launch (wfa_tile.hip).
-enum Family : int { kSmall = 0, kLarge = 1, kLean = 2, kTile = 3 };
+// kWave: short pairs, one wave per pair with the wavefronts in registers
+// (wfa_wave.hip).
+enum Family : int { kSmall = 0, kLarge = 1, kLean = 2, kTile = 3, kWave = 4 };
 
 struct LaunchShape {
   int family = 0;

@@ -10,6 +10,7 @@
 #include "wfa_device.h"
 #include "wfa_mi355x.h"
 #include "wfa_tile.h"
+#include "wfa_wave.h"
 
 namespace wfa_host {
 
@@ -99,6 +100,8 @@ struct PlanGroup {
   bool ids_on_device = false;  // d_ids holds ids (uploaded once per plan)
   double est_rec_bytes = -1;   // rough record footprint of the group (computed once)
   int lclass = -1;             // lean family: length class (0 short, 1 long)
+  wfa::WaveArgs wave{};        // wave family (wcap: most diagonals per lane): phases, set before a launch
+  bool wave_rec = false, wave_ef = false;  // ... and its kernel instance
   hipEvent_t ev[3] = {nullptr, nullptr, nullptr};
   PlanGroup() = default;
   PlanGroup(const PlanGroup&) = delete;
@@ -146,8 +149,6 @@ struct Engine {
   struct TileState {
     int shape = 0;
     std::vector<int> lo, hi;          // hull of the ranges up to each step
-    std::vector<int> m_range;         // untrimmed range of M at each step (lo, hi)
-    std::vector<long long> dsteps;
     DevBuf d_range, d_dsteps, d_job_range, d_dev, d_ends, d_flags, d_dsum, d_step_state, d_step_off, d_step0, d_step_act, d_off, d_pitch, d_jobs, d_marks, d_act, d_info, d_tab;
     HostBuf h_n;                      // jobs left, written by the device
     hipEvent_t ev[5] = {nullptr, nullptr, nullptr, nullptr, nullptr};
@@ -231,7 +232,9 @@ struct JobSet {
   int* end_rec = nullptr;      // z-drop: record byte of the end cell (0xFF: no source)
   EndsFree ef;
   wfa::HeurArgs heur{};        // wf-adaptive (none for BiWFA base jobs)
-  bool tiles = false;          // long jobs may run in tiles (no step limit, buffers may grow)
+  bool unlimited = false;      // no step limit: the wave family may run
+  bool tiles = false;          // ... and the tile family (its buffers may grow)
+  bool nibbles = false;        // 8-bit symbols that differ in their low four bits
 };
 
 // The aligner's wf-adaptive parameters (none unless the strategy is wf-adaptive).
@@ -287,7 +290,8 @@ struct wfa_device_batch_t {
   std::vector<int> status, score, ops_begin, end_k, end_off;
   wfa_host::EndsFree ef;                   // form of the last run
   wfa::HeurArgs heur{};                    // heuristic of the last run
-  bool tiles = false;                      // whether the last run could take long pairs in tiles
+  bool unlimited = false, tiles = false;   // JobSet::unlimited and tiles of the last run
+  bool nibbles = false;                    // 8-bit symbols that all differ in their low four bits
   bool have_results = false;
   bool host_results = false;
   bool ops_on_device = false;

@@ -770,8 +770,13 @@ struct OpWriterBack {
 // Near the matrix borders only gaps can reach a cell (offsets of valid M cells
 // are never negative), so walking to score 0 emits the same characters as the
 // reference's shortcut at v == 0 or h == 0.
-template <int BITS>
-__global__ void __launch_bounds__(256) wfa_backtrace_kernel(BacktraceArgs a) {
+//
+// WAVE: the records of the wave family (wfa_wave.hip): no blocks to follow,
+// the word with a cell's byte is found from its step and diagonal, and the
+// word read last is kept (its other bytes are neighbouring steps' or
+// diagonals').  Scores are then counted in steps (units of g).
+template <int BITS, bool WAVE>
+__device__ __forceinline__ void trace_pair(const BacktraceArgs& a) {
   constexpr int SPW = 64 / BITS;
   const int q = blockIdx.x * blockDim.x + threadIdx.x;
   if (q >= a.n_pairs) return;
@@ -783,10 +788,18 @@ __global__ void __launch_bounds__(256) wfa_backtrace_kernel(BacktraceArgs a) {
   // dropped at (wavefront_unialign.c:175-200), like an ends-free end cell.
   const bool zd = a.status[p] == kDevZdropped;
   if (a.status[p] != kDevCompleted && !zd) { a.ops_begin[p] = cap; return; }
-  const Penalties pen = a.pen;
+  Penalties pen = a.pen;
   const int cbeg = a.comp_begin_p ? (int)a.comp_begin_p[p] : a.comp_begin;
   int comp = a.comp_end_p ? (int)a.comp_end_p[p] : a.comp_end;
   int s = a.score[p];
+  if constexpr (WAVE) {
+    s /= pen.g;
+    pen.x /= pen.g;
+    pen.o1 /= pen.g;
+    pen.e1 /= pen.g;
+    pen.o2 /= pen.g;
+    pen.e2 /= pen.g;
+  }
   int k = tlen - plen;
   int pos = cap;
   int nx = 0, nid = 0;
@@ -829,8 +842,10 @@ __global__ void __launch_bounds__(256) wfa_backtrace_kernel(BacktraceArgs a) {
   }
   bool mark = comp == kM;  // the next operation written leads into an M cell
   uint32_t blk = a.last_block[p];
-  uint4 hdr = make_uint4(0, 0, 0, kNoBlock);
+  uint4 hdr = make_uint4(0, 0, 0, kNoBlock);  // WAVE: the units of the phases' records
   if (blk != kNoBlock && blk < a.rec_units) hdr = a.rec_arena[blk];
+  unsigned long long word_at = ~0ull;
+  uint32_t word = 0;
   OpWriterBack bw{out, pos, pos, OpChunk{}};
   while (s > 0 && !bad && !direct) {
     if (bw.p <= 0) {
@@ -838,7 +853,37 @@ __global__ void __launch_bounds__(256) wfa_backtrace_kernel(BacktraceArgs a) {
       break;
     }
     uint32_t rec;
-    if (first) {
+    if constexpr (WAVE) {
+      const int i = s - 1;
+      const int ph = (i >= a.wave_last[0] ? 1 : 0) + (i >= a.wave_last[1] ? 1 : 0) + (i >= a.wave_last[2] ? 1 : 0);
+      const int begin = ph == 0 ? 0 : ph == 1 ? a.wave_last[0] : ph == 2 ? a.wave_last[1] : a.wave_last[2];
+      const uint32_t base = ph == 0 ? hdr.x : ph == 1 ? hdr.y : ph == 2 ? hdr.z : hdr.w;
+      const int t = i - begin, kk = k - (a.wave_center - (32 << ph)), c = kk & ((1 << ph) - 1);
+      if (blk == kNoBlock || (unsigned)kk >= (64u << ph)) {
+        bad = true;
+        break;
+      }
+      const int group = ph < 3 ? t >> (2 - ph) : 2 * t + (c >> 2);
+      const int byte = ph < 3 ? ((t & ((4 >> ph) - 1)) << ph) + c : c & 3;
+      const unsigned long long at = (unsigned long long)base * 4 + (unsigned)(group * 64 + (kk >> ph));
+      if (at >= a.rec_units * 4) {
+        bad = true;
+        break;
+      }
+      if (at != word_at) {
+        word_at = at;
+        word = reinterpret_cast<const uint32_t*>(a.rec_arena)[at];
+      }
+      const uint32_t b = word >> (8 * byte);
+      if (a.wave == 5) {
+        // source 4 X, 3 D2, 2 D1, 1 I2, 0 I1 in bits 1..3; flags of I1, D1, I2, D2 from bit 4
+        rec = (4u - ((b >> 1) & 7u)) | (((b >> 4) & 15u) << 3);
+      } else {
+        // source 2 X, 1 D1, 0 I1 in bits 1..2; flags of I1 and D1 in bits 6 and 7
+        rec = 4u - (b & 6u);
+        if (a.wave == 3) rec |= ((b >> 6) & 3u) << 3;
+      }
+    } else if (first) {
       first = false;
       rec = (uint32_t)endrec;
     } else {
@@ -1009,6 +1054,15 @@ __global__ void __launch_bounds__(256) wfa_backtrace_kernel(BacktraceArgs a) {
   a.ops_begin[p] = start;
 }
 
+template <int BITS>
+__global__ void __launch_bounds__(256) wfa_backtrace_kernel(BacktraceArgs a) {
+  trace_pair<BITS, false>(a);
+}
+template <int BITS>
+__global__ void __launch_bounds__(256) wfa_wave_backtrace_kernel(BacktraceArgs a) {
+  trace_pair<BITS, true>(a);
+}
+
 __global__ void wfa_reset_kernel(Counters* c, int all) {
   if (threadIdx.x < kMaxQueues) c->queue[threadIdx.x * kQueueStride] = 0u;
   if (threadIdx.x == 0) {
@@ -1096,9 +1150,14 @@ hipError_t launch_backtrace(const BacktraceArgs& a, hipStream_t stream) {
   if (a.n_pairs <= 0) return hipSuccess;
   const int block = 256;
   const int grid = (a.n_pairs + block - 1) / block;
-  if (a.bits == 2) hipLaunchKernelGGL(wfa_backtrace_kernel<2>, dim3(grid), dim3(block), 0, stream, a);
-  else if (a.bits == 8) hipLaunchKernelGGL(wfa_backtrace_kernel<8>, dim3(grid), dim3(block), 0, stream, a);
-  else return hipErrorInvalidValue;
+  if (a.bits != 2 && a.bits != 8) return hipErrorInvalidValue;
+  if (a.wave) {
+    if (a.bits == 2) hipLaunchKernelGGL((wfa_wave_backtrace_kernel<2>), dim3(grid), dim3(block), 0, stream, a);
+    else hipLaunchKernelGGL((wfa_wave_backtrace_kernel<8>), dim3(grid), dim3(block), 0, stream, a);
+  } else {
+    if (a.bits == 2) hipLaunchKernelGGL((wfa_backtrace_kernel<2>), dim3(grid), dim3(block), 0, stream, a);
+    else hipLaunchKernelGGL((wfa_backtrace_kernel<8>), dim3(grid), dim3(block), 0, stream, a);
+  }
   return hipGetLastError();
 }
 

@@ -198,21 +198,6 @@ __device__ __forceinline__ int lcp16(const uint32_t* P, int pb, const uint32_t* 
   }
 }
 
-// The kernel arguments, reread from the kernel-argument segment where a
-// value is needed outside the step loop (the asm makes each pointer opaque,
-// so the compiler reloads instead of keeping every field in scalar
-// registers across the loop).
-using KernArgs = const __attribute__((address_space(4))) ForwardArgs*;
-__device__ __forceinline__ KernArgs args_now() {
-#if defined(__HIP_DEVICE_COMPILE__)
-  KernArgs p = (KernArgs)__builtin_amdgcn_kernarg_segment_ptr();
-  asm volatile("" : "+s"(p));
-  return p;
-#else
-  return nullptr;  // host pass of the single-source compile: never executed
-#endif
-}
-
 // Ring elements before the packed sequences in LDS (16-byte aligned): M in
 // R slots, I1 and D1 in two slots each (they are read one step later only).
 template <int R, int WCAP>

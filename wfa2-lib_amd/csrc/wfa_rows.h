@@ -18,27 +18,16 @@
 // already packed for the lane's N cells.
 #pragma once
 #include "wfa_common.h"
+#include "wfa_shapes.h"
 
 namespace wfa {
-
-// Distances between wavefronts in steps (score / g), known at compile time.
-template <int NC_, int DX_, int DO1_, int DE1_, int DO2_, int DE2_>
-struct SlotShape {
-  static constexpr int NC = NC_, DX = DX_, DO1 = DO1_, DE1 = DE1_, DO2 = DO2_, DE2 = DE2_;
-  static constexpr int RM = DX > DO1 ? DX : DO1;  // M rows kept in registers (the second gap's come from memory)
-  static constexpr int SH = NC == 5 ? 4 : 3;      // bits below the offset
-  static constexpr int kTagX = NC == 5 ? 4 : 2, kTagD2 = 3, kTagD1 = NC == 5 ? 2 : 1, kTagI2 = 1;
-  static constexpr int kGapRows = 2 * DE1 + (NC == 5 ? 2 * DE2 : 0);
-};
-using Shape2p = SlotShape<5, 4, 8, 2, 25, 1>;  // gap-affine-2p (x 4, o1 6, e1 2, o2 24, e2 1) and its multiples
-using ShapeAffine = SlotShape<3, 2, 4, 1, 0, 1>;  // gap-affine (x 4, o 6, e 2) and its multiples
 
 constexpr int kNullTagged = -(1 << 30);
 
 template <class S, int N>
 struct WaveRows {
   int m[S::RM][N];  // row i in m[i % RM]
-  int i1[S::DE1][N], d1[S::DE1][N];
+  int i1[S::DE1][N], d1[S::DE1][N];  // NC > 1
   int i2[S::DE2][N], d2[S::DE2][N];  // NC == 5
 };
 
@@ -50,29 +39,54 @@ __device__ __forceinline__ int from_upper_lane(int v) {
   return __builtin_amdgcn_update_dpp(kNullTagged, v, 0x130, 0xf, 0xf, false);  // wave_shl:1
 }
 
-// 16 symbols of a 2-bit packed sequence whose first symbol sits at bit `bit`
-// of W (v_alignbit takes the shift modulo 32 by itself).
+// First / last diagonal whose bit is set: lane l holds the bits of its N
+// diagonals kt + N * l + c.
+template <int N>
+__device__ __forceinline__ int first_diagonal(uint32_t bits, int kt) {
+  const unsigned long long bal = __ballot(bits != 0);
+  if (!bal) return INT_MAX;
+  const int l = (int)__builtin_ctzll(bal);
+  return kt + N * l + (int)__builtin_ctz((unsigned)lane_of((int)bits, l));
+}
+template <int N>
+__device__ __forceinline__ int last_diagonal(uint32_t bits, int kt) {
+  const unsigned long long bal = __ballot(bits != 0);
+  if (!bal) return INT_MIN;
+  const int l = 63 - (int)__builtin_clzll(bal);
+  return kt + N * l + 31 - (int)__builtin_clz((unsigned)lane_of((int)bits, l));
+}
+
+// The 32 bits of a packed sequence from bit `bit` of W (v_alignbit takes the
+// shift modulo 32 by itself).
 template <typename P32>
-__device__ __forceinline__ uint32_t window16(P32 W, unsigned bit) {
+__device__ __forceinline__ uint32_t window32(P32 W, unsigned bit) {
   const unsigned w = bit >> 5;
   return __builtin_amdgcn_alignbit(W[w + 1], W[w], bit);
 }
 
-// Matching symbols at the start of a 16-symbol window whose xor is x (0..16):
-// v_ffbl gives -1 for x == 0, which the shift turns into a large value.
-__device__ __forceinline__ int match_run16(uint32_t x, int cap) {
+// Matching symbols at the start of a window whose xor is x (0..32 / BITS), at
+// most cap: v_ffbl gives -1 for x == 0, which the shift turns into a large
+// value.
+template <int BITS>
+__device__ __forceinline__ int match_run(uint32_t x, int cap) {
   uint32_t f;
   asm("v_ffbl_b32 %0, %1" : "=v"(f) : "v"(x));
-  return min(min((int)(f >> 1), 16), cap);
+  return min(min((int)(f / BITS), 32 / BITS), cap);
 }
 
-// The sequences of the pair in LDS: symbol 0 of the pattern / text at bit
-// pbit / tbit of P / T.
+// The sequences of the pair, BITS bits per symbol: symbol 0 of the pattern /
+// text at bit pbit / tbit of P / T.
+template <int BITS>
 struct WaveSeqs {
   const uint32_t* P;
   const uint32_t* T;
   unsigned pbit, tbit;
   int plen, tlen;
+  static constexpr int kSpan = 32 / BITS;  // symbols per window
+  // matching symbols (at most cap) of the window at text offset h of diagonal h - v
+  __device__ __forceinline__ int run(int h, int v, int cap) const {
+    return match_run<BITS>(window32(T, tbit + (unsigned)(BITS * h)) ^ window32(P, pbit + (unsigned)(BITS * v)), cap);
+  }
 };
 
 // What a step tells about its cells.
@@ -81,7 +95,9 @@ struct StepCells {
   int h[N];        // extended M offset (meaningless where !ok)
   bool ok[N];      // valid M cell
   bool oob[N];     // a path reaches the cell, but outside the matrix
-  uint32_t rec[(N + 3) / 4];  // record bytes
+  // Record bytes, shifted in from the top: after four cells (of one step, or
+  // with N < 4 of consecutive steps) a word holds them in order.
+  uint32_t rec[(N + 3) / 4];
 };
 
 // The cells of one step from their source rows (tagged values of the lane's N
@@ -90,15 +106,15 @@ struct StepCells {
 // rows replace i1, d1, i2, d2; the new M row goes to m (which may be mo).
 // wavefront_compute_affine.c:44-86, wavefront_compute_affine2p.c:45-106,
 // wavefront_extend_kernels.c:68-123.
-template <class S, int N>
+template <class S, int N, int BITS>
 __device__ __forceinline__ void wave_cells(const int* mx, const int* mo, int* i1, int* d1, const int* mo2, int* i2,
-                                           int* d2, int* m, int k0, const WaveSeqs& q, StepCells<N>& out) {
-  constexpr int SH = S::SH, ONE = 1 << SH;
+                                           int* d2, int* m, int k0, const WaveSeqs<BITS>& q, StepCells<N>& out) {
+  constexpr int SH = S::SH, ONE = 1 << SH, SPAN = WaveSeqs<BITS>::kSpan;
   int a1[N], b1[N], a2[N], b2[N];
 #pragma unroll
   for (int c = 0; c < N; ++c) {
-    a1[c] = max(mo[c], i1[c]);
-    b1[c] = max(mo[c], d1[c]);
+    a1[c] = S::NC == 1 ? mo[c] : max(mo[c], i1[c]);
+    b1[c] = S::NC == 1 ? mo[c] : max(mo[c], d1[c]);
     if constexpr (S::NC == 5) {
       a2[c] = max(mo2[c], i2[c]);
       b2[c] = max(mo2[c], d2[c]);
@@ -116,47 +132,50 @@ __device__ __forceinline__ void wave_cells(const int* mx, const int* mo, int* i1
   for (int c = 0; c < N; ++c) {
     const int ins1 = (c ? a1[c > 0 ? c - 1 : 0] : a1l) + ONE;
     const int del1 = (c + 1 < N ? b1[c + 1 < N ? c + 1 : 0] : b1u) + 2 * S::kTagD1;
-    const int x = mx[c] + ONE + 2 * S::kTagX;
-    int best = max(max(ins1, del1), x);
+    int best = max(ins1, del1);
+    if constexpr (S::kMismatch) best = max(best, mx[c] + ONE + 2 * S::kTagX);
     int ins2 = 0, del2 = 0;
     if constexpr (S::NC == 5) {
       ins2 = (c ? a2[c > 0 ? c - 1 : 0] : a2l) + ONE + 2 * S::kTagI2;
       del2 = (c + 1 < N ? b2[c + 1 < N ? c + 1 : 0] : b2u) + 2 * S::kTagD2;
       best = max(max(best, ins2), del2);
     }
-    i1[c] = (ins1 & ~(ONE - 1)) | 1;
-    d1[c] = (del1 & ~(ONE - 1)) | 1;
+    if constexpr (S::NC > 1) {
+      i1[c] = (ins1 & ~(ONE - 1)) | 1;
+      d1[c] = (del1 & ~(ONE - 1)) | 1;
+    }
     if constexpr (S::NC == 5) {
       i2[c] = (ins2 & ~(ONE - 1)) | 1;
       d2[c] = (del2 & ~(ONE - 1)) | 1;
     }
     // record byte: NC == 5: source and flag of the best (4 bits), then the
     // flags of I1, D1, I2, D2; NC == 3: 6 bits of the best (source in bits
-    // 1..2), then the flags of I1 and D1
+    // 1..2), then the flags of I1 and D1; NC == 1: 8 bits of the best
     uint32_t& acc = out.rec[c / 4];
     if constexpr (S::NC == 5) {
-      acc = __builtin_amdgcn_alignbit((uint32_t)best, c % 4 ? acc : 0u, 4);
+      acc = __builtin_amdgcn_alignbit((uint32_t)best, acc, 4);
       acc = __builtin_amdgcn_alignbit((uint32_t)ins1, acc, 1);
       acc = __builtin_amdgcn_alignbit((uint32_t)del1, acc, 1);
       acc = __builtin_amdgcn_alignbit((uint32_t)ins2, acc, 1);
       acc = __builtin_amdgcn_alignbit((uint32_t)del2, acc, 1);
-    } else {
-      acc = __builtin_amdgcn_alignbit((uint32_t)best, c % 4 ? acc : 0u, 6);
+    } else if constexpr (S::NC == 3) {
+      acc = __builtin_amdgcn_alignbit((uint32_t)best, acc, 6);
       acc = __builtin_amdgcn_alignbit((uint32_t)ins1, acc, 1);
       acc = __builtin_amdgcn_alignbit((uint32_t)del1, acc, 1);
+    } else {
+      acc = __builtin_amdgcn_alignbit((uint32_t)best, acc, 8);
     }
     // null-after-max, then one 16-symbol window of the extension
     const int off = best >> SH, k = k0 + c, v = off - k;
     const bool ok = ((unsigned)off <= (unsigned)q.tlen) & ((unsigned)v <= (unsigned)q.plen);
     const int o = ok ? off : 0, vv = ok ? v : 0;
     const int r = min(q.tlen - o, q.plen - vv);
-    const uint32_t d = window16(q.T, q.tbit + 2u * (unsigned)o) ^ window16(q.P, q.pbit + 2u * (unsigned)vv);
-    const int n = match_run16(d, r);
+    const int n = q.run(o, vv, r);
     out.ok[c] = ok;
     out.oob[c] = !ok & (best >= 0);
     out.h[c] = o + n;
     rem[c] = r - n;
-    full |= (ok & (n == 16) & (r > 16)) ? 1u << c : 0u;
+    full |= (ok & (n == SPAN) & (r > SPAN)) ? 1u << c : 0u;
   }
   // long runs (rare away from the main diagonal): more windows, cell by cell
   if (__ballot(full != 0)) {
@@ -166,12 +185,10 @@ __device__ __forceinline__ void wave_cells(const int* mx, const int* mo, int* i1
       if (__ballot(more)) {
         int h = out.h[c], r = rem[c];
         while (more) {
-          const uint32_t d = window16(q.T, q.tbit + 2u * (unsigned)h) ^
-                             window16(q.P, q.pbit + 2u * (unsigned)(h - (k0 + c)));
-          const int n = match_run16(d, r);
+          const int n = q.run(h, h - (k0 + c), r);
           h += n;
           r -= n;
-          more = (n == 16) & (r > 0);
+          more = (n == SPAN) & (r > 0);
         }
         out.h[c] = h;
       }
@@ -183,12 +200,12 @@ __device__ __forceinline__ void wave_cells(const int* mx, const int* mo, int* i1
 
 // Step i (compile-time phase PH = i mod the unroll) over rows in registers;
 // o2: row i - DO2, tagged (NC == 5).  The oldest rows are replaced by the new.
-template <class S, int N, int PH>
-__device__ __forceinline__ void wave_step(WaveRows<S, N>& w, const int* o2, int k0, const WaveSeqs& q,
+template <class S, int N, int PH, int BITS>
+__device__ __forceinline__ void wave_step(WaveRows<S, N>& w, const int* o2, int k0, const WaveSeqs<BITS>& q,
                                           StepCells<N>& out) {
-  constexpr int rx = (PH + 8 * S::RM - S::DX) % S::RM, ro = (PH + 8 * S::RM - S::DO1) % S::RM, rn = PH % S::RM;
+  constexpr int rx = (PH + 8 * S::RM - (S::kMismatch ? S::DX : 0)) % S::RM, ro = (PH + 8 * S::RM - S::DO1) % S::RM, rn = PH % S::RM;
   constexpr int g1 = PH % S::DE1, g2 = PH % S::DE2;
-  wave_cells<S, N>(w.m[rx], w.m[ro], w.i1[g1], w.d1[g1], o2, w.i2[g2], w.d2[g2], w.m[rn], k0, q, out);
+  wave_cells<S, N, BITS>(w.m[rx], w.m[ro], w.i1[g1], w.d1[g1], o2, w.i2[g2], w.d2[g2], w.m[rn], k0, q, out);
 }
 
 }  // namespace wfa

@@ -84,23 +84,6 @@ __device__ __forceinline__ void store_row(int* p, const int* r) {
   for (int c = 0; c < N; c += 4) *reinterpret_cast<int4*>(p + c) = make_int4(r[c], r[c + 1], r[c + 2], r[c + 3]);
 }
 
-// First / last diagonal whose bit is set: lane l holds the bits of its N
-// diagonals kt + N * l + c.
-template <int N>
-__device__ __forceinline__ int first_diagonal(uint32_t bits, int kt) {
-  const unsigned long long bal = __ballot(bits != 0);
-  if (!bal) return INT_MAX;
-  const int l = (int)__builtin_ctzll(bal);
-  return kt + N * l + (int)__builtin_ctz((unsigned)lane_of((int)bits, l));
-}
-template <int N>
-__device__ __forceinline__ int last_diagonal(uint32_t bits, int kt) {
-  const unsigned long long bal = __ballot(bits != 0);
-  if (!bal) return INT_MIN;
-  const int l = 63 - (int)__builtin_clzll(bal);
-  return kt + N * l + 31 - (int)__builtin_clz((unsigned)lane_of((int)bits, l));
-}
-
 // One block of T steps [ib, ib + T) of the active pairs: blockIdx.y the pair,
 // blockIdx.x a group of kTileWaves tiles.
 template <class S, bool REC>
@@ -141,7 +124,7 @@ __global__ void __launch_bounds__(64 * kTileWaves) wfa_tile_kernel(TileArgs a) {
   if (tile >= tiles) return;
   const int first = left + 4 * (quads * tile / tiles);  // the tile's own diagonals [first, past)
   const int past = left + 4 * (quads * (tile + 1) / tiles);
-  const WaveSeqs q{reinterpret_cast<const uint32_t*>(seqP), reinterpret_cast<const uint32_t*>(seqT),
+  const WaveSeqs<2> q{reinterpret_cast<const uint32_t*>(seqP), reinterpret_cast<const uint32_t*>(seqT),
                    2u * (unsigned)(ppos & 31), 2u * (unsigned)(tpos & 31), plen, tlen};
   const int kt = first - H, k0 = kt + N * lane;
   const bool own = k0 >= first && k0 < past;
@@ -215,7 +198,8 @@ __global__ void __launch_bounds__(64 * kTileWaves) wfa_tile_kernel(TileArgs a) {
       if (t + 1 < T) load(o2n, mrow(so2), i + 1 - S::DO2 >= ib - T ? in1 : in2);  // one step ahead: a row of an earlier block
     }
     StepCells<N> cell;
-    wave_step<S, N, PH>(w, o2, k0, q, cell);
+    for (uint32_t& r : cell.rec) r = 0;
+    wave_step<S, N, PH, 2>(w, o2, k0, q, cell);
     if constexpr (REC) {
       if (rec_own) {
 #pragma unroll
@@ -556,11 +540,12 @@ __global__ void __launch_bounds__(64 * kStepWaves) tile_step_kernel(StepArgs a, 
       load_gap(d2, kD2, i - S::DE2, e2);
     }
     const long long ppos = a.pat_pos[job], tpos = a.txt_pos[job];
-    const WaveSeqs q{reinterpret_cast<const uint32_t*>(a.words + (ppos >> 5)),
+    const WaveSeqs<2> q{reinterpret_cast<const uint32_t*>(a.words + (ppos >> 5)),
                      reinterpret_cast<const uint32_t*>(a.words + (tpos >> 5)), 2u * (unsigned)(ppos & 31),
                      2u * (unsigned)(tpos & 31), plen, tlen};
     StepCells<N> cell;
-    wave_cells<S, N>(mx, mo, i1, d1, mo2, i2, d2, m, k0, q, cell);
+    for (uint32_t& r : cell.rec) r = 0;
+    wave_cells<S, N, 2>(mx, mo, i1, d1, mo2, i2, d2, m, k0, q, cell);
     if (own) {
       store_row<N>(st + (long long)R::m(i) * pitch, m);
       store_row<N>(st + (long long)R::gap(kI1, i) * pitch, i1);
@@ -813,10 +798,8 @@ __global__ void __launch_bounds__(64) tile_backtrace_kernel(TileTraceArgs a) {
       for (;;) {
         const int rem = min(plen - v, tlen - h);
         const int at = min(16 * lane, rem);
-        uint32_t x;
-        if constexpr (LDS) x = window16(sT, tbit + 2u * (unsigned)(h + at)) ^ window16(sP, pbit + 2u * (unsigned)(v + at));
-        else x = window16(Q, tbit + 2u * (unsigned)(h + at)) ^ window16(P, pbit + 2u * (unsigned)(v + at));
-        const int m1 = match_run16(x, rem - at);
+        const WaveSeqs<2> q{LDS ? sP : P, LDS ? sT : Q, pbit, tbit, plen, tlen};
+        const int m1 = q.run(h + at, v + at, rem - at);
         const unsigned long long stop = __ballot(m1 < 16);
         const int f = stop ? (int)__builtin_ctzll(stop) : 0;
         const int m = stop ? 16 * f + lane_of(m1, f) : 1024;

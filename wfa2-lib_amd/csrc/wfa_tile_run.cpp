@@ -6,6 +6,7 @@
 #include <cstring>
 
 #include "wfa_internal.h"
+#include "wfa_shapes.h"
 
 namespace wfa_host {
 namespace {
@@ -19,74 +20,51 @@ constexpr double kTileRecordShareOfL2 = 0.5;
 // Blocks between two looks at the number of jobs left.
 constexpr int kTileFirstChunk = 4, kTileChunk = 16;
 
-struct Range {
-  int lo = 1, hi = -1;
-  bool valid() const { return lo <= hi; }
-};
+bool put(DevBuf& d, const void* from, size_t bytes, hipStream_t st) {
+  return d.ensure(bytes) && hip_ok(hipMemcpyAsync(d.p, from, bytes, hipMemcpyHostToDevice, st), "range table") &&
+         hip_ok(hipStreamSynchronize(st), "range table");
+}
 
 }  // namespace
 
-// The ranges of every step from 0 to at least `steps`, which are the same for
-// all pairs until an end cell leaves the matrix
-// (wavefront_compute_limits_input, wavefront_compute.c:40-86, with every
-// range as wide as its sources make it).  Returns false on an allocation or
-// copy failure.
+// The table of at least `steps` steps for a tile shape: per step the range of
+// M (lo > hi: none), the hull of the ranges so far, and the diagonal-steps up
+// to it.
 bool tile_table(Engine* e, int shape, int steps) {
   Engine::TileState& t = e->tile;
   if (t.shape == shape && (int)t.lo.size() >= steps) return true;
-  const wfa::TileGeometry g = wfa::tile_geometry(shape);
   steps = std::max(steps, 4096);
   if (t.shape == shape) steps = std::max(steps, 2 * (int)t.lo.size());
-  t.shape = shape;
+  t.shape = 0;
+  const wfa::TileGeometry g = wfa::tile_geometry(shape);
+  std::vector<wfa::StepRanges> rows((size_t)steps + 1);
+  rows[0].c[wfa::kM].lo = rows[0].c[wfa::kM].hi = 0;
+  std::vector<int> m_range(2 * (size_t)steps);
+  std::vector<long long> dsteps((size_t)steps + 1, 0);
   t.lo.assign(steps, 0);
   t.hi.assign(steps, 0);
-  t.m_range.assign(2 * (size_t)steps, 0);
-  t.dsteps.assign((size_t)steps + 1, 0);
-  const bool two = g.do2 > 0;
-  // row r at index r + 1 (row -1: score 0, M = [0, 0])
-  std::vector<Range> M(steps + 1), I1(steps + 1), D1(steps + 1), I2(steps + 1), D2(steps + 1);
-  M[0] = Range{0, 0};
-  int hull_lo = 0, hull_hi = 0;
+  int lo = 0, hi = 0;
   for (int i = 0; i < steps; ++i) {
-    auto at = [&](const std::vector<Range>& v, int back) {
-      const int r = i + 1 - back;
-      return r >= 0 ? v[r] : Range{};
-    };
-    const Range mx = at(M, g.dx), mo = at(M, g.do1), i1 = at(I1, g.de1), d1 = at(D1, g.de1);
-    const Range mo2 = two ? at(M, g.do2) : Range{}, i2 = two ? at(I2, g.de2) : Range{},
-                d2 = two ? at(D2, g.de2) : Range{};
-    Range m;
-    auto add = [](Range& r, const Range& s, int d) {
-      if (!s.valid()) return;
-      if (!r.valid()) { r = Range{s.lo + d, s.hi + d}; return; }
-      r.lo = std::min(r.lo, s.lo + d);
-      r.hi = std::max(r.hi, s.hi + d);
-    };
-    add(I1[i + 1], mo, 1); add(I1[i + 1], i1, 1);
-    add(D1[i + 1], mo, -1); add(D1[i + 1], d1, -1);
-    add(I2[i + 1], mo2, 1); add(I2[i + 1], i2, 1);
-    add(D2[i + 1], mo2, -1); add(D2[i + 1], d2, -1);
-    // limits: each source contributes its range shifted as its gap moves it;
-    // an opening contributes both ways
-    add(m, mx, 0); add(m, I1[i + 1], 0); add(m, D1[i + 1], 0); add(m, I2[i + 1], 0); add(m, D2[i + 1], 0);
-    M[i + 1] = m;
-    t.dsteps[i + 1] = t.dsteps[i] + (m.valid() ? m.hi - m.lo + 1 : 0);
+    rows[i + 1] = wfa::next_ranges(g.do2 ? 5 : 3, g.dx, g.do1, g.de1, g.do2, g.de2, [&](int back, int c) {
+      return i + 1 - back >= 0 ? rows[i + 1 - back].c[c] : wfa::StepRange{};
+    });
+    const wfa::StepRange m = rows[i + 1].c[wfa::kM];
+    dsteps[i + 1] = dsteps[i] + (m.valid() ? m.hi - m.lo + 1 : 0);
     if (m.valid()) {
-      hull_lo = std::min(hull_lo, m.lo);
-      hull_hi = std::max(hull_hi, m.hi);
+      lo = std::min(lo, m.lo);
+      hi = std::max(hi, m.hi);
     }
-    t.lo[i] = hull_lo;
-    t.hi[i] = hull_hi;
-    t.m_range[2 * (size_t)i] = m.lo;
-    t.m_range[2 * (size_t)i + 1] = m.hi;
+    t.lo[i] = lo;
+    t.hi[i] = hi;
+    m_range[2 * (size_t)i] = m.lo;
+    m_range[2 * (size_t)i + 1] = m.hi;
   }
   hipStream_t st = e->stream;
-  return t.d_range.ensure(t.m_range.size() * sizeof(int)) && t.d_dsteps.ensure(t.dsteps.size() * sizeof(long long)) &&
-         hip_ok(hipMemcpyAsync(t.d_range.p, t.m_range.data(), t.m_range.size() * sizeof(int), hipMemcpyHostToDevice, st),
-                "tile table") &&
-         hip_ok(hipMemcpyAsync(t.d_dsteps.p, t.dsteps.data(), t.dsteps.size() * sizeof(long long),
-                               hipMemcpyHostToDevice, st), "tile table") &&
-         hip_ok(hipStreamSynchronize(st), "tile table");
+  if (!put(t.d_range, m_range.data(), m_range.size() * sizeof(int), st) ||
+      !put(t.d_dsteps, dsteps.data(), dsteps.size() * sizeof(long long), st))
+    return false;
+  t.shape = shape;
+  return true;
 }
 
 // Whether a job of these lengths can run in tiles: its sequences in LDS.

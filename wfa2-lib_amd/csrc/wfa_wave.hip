@@ -1,0 +1,577 @@
+// Short pairs: one wave per pair, its wavefronts in registers.
+//
+// A pair's diagonals are spread over the 64 lanes of one wave, N neighbours
+// per lane (wfa_rows.h), with the score-0 diagonals in the middle.  Rows of
+// the last steps sit in registers (moved along at each step), a gap source is a
+// neighbouring register or a DPP shift,
+// and LDS holds nothing but the two packed sequences: the step has no ring,
+// no clamped index, no per-source range and no LDS round trip but the
+// extension's.  N starts at the least that holds the score-0 diagonals and
+// doubles as the wavefront outgrows the wave (1 up to 64 diagonals, then 2, 4,
+// 8); the step at which it does is the same for every pair.
+//
+// Ranges need no bookkeeping either: until a cell leaves the matrix nothing
+// is trimmed (wavefront_compute.c:579-613) and the widths are tabulated; after
+// that the limits are read off the cells, as in the end tiles of wfa_tile.hip.
+//
+// Records: a word per lane holds four cells (of one step, or of 4 / N
+// consecutive ones), so a wave writes 256 contiguous bytes per four cells of
+// its lanes, and the place of every record byte follows from the step and the
+// diagonal: the backtrace reads no headers.
+#include <climits>
+
+#include "wfa_rows.h"
+#include "wfa_wave.h"
+
+namespace wfa {
+namespace {
+
+// One copy of a shape's table in device memory, one for the host.
+template <class S>
+__device__ const WaveTable wave_table = make_wave_table<S>();
+template <class S>
+constexpr WaveTable host_wave_table = make_wave_table<S>();
+
+// Everything of one pair that outlives a step.
+struct WavePair {
+  int plen, tlen, kend;
+  int i;            // steps done: the last row is i - 1
+  int status;       // 1: running
+  int dev;          // exact minus tabulated widths
+  int slot;         // ring row about to be written (a second gap)
+  bool exact;
+  uint32_t hist_m, hist_gap;  // exact: components with a valid cell in the last steps (WaveTable)
+  int end_k, end_off;
+  uint32_t base[kWavePhases];  // record units of each phase
+};
+
+// With a second gap the M rows of the last 25 steps are needed: they sit in
+// LDS, 16 bits a cell (offset << 4; at most 1,024 symbols), a row holding the
+// diagonals of the widest phase in order, so that a phase reads and writes
+// its lanes' cells in one access each and a change of phase moves nothing.
+constexpr int kRingRows = 26;
+constexpr int kRingNull = -32768;
+template <int NMAX>
+struct WaveRing {
+  int16_t* rows;
+  static constexpr int kPitch = 64 * NMAX;
+  static constexpr int kBytes = kRingRows * kPitch * 2;
+  __device__ __forceinline__ void clear() const {
+    const uint32_t v = 0x80008000u;
+    for (int x = threadIdx.x & 63; x < kBytes / 16; x += 64) reinterpret_cast<uint4*>(rows)[x] = make_uint4(v, v, v, v);
+  }
+  // the lane's N cells of the row `back` steps ago (at: this lane's first
+  // cell in a row; slot: the row about to be written)
+  template <int N>
+  __device__ __forceinline__ void read(int* r, int at, int slot, int back) const {
+    int x = slot - back;
+    if (x < 0) x += kRingRows;
+    const int16_t* p = rows + x * kPitch + at;
+    if constexpr (N == 1) {
+      r[0] = p[0];
+    } else {
+#pragma unroll
+      for (int c = 0; c < N; c += 2) {
+        const int v = *reinterpret_cast<const int*>(p + c);
+        r[c] = (int)(int16_t)v;
+        r[c + 1] = v >> 16;
+      }
+    }
+  }
+  template <int N>
+  __device__ __forceinline__ void write(const int* m, int at, int slot) const {
+    int16_t* p = rows + slot * kPitch + at;
+    if constexpr (N == 1) {
+      p[0] = (int16_t)max(m[0], kRingNull);
+    } else {
+#pragma unroll
+      for (int c = 0; c < N; c += 2)
+        *reinterpret_cast<uint32_t*>(p + c) =
+            ((uint32_t)max(m[c], kRingNull) & 0xFFFFu) | ((uint32_t)max(m[c + 1], kRingNull) << 16);
+    }
+  }
+};
+
+struct WaveChunk {  // record chunk of this wave (16-byte units)
+  uint32_t cur, end;
+};
+
+// Room for `units` of records in the wave's chunk, or a new chunk.
+__device__ __forceinline__ bool reserve_records(WaveChunk& ch, uint32_t units) {
+  if (ch.cur + units <= ch.end) return true;
+  KernArgs A = args_now();
+  const uint32_t want = units > kChunkUnits ? units : kChunkUnits;
+  unsigned long long b = 0;
+  if ((threadIdx.x & 63) == 0) b = atomicAdd(A->rec_top, (unsigned long long)want);
+  const unsigned blo = (unsigned)lane_of((int)(unsigned)(b & 0xFFFFFFFFull), 0);
+  const unsigned bhi = (unsigned)lane_of((int)(unsigned)(b >> 32), 0);
+  if (bhi != 0 || (unsigned long long)blo + want > A->rec_units) {
+    ch.cur = ch.end = 0;
+    return false;
+  }
+  ch.cur = blo;
+  ch.end = blo + want;
+  return true;
+}
+
+// The steps of one phase (N diagonals per lane): from row p.i up to the last
+// step whose wavefront fits, or the end of the pair.
+template <class S, int N, int NMAX, int BITS, bool REC, bool EF>
+__device__ __forceinline__ void wave_phase(WavePair& p, WaveChunk& ch, WaveRows<S, N>& w, const WaveSeqs<BITS>& q,
+                                           const WaveRing<NMAX>& ring) {
+  KernArgs A = args_now();
+  static_assert(S::DE1 <= 2 && S::DE2 == 1 && S::DO2 < kRingRows, "gap rows");
+  constexpr int PH = N == 1 ? 0 : N == 2 ? 1 : N == 4 ? 2 : 3;
+  constexpr int G = N < 4 ? 4 / N : 1;  // steps per record word
+  const int lane = threadIdx.x & 63;
+  const int kt = (EF ? A->wave.center : 0) - 32 * N, k0 = kt + N * lane;
+  const int first = PH ? A->wave.last[PH ? PH - 1 : 0] : 0, last = A->wave.last[PH];
+  const int pef = EF ? A->pef : 0, tef = EF ? A->tef : 0;
+  uint32_t* rec = nullptr;
+  if constexpr (REC) {
+    const uint32_t units = (uint32_t)((last - first + G - 1) / G * (N > 4 ? N / 4 : 1)) * 16u;
+    if (!reserve_records(ch, units)) {
+      p.status = kDevArenaFull;
+      return;
+    }
+    p.base[PH] = ch.cur;
+    rec = reinterpret_cast<uint32_t*>(A->rec_arena + ch.cur) + lane;
+  }
+  uint32_t endm = 0;  // the lane's cell on the end diagonal
+#pragma unroll
+  for (int c = 0; c < N; ++c) endm |= (k0 + c == p.kend) ? 1u << c : 0u;
+  StepCells<N> cell;
+#pragma unroll
+  for (uint32_t& r : cell.rec) r = 0;
+  int i = p.i;
+  while (i < last) {
+    // w.m[r]: row i - 1 - r, and so the gap rows (of the last DE1 steps)
+    int m[N];
+    constexpr int og = S::DE1 - 1;
+    if constexpr (S::NC == 5) {
+      int mx[N], mo[N], mo2[N];
+      const int at = k0 - (kt - 32 * (NMAX - N));
+      ring.template read<N>(mx, at, p.slot, S::DX);
+      ring.template read<N>(mo, at, p.slot, S::DO1);
+      ring.template read<N>(mo2, at, p.slot, S::DO2);
+      wave_cells<S, N, BITS>(mx, mo, w.i1[og], w.d1[og], mo2, w.i2[0], w.d2[0], m, k0, q, cell);
+      ring.template write<N>(m, at, p.slot);
+      p.slot = p.slot + 1 == kRingRows ? 0 : p.slot + 1;
+    } else {
+      wave_cells<S, N, BITS>(w.m[S::kMismatch ? S::DX - 1 : 0], w.m[S::DO1 - 1], w.i1[og], w.d1[og], nullptr, nullptr,
+                             nullptr, m, k0, q, cell);
+#pragma unroll
+      for (int r = S::RM - 1; r > 0; --r)
+#pragma unroll
+        for (int c = 0; c < N; ++c) w.m[r][c] = w.m[r - 1][c];
+#pragma unroll
+      for (int c = 0; c < N; ++c) w.m[0][c] = m[c];
+    }
+    if constexpr (S::NC > 1 && S::DE1 == 2) {
+#pragma unroll
+      for (int c = 0; c < N; ++c) {
+        const int ni = w.i1[1][c], nd = w.d1[1][c];
+        w.i1[1][c] = w.i1[0][c];
+        w.d1[1][c] = w.d1[0][c];
+        w.i1[0][c] = ni;
+        w.d1[0][c] = nd;
+      }
+    }
+    ++i;
+    if constexpr (REC) {
+      if (G == 1 || ((i - first) & (G - 1)) == 0) {
+#pragma unroll
+        for (int c = 0; c < (N + 3) / 4; ++c) rec[64 * c] = cell.rec[c];
+        rec += 64 * ((N + 3) / 4);
+      }
+    }
+    bool out = false, fin = false;
+#pragma unroll
+    for (int c = 0; c < N; ++c) {
+      out |= cell.oob[c];
+      if constexpr (EF) fin |= cell.ok[c] & endsfree_done(cell.h[c], k0 + c, p.plen, p.tlen, pef, tef);
+      else fin |= cell.ok[c] & (cell.h[c] >= p.tlen) & (((endm >> c) & 1u) != 0);
+    }
+    const unsigned long long bfin = __ballot(fin);
+    if (__ballot(out) || p.exact) {
+      // limits and trimming from the cells
+      KernArgs B = args_now();
+      if (!p.exact) {
+        p.exact = true;
+        p.hist_m = wave_table<S>.hist_m[i - 1];
+        p.hist_gap = wave_table<S>.hist_gap[i - 1];
+      }
+      uint32_t okm = 0, reach = 0;
+#pragma unroll
+      for (int c = 0; c < N; ++c) {
+        okm |= cell.ok[c] ? 1u << c : 0u;
+        reach |= (cell.ok[c] | cell.oob[c]) ? 1u << c : 0u;
+      }
+      int lo = first_diagonal<N>(reach, kt), hi = last_diagonal<N>(reach, kt);
+      const bool some = lo <= hi;
+      if (B->pen.metric > kEdit) {
+        // a null source still contributes the limits (1, -1), shifted as its
+        // gap moves it (wavefront_compute.c:40-86)
+        auto null_m = [&](int back) { return !((p.hist_m >> (back - 1)) & 1u); };
+        auto null_gap = [&](int c, int back) { return !((p.hist_gap >> (4 * (back - 1) + c - kI1)) & 1u); };
+        if (null_m(S::DX > 0 ? S::DX : 1)) { lo = min(lo, 1); hi = max(hi, -1); }
+        if (null_m(S::DO1)) { lo = min(lo, 0); hi = max(hi, 0); }
+        if constexpr (S::NC > 1) {
+          if (null_gap(kI1, S::DE1)) { lo = min(lo, 2); hi = max(hi, 0); }
+          if (null_gap(kD1, S::DE1)) { lo = min(lo, 0); hi = max(hi, -2); }
+        }
+        if constexpr (S::NC == 5) {
+          if (null_m(S::DO2)) { lo = min(lo, 0); hi = max(hi, 0); }
+          if (null_gap(kI2, S::DE2)) { lo = min(lo, 2); hi = max(hi, 0); }
+          if (null_gap(kD2, S::DE2)) { lo = min(lo, 0); hi = max(hi, -2); }
+        }
+      }
+      const int tlo = wave_table<S>.lo[i - 1], thi = wave_table<S>.hi[i - 1];
+      p.dev += (some ? hi - lo + 1 : 0) - (tlo <= thi ? thi - tlo + 1 + (EF ? B->pbf + B->tbf : 0) : 0);
+      p.hist_m = (p.hist_m << 1) | (__ballot(okm != 0) ? 1u : 0u);
+      p.hist_gap <<= 4;
+      if constexpr (S::NC > 1) {
+        auto trim = [&](int* g, int comp) {
+          uint32_t vm = 0;
+#pragma unroll
+          for (int c = 0; c < N; ++c) vm |= in_bounds(g[c] >> S::SH, k0 + c, p.plen, p.tlen) ? 1u << c : 0u;
+          const int f = first_diagonal<N>(vm, kt), l = last_diagonal<N>(vm, kt);
+#pragma unroll
+          for (int c = 0; c < N; ++c) g[c] = (k0 + c < f || k0 + c > l) ? kNullTagged : g[c];
+          p.hist_gap |= f <= l ? 1u << (comp - kI1) : 0u;
+        };
+        trim(w.i1[0], kI1);
+        trim(w.d1[0], kD1);
+        if constexpr (S::NC == 5) {
+          trim(w.i2[0], kI2);
+          trim(w.d2[0], kD2);
+        }
+      }
+    }
+    if (bfin) {
+      if constexpr (EF) {
+        uint32_t fm = 0;
+        int off = 0;
+#pragma unroll
+        for (int c = N - 1; c >= 0; --c) {
+          const bool f = cell.ok[c] & endsfree_done(cell.h[c], k0 + c, p.plen, p.tlen, pef, tef);
+          fm |= f ? 1u << c : 0u;
+          off = f ? cell.h[c] : off;
+        }
+        p.end_k = first_diagonal<N>(fm, kt);
+        p.end_off = lane_of(off, (int)__builtin_ctzll(bfin));
+      }
+      p.status = kDevCompleted;
+      break;
+    }
+  }
+  if constexpr (REC && G > 1) {
+    // the started record word, its steps moved down to their places
+    const int rest = (i - first) & (G - 1);
+    if (rest) rec[0] = cell.rec[0] >> (8 * N * (G - rest));
+  }
+  p.i = i;
+  if constexpr (REC) ch.cur = p.base[PH] + (uint32_t)((i - first + G - 1) / G * (N > 4 ? N / 4 : 1)) * 16u;
+}
+
+// Rows of N diagonals per lane spread over 2N per lane: the lane's first N
+// come from lane 2l - 32, its last N from lane 2l - 31.
+template <class S, int N>
+__device__ __forceinline__ void widen(const WaveRows<S, N>& w, WaveRows<S, 2 * N>& x) {
+  const int lane = threadIdx.x & 63;
+  const bool in = lane >= 16 && lane < 48;
+  const int from = 4 * (2 * lane - 32);
+  auto spread = [&](const int* a, int* b) {
+#pragma unroll
+    for (int c = 0; c < N; ++c) {
+      const int u = __builtin_amdgcn_ds_bpermute(from, a[c]), v = __builtin_amdgcn_ds_bpermute(from + 4, a[c]);
+      b[c] = in ? u : kNullTagged;
+      b[N + c] = in ? v : kNullTagged;
+    }
+  };
+  if constexpr (S::NC < 5) {
+#pragma unroll
+    for (int r = 0; r < S::RM; ++r) spread(w.m[r], x.m[r]);
+  } else {
+    spread(w.i2[0], x.i2[0]);
+    spread(w.d2[0], x.d2[0]);
+  }
+  if constexpr (S::NC > 1) {
+#pragma unroll
+    for (int r = 0; r < S::DE1; ++r) {
+      spread(w.i1[r], x.i1[r]);
+      spread(w.d1[r], x.d1[r]);
+    }
+  }
+}
+
+// Row -1 (score 0): offset 0 at diagonal 0, or, ends-free, the free
+// beginnings (wavefront_aligner.c:252-307), each extended; every other row
+// NULL.  Returns whether the alignment ends there.
+template <class S, int N, int NMAX, int BITS, bool EF>
+__device__ __forceinline__ bool wave_start(WavePair& p, WaveRows<S, N>& w, const WaveSeqs<BITS>& q,
+                                           const WaveRing<NMAX>& ring) {
+  KernArgs A = args_now();
+  const int lane = threadIdx.x & 63;
+  const int kt = (EF ? A->wave.center : 0) - 32 * N, k0 = kt + N * lane;
+#pragma unroll
+  for (int r = 0; r < S::RM; ++r)
+#pragma unroll
+    for (int c = 0; c < N; ++c) w.m[r][c] = kNullTagged;
+  if constexpr (S::NC > 1) {
+#pragma unroll
+    for (int r = 0; r < S::DE1; ++r)
+#pragma unroll
+      for (int c = 0; c < N; ++c) w.i1[r][c] = w.d1[r][c] = kNullTagged;
+  }
+  if constexpr (S::NC == 5) {
+#pragma unroll
+    for (int c = 0; c < N; ++c) w.i2[0][c] = w.d2[0][c] = kNullTagged;
+    ring.clear();
+    wave_sync();
+  }
+  int m0[N];
+  const int lo = EF ? -A->pbf : 0, hi = EF ? A->tbf : 0;
+  uint32_t done = 0;
+  int off = 0;
+#pragma unroll
+  for (int c = N - 1; c >= 0; --c) {
+    const int k = k0 + c;
+    int h = k > 0 ? k : 0;
+    bool more = k >= lo && k <= hi;
+    const bool on = more;
+    while (more) {
+      const int r = min(p.tlen - h, p.plen - (h - k));
+      const int n = r > 0 ? q.run(h, h - k, r) : 0;
+      h += n;
+      more = (n == WaveSeqs<BITS>::kSpan) & (r > n);
+    }
+    m0[c] = on ? h << S::SH : kNullTagged;
+    const bool fin = on && (EF ? endsfree_done(h, k, p.plen, p.tlen, A->pef, A->tef) : (k == p.kend && h >= p.tlen));
+    done |= fin ? 1u << c : 0u;
+    off = fin ? h : off;
+  }
+  if constexpr (S::NC == 5) {
+    ring.template write<N>(m0, k0 - (kt - 32 * (NMAX - N)), 0);
+    p.slot = 1;
+  } else {
+#pragma unroll
+    for (int c = 0; c < N; ++c) w.m[0][c] = m0[c];
+  }
+  const unsigned long long b = __ballot(done != 0);
+  if (b) {
+    p.end_k = first_diagonal<N>(done, kt);
+    p.end_off = lane_of(off, (int)__builtin_ctzll(b));
+  }
+  return b != 0;
+}
+
+// NMAX: most diagonals per lane (4: pairs up to 254 diagonals, 8: 510).
+// SRC: bits per symbol of the packed sequences in memory.  8-bit symbols that
+// differ in their low four bits are kept as 4-bit ones in LDS.
+template <class S, int NMAX, int SRC, bool REC, bool EF>
+__global__ void __launch_bounds__(64, S::NC == 5 ? (NMAX == 8 ? 2 : 3) : (NMAX == 8 ? 3 : 5)) wfa_wave_kernel(ForwardArgs a) {
+  constexpr int BITS = SRC == 2 ? 2 : 4;
+  extern __shared__ __align__(16) unsigned char smem[];
+  uint32_t* seqP = reinterpret_cast<uint32_t*>(smem);
+  uint32_t* seqT = seqP + a.wave.lds_words;
+  __shared__ __align__(16) int16_t ring_lds[S::NC == 5 ? WaveRing<NMAX>::kBytes / 2 : 8];
+  const WaveRing<NMAX> ring{ring_lds};
+  const int lane = threadIdx.x;
+  WaveChunk ch{0, 0};
+  unsigned long long wg_dsteps = 0;
+  bool q_first = true;
+  for (;;) {
+    KernArgs A = args_now();
+    int qv = 0;
+    if (!q_first && lane == 0) qv = (int)atomicAdd(work_queue(A->queue, A->queues), 1u);
+    const int qi = work_item(A->queues, q_first, lane_of(qv, 0));
+    q_first = false;
+    if (qi >= A->n_pairs) break;
+    const int id = A->order ? A->order[qi] : qi;
+    WavePair p;
+    p.plen = A->plen[id];
+    p.tlen = A->tlen[id];
+    p.kend = p.tlen - p.plen;
+    p.i = 0;
+    p.status = 1;
+    p.dev = 0;
+    p.exact = false;
+    p.slot = 0;
+    p.hist_m = p.hist_gap = 0;
+    p.end_k = p.kend;
+    p.end_off = p.tlen;
+    for (int x = 0; x < kWavePhases; ++x) p.base[x] = 0;
+    const long long ppos = A->pat_pos[id], tpos = A->txt_pos[id];
+    WaveSeqs<BITS> q{seqP, seqT, 0u, 0u, p.plen, p.tlen};
+    wave_sync();  // the previous pair is done reading the sequences
+    if constexpr (SRC == 2) {
+      q.pbit = 2u * (unsigned)(ppos & 31);
+      q.tbit = 2u * (unsigned)(tpos & 31);
+      const uint64_t* gP = A->words + (ppos >> 5);
+      const uint64_t* gT = A->words + (tpos >> 5);
+      const int nwp = ((int)(ppos & 31) + p.plen) / 32 + 2, nwt = ((int)(tpos & 31) + p.tlen) / 32 + 2;
+      uint64_t* dP = reinterpret_cast<uint64_t*>(seqP);
+      uint64_t* dT = reinterpret_cast<uint64_t*>(seqT);
+      for (int x = lane; x < nwp; x += 64) dP[x] = gP[x];
+      for (int x = lane; x < nwt; x += 64) dT[x] = gT[x];
+    } else {
+      q.pbit = 4u * (unsigned)(ppos & 7);
+      q.tbit = 4u * (unsigned)(tpos & 7);
+      // eight bytes to eight nibbles
+      auto squeeze = [](uint64_t v) {
+        v &= 0x0F0F0F0F0F0F0F0Full;
+        v = (v | (v >> 4)) & 0x00FF00FF00FF00FFull;
+        v = (v | (v >> 8)) & 0x0000FFFF0000FFFFull;
+        return (uint32_t)(v | (v >> 16));
+      };
+      const uint64_t* gP = A->words + (ppos >> 3);
+      const uint64_t* gT = A->words + (tpos >> 3);
+      const int nwp = ((int)(ppos & 7) + p.plen) / 8 + 2, nwt = ((int)(tpos & 7) + p.tlen) / 8 + 2;
+      for (int x = lane; x < nwp; x += 64) seqP[x] = squeeze(gP[x]);
+      for (int x = lane; x < nwt; x += 64) seqT[x] = squeeze(gT[x]);
+    }
+    wave_sync();
+    uint32_t header = kNoBlock;
+    if constexpr (REC) {
+      // the pair's header: the units of its phases' records
+      if (reserve_records(ch, 1)) header = ch.cur++;
+      else p.status = kDevArenaFull;
+    }
+    // phases: rows of 1, 2, 4 (and 8) diagonals per lane in turn
+    WaveRows<S, 1> w1;
+    WaveRows<S, 2> w2;
+    WaveRows<S, 4> w4;
+    const int phase0 = EF ? A->wave.phase0 : 0;
+    bool ended = false;
+    if (p.status == 1) {
+      if (phase0 == 0) ended = wave_start<S, 1, NMAX, BITS, EF>(p, w1, q, ring);
+      else if (phase0 == 1) ended = wave_start<S, 2, NMAX, BITS, EF>(p, w2, q, ring);
+      else ended = wave_start<S, 4, NMAX, BITS, EF>(p, w4, q, ring);
+      if (ended) p.status = kDevCompleted;
+    }
+    if (p.status == 1 && phase0 == 0) {
+      wave_phase<S, 1, NMAX, BITS, REC, EF>(p, ch, w1, q, ring);
+      if (p.status == 1) widen<S, 1>(w1, w2);
+    }
+    if (p.status == 1 && phase0 <= 1) {
+      wave_phase<S, 2, NMAX, BITS, REC, EF>(p, ch, w2, q, ring);
+      if (p.status == 1) widen<S, 2>(w2, w4);
+    }
+    if (p.status == 1) wave_phase<S, 4, NMAX, BITS, REC, EF>(p, ch, w4, q, ring);
+    if constexpr (NMAX >= 8) {
+      if (p.status == 1) {
+        WaveRows<S, 8> w8;
+        widen<S, 4>(w4, w8);
+        wave_phase<S, 8, NMAX, BITS, REC, EF>(p, ch, w8, q, ring);
+      }
+    }
+    if (p.status == 1) p.status = kDevRingOverflow;  // wider than the wave holds
+    KernArgs B = args_now();
+    const bool good = p.status == kDevCompleted;
+    const int ds = good ? wave_table<S>.dsteps[p.i] + p.dev + (EF ? wave_table<S>.nonnull[p.i] * (B->pbf + B->tbf) : 0) : 0;
+    if (lane == 0) {
+      B->out_status[id] = p.status;
+      B->out_score[id] = p.i * B->pen.g;
+      B->out_last_block[id] = header;
+      B->out_dsteps[id] = (long long)ds;
+      if (REC && good) B->rec_arena[header] = make_uint4(p.base[0], p.base[1], p.base[2], p.base[3]);
+      if (B->out_end_k) {
+        B->out_end_k[id] = p.end_k;
+        B->out_end_off[id] = p.end_off;
+      }
+      if (!good) atomicAdd(B->retry_count, 1u);
+    }
+    wg_dsteps += (unsigned long long)ds;
+  }
+  if (lane == 0 && wg_dsteps) atomicAdd(args_now()->dsteps_total, wg_dsteps);
+}
+
+template <class S>
+bool wave_matches(const Penalties& p) {
+  if (p.g <= 0 || p.ncomp != S::NC) return false;
+  if (S::NC == 1) {
+    if (!S::kMismatch) return p.metric == kIndel;
+    return p.metric != kIndel && p.x == S::DX * p.g && p.o1 == S::DO1 * p.g;
+  }
+  return p.x == S::DX * p.g && p.o1 + p.e1 == S::DO1 * p.g && p.e1 == S::DE1 * p.g &&
+         (S::NC != 5 || (p.o2 + p.e2 == S::DO2 * p.g && p.e2 == S::DE2 * p.g));
+}
+
+template <class S, int SRC, bool EF>
+const void* wave_fn(int nmax, bool rec) {
+  if (nmax <= 4)
+    return rec ? reinterpret_cast<const void*>(&wfa_wave_kernel<S, 4, SRC, true, EF>)
+               : reinterpret_cast<const void*>(&wfa_wave_kernel<S, 4, SRC, false, EF>);
+  return rec ? reinterpret_cast<const void*>(&wfa_wave_kernel<S, 8, SRC, true, EF>)
+             : reinterpret_cast<const void*>(&wfa_wave_kernel<S, 8, SRC, false, EF>);
+}
+template <class S>
+const void* wave_fn_of(int nmax, bool rec, int bits, bool ef) {
+  if (bits == 2) return ef ? wave_fn<S, 2, true>(nmax, rec) : wave_fn<S, 2, false>(nmax, rec);
+  return ef ? wave_fn<S, 8, true>(nmax, rec) : wave_fn<S, 8, false>(nmax, rec);
+}
+const void* select_wave(int shape, int nmax, bool rec, int bits, bool ef) {
+  switch (shape) {
+    case 1: return wave_fn_of<ShapeAffine>(nmax, rec, bits, ef);
+    case 2: return wave_fn_of<Shape2p>(nmax, rec, bits, ef);
+    case 3: return wave_fn_of<ShapeEdit>(nmax, rec, bits, ef);
+    case 4: return wave_fn_of<ShapeIndel>(nmax, rec, bits, ef);
+    case 5: return wave_fn_of<ShapeLinear>(nmax, rec, bits, ef);
+  }
+  return nullptr;
+}
+
+}  // namespace
+
+int wave_shape(const Penalties& pen) {
+  if (wave_matches<ShapeAffine>(pen)) return 1;
+  if (wave_matches<Shape2p>(pen)) return 2;
+  if (wave_matches<ShapeEdit>(pen)) return 3;
+  if (wave_matches<ShapeIndel>(pen)) return 4;
+  if (wave_matches<ShapeLinear>(pen)) return 5;
+  return 0;
+}
+
+bool wave_phases(int shape, int pbf, int tbf, int nmax, WaveArgs* w) {
+  const WaveTable* t = shape == 1 ? &host_wave_table<ShapeAffine> : shape == 2 ? &host_wave_table<Shape2p>
+                     : shape == 3 ? &host_wave_table<ShapeEdit>
+                     : shape == 4 ? &host_wave_table<ShapeIndel> : shape == 5 ? &host_wave_table<ShapeLinear> : nullptr;
+  if (!t) return false;
+  *w = WaveArgs{};
+  w->center = (tbf - pbf) / 2;
+  w->phase0 = -1;
+  for (int ph = 0; ph < kWavePhases; ++ph) {
+    const int n = 1 << ph, kt = w->center - 32 * n;
+    // wavefronts keep clear of the wave's first and last diagonal
+    auto fits = [&](int lo, int hi) { return lo - pbf > kt && hi + tbf < kt + 64 * n - 1; };
+    int steps = 0;
+    if (n <= nmax && fits(0, 0)) {
+      while (steps < kWaveSteps && fits(t->hull_lo[steps], t->hull_hi[steps])) ++steps;
+      if (w->phase0 < 0) w->phase0 = ph;
+    }
+    const int per_word = n < 4 ? 4 / n : 1;
+    w->last[ph] = steps / per_word * per_word;
+    if (ph && w->last[ph] < w->last[ph - 1]) w->last[ph] = w->last[ph - 1];
+  }
+  return w->phase0 >= 0 && w->phase0 <= 2;
+}
+
+size_t wave_lds_bytes(int lds_words) { return (size_t)2 * lds_words * sizeof(uint32_t); }
+
+int wave_max_blocks_per_cu(int shape, int nmax, bool rec, int bits, bool ef, size_t lds) {
+  const void* f = select_wave(shape, nmax, rec, bits, ef);
+  int n = 0;
+  if (!f || hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, f, 64, lds) != hipSuccess) return 0;
+  return n;
+}
+
+hipError_t launch_forward_wave(const ForwardArgs& a, int shape, int nmax, int bits, const LaunchShape& ls,
+                               hipStream_t stream) {
+  const void* f = select_wave(shape, nmax, a.records != 0, bits, a.endsfree != 0);
+  if (!f || ls.block != 64) return hipErrorInvalidValue;
+  void* args[] = {const_cast<ForwardArgs*>(&a)};
+  return hipLaunchKernel(f, dim3(ls.grid), dim3(64), args, ls.lds_bytes, stream);
+}
+
+}  // namespace wfa
