@@ -197,6 +197,8 @@ Engine::~Engine() {
   if (plain.graph) (void)hipGraphDestroy(plain.graph);
   for (auto& ev : tile.ev)
     if (ev) (void)hipEventDestroy(ev);
+  for (auto& ev : bi_tiles.ev)
+    if (ev) (void)hipEventDestroy(ev);
 }
 
 Engine* engine_of(wavefront_aligner_t* wf) { return static_cast<Engine*>(wf->device); }

@@ -17,6 +17,7 @@
 #include <vector>
 
 #include "wfa_internal.h"
+#include "wfa_shapes.h"
 
 namespace wfa_host {
 namespace {
@@ -128,6 +129,146 @@ bool pair_searches_enabled() {
 // 100 kbp pair take 100 KB of gfx950's 160 KB per CU).
 constexpr size_t kBreakpointSeqLdsBytes = 120 * 1024;
 
+// Sub-problems of at least this many symbols (both sequences) are advanced in
+// tiles first.  Below, one workgroup steps through the whole search in less
+// than the launches of its blocks take.  64 pairs of 20-60 kbp: from 4,096
+// symbols 69.2 ms, from 2,048 67.0 ms, from 1,024 66.8 ms, from 512 66.4 ms
+// (few sub-problems of a long pair are that small); one workgroup or team per
+// search throughout, 482 ms.
+constexpr int kBiTileMinSize = 1024;
+// Rows of the sub-problems of one launch, and their number (the grid has two
+// rows of workgroups for each).
+constexpr size_t kBiTileStateBytes = size_t(8) << 30;
+constexpr size_t kBiTileMaxProblems = 16384;
+
+// Tables of the tiles' ranges for the begin components M, I1 and D1.
+bool bi_table(Engine* e, int steps) {
+  Engine::BiTiles& t = e->bi_tiles;
+  if (t.steps >= steps) return true;
+  steps = std::max({steps, 4096, 2 * t.steps});
+  std::vector<int> hull((size_t)3 * steps * 2);
+  std::vector<long long> dsteps((size_t)3 * (steps + 1), 0);
+  t.lo.assign(steps, 0);
+  t.hi.assign(steps, 0);
+  const wfa::TileGeometry g = wfa::tile_geometry(1);
+  for (int begin = 0; begin < 3; ++begin) {
+    std::vector<wfa::StepRanges> rows((size_t)steps + 1);
+    rows[0].c[begin].lo = rows[0].c[begin].hi = 0;
+    int lo = 0, hi = 0;
+    long long* ds = dsteps.data() + (size_t)begin * (steps + 1);
+    for (int i = 0; i < steps; ++i) {
+      auto row = [&](int back, int c) { return i + 1 - back >= 0 ? rows[i + 1 - back].c[c] : wfa::StepRange{}; };
+      rows[i + 1] = wfa::next_ranges(3, g.dx, g.do1, g.de1, 0, 0, row);
+      const wfa::StepRange m = rows[i + 1].c[wfa::kM];
+      ds[i + 1] = ds[i] + wfa::step_diagonals(m, 3, g.dx, g.do1, g.de1, 0, 0, row);
+      if (m.valid()) {
+        lo = std::min(lo, m.lo);
+        hi = std::max(hi, m.hi);
+      }
+      hull[2 * ((size_t)begin * steps + i)] = lo;
+      hull[2 * ((size_t)begin * steps + i) + 1] = hi;
+      t.lo[i] = std::min(t.lo[i], lo);
+      t.hi[i] = std::max(t.hi[i], hi);
+    }
+  }
+  t.steps = 0;
+  hipStream_t st = e->stream;
+  if (!t.d_hull.ensure(hull.size() * sizeof(int)) || !t.d_dsteps.ensure(dsteps.size() * sizeof(long long)) ||
+      !hip_ok(hipMemcpyAsync(t.d_hull.p, hull.data(), hull.size() * sizeof(int), hipMemcpyHostToDevice, st), "bi table") ||
+      !hip_ok(hipMemcpyAsync(t.d_dsteps.p, dsteps.data(), dsteps.size() * sizeof(long long), hipMemcpyHostToDevice, st),
+              "bi table") ||
+      !hip_ok(hipStreamSynchronize(st), "bi table"))
+    return false;
+  t.steps = steps;
+  return true;
+}
+
+// Advances the sub-problems probs[0..n) (already in d_probs) in tiles until
+// the block in which phase 1 ends, and sets a's resume fields; without memory
+// for their rows the search runs from the start.
+bool bi_fast_forward(Engine* e, const std::vector<wfa::BiProblem>& probs, wfa::BiArgs& a) {
+  Engine::BiTiles& t = e->bi_tiles;
+  const int n = (int)probs.size(), T = wfa::bi_tile_steps(), U = wfa::bi_tile_useful();
+  hipStream_t st = e->stream;
+  // a side that never meets the other ends at its own end: no more steps
+  // than that alignment can cost
+  const wfa::TileGeometry g = wfa::tile_geometry(1);
+  int max_steps = 0, lw = 0;
+  int64_t ints = 0;
+  std::vector<int64_t> off(n);
+  for (int i = 0; i < n; ++i) {
+    const int pl = probs[i].pe - probs[i].pb, tl = probs[i].te - probs[i].tb;
+    const int64_t mn = std::min(pl, tl), mx = std::max(pl, tl);
+    max_steps = (int)std::max<int64_t>(max_steps, mn * g.dx + 2 * g.do1 + (mx - mn) * g.de1);
+    lw = std::max(lw, (int)mx / 32 + 4);
+    off[i] = ints;
+    ints += (int64_t)2 * wfa::kBiTileRows * wfa::tile_pitch(pl, tl);
+  }
+  const int max_blocks = max_steps / T + 2;  // (a search not done by then starts over: wfa_breakpoint_kernel)
+  if (!bi_table(e, (max_blocks + 1) * T)) return false;
+  if (!t.h_n.ensure(4096) || !t.d_state.ensure((size_t)ints * 4) || !t.d_off.ensure((size_t)n * 8) ||
+      !t.d_marks.ensure((size_t)n * 5 * 4) || !t.d_act.ensure((size_t)2 * n * 4 + 64))
+    return true;
+  for (auto& ev : t.ev)
+    if (!ev && !hip_ok(hipEventCreateWithFlags(&ev, hipEventDisableTiming), "hipEventCreate")) return false;
+  volatile int* h_n = t.h_n.as<int>();
+  int* n_act = t.d_act.as<int>();
+  int* act[2] = {n_act + 16, n_act + 16 + n};
+  wfa::BiTileArgs f{};
+  f.n = n;
+  f.probs = a.probs;
+  f.words = a.words;
+  f.rev_words = a.rev_words;
+  f.fwd_ppos = a.fwd_ppos;
+  f.fwd_tpos = a.fwd_tpos;
+  f.rev_ppos = a.rev_ppos;
+  f.rev_tpos = a.rev_tpos;
+  f.plen_total = a.plen_total;
+  f.tlen_total = a.tlen_total;
+  f.state = t.d_state.as<int>();
+  f.st_off = t.d_off.as<int64_t>();
+  f.done = t.d_marks.as<int>();
+  f.far = f.done + n;
+  f.hull = t.d_hull.as<int2>();
+  f.steps = t.steps;
+  f.lmax_words = lw;
+  if (!hip_ok(hipMemcpyAsync(t.d_off.p, off.data(), (size_t)n * 8, hipMemcpyHostToDevice, st), "bi tiles") ||
+      !hip_ok(wfa::launch_tile_fill(f.state, ints, st), "bi tile fill") ||
+      !hip_ok(wfa::launch_bi_tile_init(f, act[0], n_act, st), "bi tile init") ||
+      !hip_ok(hipStreamSynchronize(st), "bi tiles"))  // (off is read by then)
+    return false;
+  int known = n, which = 0, chunk = 0;
+  for (int blk = 0; blk < max_blocks && known > 0;) {
+    const int to = std::min(max_blocks, blk + (chunk < 4 ? 4 : 16));
+    for (; blk < to; ++blk) {
+      f.act = act[which];
+      f.n_act = n_act + which;
+      f.blk = blk;
+      const int lo = blk ? t.lo[(size_t)blk * T - 1] : 0, hi = blk ? t.hi[(size_t)blk * T - 1] : 0;
+      if (!hip_ok(wfa::launch_bi_tile_block(f, known, (hi - lo + 2 * T + 8) / U + 1, st), "bi tile launch")) return false;
+    }
+    const int slot = chunk & 1;
+    if (!hip_ok(wfa::launch_tile_compact(act[which], n_act + which, f.done, nullptr, blk, act[which ^ 1],
+                                         n_act + (which ^ 1), const_cast<int*>(h_n) + slot, st), "bi tile compact") ||
+        !hip_ok(hipEventRecord(t.ev[slot], st), "bi tile event"))
+      return false;
+    which ^= 1;
+    if (chunk > 0) {
+      if (!hip_ok(hipEventSynchronize(t.ev[slot ^ 1]), "bi tiles")) return false;
+      known = h_n[slot ^ 1];
+    }
+    ++chunk;
+  }
+  a.resume = f.done;
+  a.resume_state = f.state;
+  a.resume_off = f.st_off;
+  a.resume_far = f.far;
+  a.resume_dsteps = t.d_dsteps.as<long long>();
+  a.resume_table = t.steps + 1;
+  a.resume_block = T;
+  return true;
+}
+
 // Runs the breakpoint search of `nodes` (grouped by size) and returns the outcomes.
 bool run_breakpoints(wavefront_aligner_t* wf, Engine* e, wfa_device_batch_t* b, const std::vector<Node>& nodes,
                      std::vector<wfa::BiOutcome>& out, RunTotals* tot) {
@@ -145,10 +286,39 @@ bool run_breakpoints(wavefront_aligner_t* wf, Engine* e, wfa_device_batch_t* b, 
   }
   hipStream_t st = e->stream;
   const wfa::HeurArgs heur = heuristic_of(wf);
-  for (int gi = 0; gi < 3; ++gi) {
-    std::vector<int> ids = groups[gi];
+  const bool tiles_ok = wfa::tile_shape(pen) == 1 && b->bits == 2 && heur.cut() == 0 &&
+                        (wf->system.max_alignment_steps <= 0 || wf->system.max_alignment_steps == INT_MAX);
+  // large sub-problems in tiles: as many at once as their rows' memory allows
+  std::vector<std::vector<int>> runs(groups, groups + 3);
+  std::vector<int> run_block = {64, 256, 1024};
+  if (tiles_ok) {
+    for (int gi = 0; gi < 3; ++gi) {
+      int64_t bytes = INT64_MAX;
+      std::vector<int> rest;
+      for (int i : groups[gi]) {
+        const wfa::BiProblem& p = nodes[i].prob;
+        const int pl = p.pe - p.pb, tl = p.te - p.tb;
+        if (pl + tl < kBiTileMinSize || 2 * (size_t)(std::max(pl, tl) / 32 + 4) * 8 > wfa::kTileSeqLdsBytes) {
+          rest.push_back(i);
+          continue;
+        }
+        const int64_t need = (int64_t)2 * wfa::kBiTileRows * wfa::tile_pitch(pl, tl) * 4;
+        if (bytes > (int64_t)kBiTileStateBytes - need || runs.back().size() >= kBiTileMaxProblems) {
+          runs.emplace_back();
+          run_block.push_back(run_block[gi]);
+          bytes = 0;
+        }
+        runs.back().push_back(i);
+        bytes += need;
+      }
+      runs[gi].swap(rest);
+    }
+  }
+  for (size_t ri = 0; ri < runs.size(); ++ri) {
+    const bool tile = ri >= 3;
+    const std::vector<int>& ids = runs[ri];
     if (ids.empty()) continue;
-    const int block = gi == 0 ? 64 : (gi == 1 ? 256 : 1024);
+    const int block = run_block[ri];
     // One launch over the sub-problems `sel` (indices into nodes); paired:
     // two workgroups per sub-problem.  Outcomes go to out[].
     auto launch = [&](const std::vector<int>& sel, bool paired) -> bool {
@@ -228,6 +398,7 @@ bool run_breakpoints(wavefront_aligner_t* wf, Engine* e, wfa_device_batch_t* b, 
                 (!paired || hip_ok(hipMemsetAsync(a.mail, 0, probs.size() * 4 * sizeof(unsigned long long), st),
                                    "mailboxes"));
       (void)hipEventRecord(e0, st);
+      if (ok && tile && !bi_fast_forward(e, probs, a)) return false;
       ok = ok && hip_ok(paired ? wfa::launch_breakpoint_pair(a, ncomp, b->bits, block, st)
                                : wfa::launch_breakpoint(a, ncomp, b->bits, block, grid, st),
                         "breakpoint launch");
@@ -250,7 +421,7 @@ bool run_breakpoints(wavefront_aligner_t* wf, Engine* e, wfa_device_batch_t* b, 
     // workgroups the CUs hold); not with a heuristic cut-off, or where the
     // extra ring slot would pass the 64 slots of the slot metadata.
     bool paired = false;
-    if (block == 1024 && heur.cut() == 0 && pen.nslots + 1 <= 64 && pair_searches_enabled()) {
+    if (!tile && block == 1024 && heur.cut() == 0 && pen.nslots + 1 <= 64 && pair_searches_enabled()) {
       const int spw = 64 / b->bits;
       int lw = 0;
       for (int i : ids) {

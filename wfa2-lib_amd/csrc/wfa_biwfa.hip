@@ -11,7 +11,10 @@
 // ascending order (breakpoint_indel2indel :477-573, breakpoint_m2m :798-874).
 // Each scan is a block-parallel min-reduction over k0.  The host recurses on
 // the two halves, level by level across all pairs (wfa_bialign.cpp).
+// Phase 1 of a large sub-problem runs in tiles of diagonals all over the
+// device (bi_tile_kernel) up to the block in which it ends.
 #include "wfa_common.h"
+#include "wfa_tile.h"
 
 namespace wfa {
 namespace {
@@ -535,6 +538,58 @@ __device__ int side_extend0(Side<NC, CUT>& sd, int plen, int tlen, int wcap, con
   return 0;
 }
 
+// Rows of a side that the tiles left at the start of step ib (BiTileArgs):
+// the last steps' M, I1 and D1 into the side's ring, with the ranges that the
+// slot metadata holds (first and last valid cell; the side has not touched a
+// border, so no wavefront is null and no other limit applies).
+template <int NC, int BLOCK, bool CUT>
+__device__ void side_resume(Side<NC, CUT>& sd, const int* rows, int par, int ib, int g, int plen, int tlen, int wcap,
+                            int R, BlockRed<BLOCK>& red) {
+  constexpr int SH = 3;  // bits below the offset in the tiles' rows
+  const int pitch = tile_pitch(plen, tlen), kpad = tile_kpad(plen), lane = threadIdx.x & 63;
+  const int kmin = max(-plen, -ib), kmax = min(tlen, ib);  // a step reaches one diagonal further
+  for (int age = kBiTileAges - 1; age >= 0; --age) {
+    const int i = ib - 1 - age;
+    const int s = (i + 1) * g, slot = (i + 1) % R;
+    int lo[3], hi[3], alo = INT_MAX;
+    for (int c = 0; c < 3; ++c) {
+      const int* row = rows + (long long)bi_row(par, c, age) * pitch + kpad;
+      int first = INT_MAX, last = INT_MIN;
+      for (int k = kmin + (int)threadIdx.x; k <= kmax; k += BLOCK) {
+        const int v = row[k];
+        if (v >= 0 && in_bounds(v >> SH, k, plen, tlen)) {
+          first = min(first, k);
+          last = max(last, k);
+        }
+      }
+      lo[c] = red.min_all(first);
+      hi[c] = red.max_all(last);
+      alo = min(alo, lo[c]);
+    }
+    unsigned fl = 0;
+    for (int c = 0; c < 3; ++c) {
+      if (lo[c] > hi[c]) continue;
+      fl |= 1u << c;
+      const int* row = rows + (long long)bi_row(par, c, age) * pitch + kpad;
+      int* out = sd.ring + (slot * NC + c) * wcap - alo;
+      for (int k = lo[c] + (int)threadIdx.x; k <= hi[c]; k += BLOCK) {
+        const int v = row[k];
+        out[k] = v < 0 ? kOffsetNull : v >> SH;
+      }
+    }
+    if (lane == slot) {
+      sd.meta.tag = s;
+      sd.meta.alo = alo == INT_MAX ? 0 : alo;
+      sd.meta.flags = fl;
+      for (int c = 0; c < 3; ++c) {
+        sd.meta.lo[c] = lo[c] <= hi[c] ? lo[c] : 0;
+        sd.meta.hi[c] = lo[c] <= hi[c] ? hi[c] : -1;
+      }
+    }
+    sd.cur = slot;
+  }
+}
+
 // Sequences and rings of sub-problem pr for both sides (ring: this
 // workgroup's or team's region, forward then reverse); with a.lmax_words > 0
 // the four sequences (forward and reversed pattern and text) are copied into
@@ -676,8 +731,24 @@ __global__ void __launch_bounds__(BLOCK) wfa_breakpoint_kernel(BiArgs a) {
     bool last_forward = false;
     int rc;
     // phase 1 (wavefront_bialign.c:1003-1044)
-    if (side_extend0<NC, BLOCK, BITS>(f, plen, tlen, wcap, pen, a.heur, red, &fmax)) { status = kBiEndReached; goto done; }
-    if (side_extend0<NC, BLOCK, BITS>(r, plen, tlen, wcap, pen, a.heur, red, &rmax)) { status = kBiEndReached; goto done; }
+    const int blk = (NC == 3 && !CUT && a.resume) ? a.resume[q] : 0;
+    if (blk > 0 && blk != INT_MAX) {
+      if constexpr (NC == 3 && !CUT) {
+        const int ib = blk * a.resume_block, par = (blk & 1) ^ 1;
+        const int* rows = a.resume_state + a.resume_off[q];
+        side_resume<NC, BLOCK>(f, rows, par, ib, pen.g, plen, tlen, wcap, pen.nslots, red);
+        side_resume<NC, BLOCK>(r, rows + (long long)kBiTileRows * tile_pitch(plen, tlen), par, ib, pen.g, plen, tlen,
+                               wcap, pen.nslots, red);
+        sf = sr = ib * pen.g;
+        fmax = a.resume_far[par * 2 * a.n + 2 * q];
+        rmax = a.resume_far[par * 2 * a.n + 2 * q + 1];
+        dsteps = a.resume_dsteps[pr.comp_begin * a.resume_table + ib] + a.resume_dsteps[pr.comp_end * a.resume_table + ib];
+        __syncthreads();
+      }
+    } else {
+      if (side_extend0<NC, BLOCK, BITS>(f, plen, tlen, wcap, pen, a.heur, red, &fmax)) { status = kBiEndReached; goto done; }
+      if (side_extend0<NC, BLOCK, BITS>(r, plen, tlen, wcap, pen, a.heur, red, &rmax)) { status = kBiEndReached; goto done; }
+    }
     while (true) {
       if (fmax + rmax >= max_ad) break;
       ++sf;

@@ -272,6 +272,15 @@ struct BiArgs {
   unsigned long long* mail;
   int* handover;
   unsigned long long pair_wait_ticks;  // bound of every wait, 100 MHz device clock ticks
+  // Sub-problems advanced in tiles (BiTileArgs), null otherwise: the search
+  // goes on from the start of block resume[q].
+  const int* resume;
+  const int* resume_state;     // BiTileArgs::state and st_off
+  const int64_t* resume_off;
+  const int* resume_far;       // BiTileArgs::far
+  const long long* resume_dsteps;  // [3][steps + 1]: diagonal-steps of the first i steps, by the begin component
+  int resume_table;            // steps + 1
+  int resume_block;            // steps per block
 };
 hipError_t launch_breakpoint(const BiArgs& a, int ncomp, int bits, int block, int grid, hipStream_t stream);
 // Paired workgroups, one sub-problem per team of two (2 * a.n workgroups of

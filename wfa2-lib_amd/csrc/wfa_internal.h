@@ -153,6 +153,14 @@ struct Engine {
     HostBuf h_n;                      // jobs left, written by the device
     hipEvent_t ev[5] = {nullptr, nullptr, nullptr, nullptr, nullptr};
   } tile;
+  // BiWFA sub-problems in tiles (wfa_bialign.cpp): range tables and buffers.
+  struct BiTiles {
+    int steps = 0;
+    std::vector<int> lo, hi;
+    DevBuf d_hull, d_dsteps, d_state, d_off, d_marks, d_act;
+    HostBuf h_n;
+    hipEvent_t ev[2] = {nullptr, nullptr};
+  } bi_tiles;
   // Set for the duration of a no-allocation run: plan groups take their
   // order arrays from `order`, and the HBM-ring family's grid is limited so
   // that its rings fit in ring_bytes (the engine's rec/ring/counters buffers

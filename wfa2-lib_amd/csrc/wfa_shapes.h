@@ -70,6 +70,32 @@ constexpr StepRanges next_ranges(int ncomp, int dx, int do1, int de1, int do2, i
   return r;
 }
 
+// Diagonals of a step whose sources are row(...) and whose cells reach [m.lo,
+// m.hi]: a null source still contributes the limits (1, -1), shifted as its
+// gap moves it.
+template <class Row>
+constexpr int step_diagonals(const StepRange& m, int ncomp, int dx, int do1, int de1, int do2, int de2, Row row) {
+  if (!m.valid()) return 0;
+  int lo = m.lo, hi = m.hi;
+  auto null = [&](int back, int c, int l, int h) {
+    if (row(back, c).valid()) return;
+    lo = l < lo ? l : lo;
+    hi = h > hi ? h : hi;
+  };
+  if (dx > 0) null(dx, kM, 1, -1);
+  null(do1, kM, 0, 0);
+  if (ncomp > 1) {
+    null(de1, kI1, 2, 0);
+    null(de1, kD1, 0, -2);
+  }
+  if (ncomp == 5) {
+    null(do2, kM, 0, 0);
+    null(de2, kI2, 2, 0);
+    null(de2, kD2, 0, -2);
+  }
+  return hi - lo + 1;
+}
+
 // The first steps' ranges of a shape, tabulated by the compiler.  Row i is
 // step i; row -1, score 0, holds M = [0, 0].
 constexpr int kWaveSteps = 560;  // a wave of 8 diagonals per lane is outgrown before

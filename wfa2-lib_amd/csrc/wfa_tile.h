@@ -134,6 +134,37 @@ struct TileTraceArgs {
   int lmax_words;
 };
 
+// BiWFA: both sides of every large sub-problem advanced in tiles up to the
+// block in which phase 1 ends (the sides meet, or a side reaches its end or a
+// border); the breakpoint kernel goes on from the start of that block.
+struct BiTileArgs {
+  int n;                       // sub-problems
+  const int* act;              // active ones
+  const int* n_act;
+  const BiProblem* probs;
+  const uint64_t* words;
+  const uint64_t* rev_words;
+  const int64_t* fwd_ppos;
+  const int64_t* fwd_tpos;
+  const int64_t* rev_ppos;
+  const int64_t* rev_tpos;
+  const int* plen_total;
+  const int* tlen_total;
+  int* state;                  // per side: kBiTileRows rows
+  const int64_t* st_off;       // first int of a sub-problem's forward rows; its reverse rows follow
+  int* done;                   // block in which phase 1 ends (INT_MAX: not yet)
+  int* far;                    // [2][2 n]: by block parity, furthest antidiagonal of each side
+  const int2* hull;            // [3][steps]: hull of the ranges up to each step, by the begin component
+  int steps;                   // steps in the tables
+  int blk;
+  int lmax_words;
+};
+// Rows of a side: M, I1 and D1 of the last kBiTileAges steps of a block, by
+// block parity and age (0: the latest).  The step kernels of a search need
+// four; its overlap scans look one step further back.
+constexpr int kBiTileAges = 5, kBiTileRows = 2 * 3 * kBiTileAges;
+__host__ __device__ inline int bi_row(int par, int comp, int age) { return (3 * par + comp) * kBiTileAges + age; }
+
 struct TileGeometry {
   int steps;                   // per block
   int useful;                  // diagonals per tile
@@ -145,6 +176,10 @@ struct TileGeometry {
 // 0: no instance for these penalties.
 int tile_shape(const Penalties& pen);
 TileGeometry tile_geometry(int shape);
+int bi_tile_steps();           // steps per block
+int bi_tile_useful();          // diagonals per tile
+hipError_t launch_bi_tile_init(const BiTileArgs& a, int* act, int* n_act, hipStream_t st);
+hipError_t launch_bi_tile_block(const BiTileArgs& a, int problems, int tiles, hipStream_t st);
 hipError_t launch_tile_fill(int* state, long long ints, hipStream_t st);
 hipError_t launch_tile_init(int shape, const TileArgs& a, int n, const int* jobs, int* act, int* n_act, hipStream_t st);
 hipError_t launch_tile_block(int shape, bool records, const TileArgs& a, int jobs, hipStream_t st);

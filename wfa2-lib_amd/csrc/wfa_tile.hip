@@ -837,6 +837,178 @@ __global__ void __launch_bounds__(64) tile_backtrace_kernel(TileTraceArgs a) {
   }
 }
 
+// ------------------------------------------------------------------ BiWFA
+// A side's sub-sequences (see setup_sides of the breakpoint kernels).
+struct BiSide {
+  long long ppos, tpos;
+  const uint64_t* words;
+  int plen, tlen, begin, end;
+};
+__device__ __forceinline__ BiSide bi_side(const BiTileArgs& a, int prob, int side) {
+  const BiProblem pr = a.probs[prob];
+  BiSide s;
+  s.plen = pr.pe - pr.pb;
+  s.tlen = pr.te - pr.tb;
+  if (side == 0) {
+    s.words = a.words;
+    s.ppos = a.fwd_ppos[pr.pair] + pr.pb;
+    s.tpos = a.fwd_tpos[pr.pair] + pr.tb;
+    s.begin = pr.comp_begin;
+    s.end = pr.comp_end;
+  } else {
+    s.words = a.rev_words;
+    s.ppos = a.rev_ppos[pr.pair] + (a.plen_total[pr.pair] - pr.pe);
+    s.tpos = a.rev_tpos[pr.pair] + (a.tlen_total[pr.pair] - pr.te);
+    s.begin = pr.comp_end;
+    s.end = pr.comp_begin;
+  }
+  return s;
+}
+
+struct BiGeom {
+  static constexpr int N = 4, T = 16, H = 16, U = 64 * N - 2 * H;
+};
+
+// One block of T steps of both sides of every active sub-problem, score only:
+// blockIdx.y / 2 the sub-problem, blockIdx.y % 2 the side.  Nothing is trimmed
+// here: an end cell that leaves the matrix ends the block's validity like a
+// side that reaches its end or the sides' meeting, and the breakpoint kernel
+// takes over from the rows at the block's start, which sit in the other half.
+//
+// Bound by the vector units and, while few tiles are alive, by the latency of
+// a step (131 vector instructions for a lane's four cells, 33 a cell): a
+// launch costs 5.5 us for its loads and 0.85 us (one wave per SIMD) to 1.5 us
+// (four) per step.  One workgroup or team per search instead pays a barrier
+// and a trip to its ring in HBM per step, and the longest search decides: 64
+// pairs of 20-60 kbp took 482 ms that way, 67 ms in tiles (45 ms here, 14 ms
+// in the breakpoint kernel's last block and overlap scans).
+__global__ void __launch_bounds__(64 * kTileWaves) bi_tile_kernel(BiTileArgs a) {
+  using S = ShapeAffine;
+  constexpr int N = BiGeom::N, T = BiGeom::T, H = BiGeom::H, U = BiGeom::U;
+  extern __shared__ __align__(16) unsigned char smem[];
+  __shared__ int far_lds[kTileWaves];
+  if ((int)blockIdx.y >= 2 * *a.n_act) return;
+  const int prob = a.act[blockIdx.y >> 1], side = blockIdx.y & 1;
+  if (a.done[prob] < a.blk) return;
+  const int* far_in = a.far + ((a.blk & 1) ^ 1) * 2 * a.n + 2 * prob;
+  int* far_out = a.far + (a.blk & 1) * 2 * a.n + 2 * prob;
+  const BiSide sd = bi_side(a, prob, side);
+  const int plen = sd.plen, tlen = sd.tlen;
+  if (far_in[0] + far_in[1] >= plen + tlen - 1) {  // the sides met in the block before
+    if (threadIdx.x == 0 && blockIdx.x == 0) atomicMin(a.done + prob, a.blk - 1);
+    return;
+  }
+  const int ib = a.blk * T;
+  const int2 hull = ib > 0 ? a.hull[sd.begin * a.steps + ib - 1] : make_int2(0, 0);
+  const int left = (hull.x - T) & ~3, right = (hull.y + T + 4) & ~3;
+  const int tiles = (right - left + U - 1) / U;
+  if ((int)blockIdx.x * kTileWaves >= tiles) return;
+  uint64_t* seqP = reinterpret_cast<uint64_t*>(smem);
+  uint64_t* seqT = seqP + a.lmax_words;
+  {
+    const uint64_t* gP = sd.words + (sd.ppos >> 5);
+    const uint64_t* gT = sd.words + (sd.tpos >> 5);
+    const int nwp = ((int)(sd.ppos & 31) + plen) / 32 + 2, nwt = ((int)(sd.tpos & 31) + tlen) / 32 + 2;
+    for (int i = threadIdx.x; i < nwp; i += 64 * kTileWaves) seqP[i] = gP[i];
+    for (int i = threadIdx.x; i < nwt; i += 64 * kTileWaves) seqT[i] = gT[i];
+    __syncthreads();
+  }
+  const int lane = threadIdx.x & 63, wid = uniform(threadIdx.x >> 6);
+  const int tile = (int)blockIdx.x * kTileWaves + wid;
+  int far = 0;
+  if (tile < tiles) {
+    const int quads = (right - left) / 4;
+    const int first = left + 4 * (quads * tile / tiles), past = left + 4 * (quads * (tile + 1) / tiles);
+    const WaveSeqs<2> q{reinterpret_cast<const uint32_t*>(seqP), reinterpret_cast<const uint32_t*>(seqT),
+                        2u * (unsigned)(sd.ppos & 31), 2u * (unsigned)(sd.tpos & 31), plen, tlen};
+    const int kt = first - H, k0 = kt + N * lane;
+    const bool own = k0 >= first && k0 < past;
+    const int kend = tlen - plen;
+    const bool has_end = kend >= first && kend < past;
+    const bool ends = tile == 0 || tile == tiles - 1;
+    const int pitch = tile_pitch(plen, tlen);
+    int* st = a.state + a.st_off[prob] + (long long)side * kBiTileRows * pitch + (k0 + tile_kpad(plen));
+    const int pin = (a.blk & 1) ^ 1, pout = a.blk & 1;
+    WaveRows<S, N> w;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) load_row<N>(w.m[r], st + (long long)bi_row(pin, kM, 3 - r) * pitch);
+    load_row<N>(w.i1[0], st + (long long)bi_row(pin, kI1, 0) * pitch);
+    load_row<N>(w.d1[0], st + (long long)bi_row(pin, kD1, 0) * pitch);
+    const int end_not_m = sd.end == kM ? 0 : INT_MIN, end_not_i1 = sd.end == kI1 ? 0 : INT_MIN,
+              end_not_d1 = sd.end == kD1 ? 0 : INT_MIN;
+    bool stop = false;
+    auto one = [&](auto phc, int t) {
+      constexpr int PH = decltype(phc)::value;
+      StepCells<N> cell;
+      for (uint32_t& r : cell.rec) r = 0;
+      wave_step<S, N, PH, 2>(w, nullptr, k0, q, cell);
+#pragma unroll
+      for (int c = 0; c < N; ++c) far = (cell.ok[c] & own) ? max(far, 2 * cell.h[c] - (k0 + c)) : far;
+      if (ends) {
+        bool out = false;
+#pragma unroll
+        for (int c = 0; c < N; ++c) out |= cell.oob[c] & own;
+        stop |= __ballot(out) != 0;
+      }
+      if (has_end) {
+        bool fin = false;
+#pragma unroll
+        for (int c = 0; c < N; ++c) {
+          // (masks, not a choice between the rows: that would put the rows in scratch memory)
+          const int g = max(max(w.m[PH % S::RM][c] | end_not_m, w.i1[0][c] | end_not_i1), w.d1[0][c] | end_not_d1);
+          fin |= (k0 + c == kend) & ((g >> S::SH) >= tlen);
+        }
+        stop |= __ballot(fin) != 0;
+      }
+      if (t >= T - kBiTileAges && own) {
+        store_row<N>(st + (long long)bi_row(pout, kM, T - 1 - t) * pitch, w.m[PH % S::RM]);
+        store_row<N>(st + (long long)bi_row(pout, kI1, T - 1 - t) * pitch, w.i1[0]);
+        store_row<N>(st + (long long)bi_row(pout, kD1, T - 1 - t) * pitch, w.d1[0]);
+      }
+    };
+    static_assert(T % 4 == 0 && S::RM == 4 && S::DE1 == 1, "rows of a block");
+    for (int t = 0; t < T; t += 4) {
+      one(std::integral_constant<int, 0>{}, t);
+      one(std::integral_constant<int, 1>{}, t + 1);
+      one(std::integral_constant<int, 2>{}, t + 2);
+      one(std::integral_constant<int, 3>{}, t + 3);
+    }
+    if (stop && lane == 0) atomicMin(a.done + prob, a.blk);
+    for (int o = 32; o > 0; o >>= 1) far = max(far, __shfl_xor(far, o, 64));
+  }
+  if (lane == 0) far_lds[wid] = far;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    int f = far_in[side];
+    for (int x = 0; x < kTileWaves; ++x) f = max(f, far_lds[x]);
+    atomicMax(far_out + side, f);
+  }
+}
+
+// Score 0 of both sides, and the first active list.
+__global__ void __launch_bounds__(64) bi_tile_init_kernel(BiTileArgs a, int* act, int* n_act) {
+  using S = ShapeAffine;
+  const int x = blockIdx.x * 64 + threadIdx.x;
+  if (x == 0) *n_act = a.n;
+  if (x >= 2 * a.n) return;
+  const int prob = x >> 1, side = x & 1;
+  if (side == 0) {
+    act[prob] = prob;
+    a.done[prob] = INT_MAX;
+  }
+  const BiSide sd = bi_side(a, prob, side);
+  const int pitch = tile_pitch(sd.plen, sd.tlen);
+  int h = 0;
+  if (sd.begin == kM)
+    h = lcp_extend<2>(sd.words + (sd.ppos >> 5), (int)(sd.ppos & 31), sd.words + (sd.tpos >> 5), (int)(sd.tpos & 31),
+                      sd.plen, sd.tlen, 0, 0);
+  a.state[a.st_off[prob] + ((long long)side * kBiTileRows + bi_row(1, sd.begin, 0)) * pitch + tile_kpad(sd.plen)] =
+      (h << S::SH) | (sd.begin == kM ? 0 : 1);
+  // (an end reached at score 0: found again by the breakpoint kernel)
+  const bool end0 = sd.begin == kM && sd.end == kM && sd.plen == sd.tlen && h >= sd.tlen;
+  a.far[2 * prob + side] = a.far[2 * a.n + 2 * prob + side] = end0 ? sd.plen + sd.tlen : 2 * h;
+}
+
 template <class S>
 bool shape_matches(const Penalties& p) {
   if (p.g <= 0 || p.ncomp != S::NC) return false;
@@ -866,6 +1038,21 @@ int tile_shape(const Penalties& pen) {
 }
 
 TileGeometry tile_geometry(int shape) { return shape == 2 ? geometry<Shape2p>() : geometry<ShapeAffine>(); }
+
+int bi_tile_steps() { return BiGeom::T; }
+int bi_tile_useful() { return BiGeom::U; }
+
+hipError_t launch_bi_tile_init(const BiTileArgs& a, int* act, int* n_act, hipStream_t st) {
+  hipLaunchKernelGGL(bi_tile_init_kernel, dim3((2 * a.n + 63) / 64), dim3(64), 0, st, a, act, n_act);
+  return hipGetLastError();
+}
+
+hipError_t launch_bi_tile_block(const BiTileArgs& a, int problems, int tiles, hipStream_t st) {
+  const size_t lds = (size_t)2 * a.lmax_words * sizeof(uint64_t);
+  const dim3 grid((tiles + kTileWaves - 1) / kTileWaves, 2 * problems);
+  hipLaunchKernelGGL(bi_tile_kernel, grid, dim3(64 * kTileWaves), lds, st, a);
+  return hipGetLastError();
+}
 
 hipError_t launch_tile_fill(int* state, long long ints, hipStream_t st) {
   const long long n4 = ints / 4;
