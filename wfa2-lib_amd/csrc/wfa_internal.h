@@ -324,7 +324,7 @@ struct wfa_device_batch_t {
   wfa_host::DevBuf d_run_counts, d_run_off, d_runs, d_scan_temp;
   bool runs_ready = false;
   long long total_runs = 0;
-  std::vector<long long> h_run_off;
+  wfa_host::HostBuf h_run_off;  // first run of each pair, and the total
   ~wfa_device_batch_t();
 };
 
