@@ -633,124 +633,73 @@ __global__ void __launch_bounds__(BLOCK, BLOCK == 1024 ? 4 : 1) wfa_forward_kern
   if (tid == 0 && wg_dsteps) atomicAdd(a.dsteps_total, wg_dsteps);
 }
 
-// Sixteen bytes of a CIGAR slot gathered in registers before one aligned
-// 16-byte store (the backtrace is bound by memory transactions: one lane per
-// pair, so every store of a wave touches 64 different lines).
-struct OpChunk {
-  uint32_t a0 = 0u, a1 = 0u, a2 = 0u, a3 = 0u;
-  // Byte b (0..15).  The halves are combined before the select: a select
-  // between two members would become a load from a selected address, which
-  // keeps the chunk in memory instead of registers.
-  __device__ __forceinline__ unsigned byte_at(unsigned b) const {
-    const uint64_t lo = ((uint64_t)a1 << 32) | a0, hi = ((uint64_t)a3 << 32) | a2;
-    return (unsigned)(((b & 8u) ? hi : lo) >> (8u * (b & 7u))) & 0xFFu;
+// Operations of the walk, the last one on top: four bits each (0 X, 1 I, 2 D;
+// 4: it leads into an M cell), eight to a word.  Full words grow downwards
+// from the end of the slot's free part; the started word stays in a register.
+// Eight operations are at least eight bytes of the CIGAR, so the words (and
+// the bytes that aligning their top costs) fit the slot, and the replay, which
+// pops a word before it writes that far, never overtakes them.
+struct OpStack {
+  uint32_t* top;
+  uint32_t acc;
+  int n;
+  __device__ __forceinline__ OpStack(unsigned char* end)
+      : top(reinterpret_cast<uint32_t*>(end - (reinterpret_cast<uintptr_t>(end) & 3u))), acc(0u), n(0) {}
+  __device__ __forceinline__ void push(uint32_t op) {
+    acc = (acc << 4) | op;
+    if ((++n & 7) == 0) *--top = acc;
   }
-  __device__ __forceinline__ static uint32_t span(unsigned from, unsigned to, unsigned j) {
-    const unsigned lo = from < 4 * j ? 0u : from > 4 * j + 4 ? 4u : from - 4 * j;
-    const unsigned hi = to < 4 * j ? 0u : to > 4 * j + 4 ? 4u : to - 4 * j;
-    return (uint32_t)((1ull << (8 * hi)) - (1ull << (8 * lo)));
+  __device__ __forceinline__ uint32_t pop() {
+    if ((n & 7) == 0) acc = *top++;
+    --n;
+    const uint32_t op = acc & 15u;
+    acc >>= 4;
+    return op;
   }
-  // Bytes [from, to) (0 <= from <= to <= 16), zero before, set to c4's byte
-  // (c4 holds it four times).
-  __device__ __forceinline__ void fill(unsigned from, unsigned to, uint32_t c4) {
-    a0 |= c4 & span(from, to, 0);
-    a1 |= c4 & span(from, to, 1);
-    a2 |= c4 & span(from, to, 2);
-    a3 |= c4 & span(from, to, 3);
-  }
-  __device__ __forceinline__ void store(unsigned char* at) const {
-    *reinterpret_cast<uint4*>(at) = make_uint4(a0, a1, a2, a3);
-  }
-  __device__ __forceinline__ void clear() { a0 = a1 = a2 = a3 = 0u; }
 };
 
-__device__ __forceinline__ unsigned chunk_phase(const unsigned char* at) {
-  return (unsigned)(reinterpret_cast<uintptr_t>(at) & 15u);
-}
+__device__ __forceinline__ unsigned op_char(uint32_t op) { return (0x00444958u >> (8u * (op & 3u))) & 0xFFu; }
 
-// Forward writer of the replay: consecutive bytes from position w0 of a
-// slot are combined into aligned 16-byte stores (a run of matches fills
-// whole chunks directly).  A chunk that reaches below w0 is written byte by
-// byte, and so is the partial chunk at the end (finish), so no byte outside
-// [w0, w) is touched: the neighbouring slots belong to other lanes.
-// Positions below w may sit in the chunk until it fills; the replay only
-// reads positions at or above w.
+// Forward writer of the replay from position w0 of a slot, in aligned 16-byte
+// stores (one lane per pair: a store of a wave touches 64 different lines).  The chunk holding position w starts out as matches, so a run of
+// matches is nothing but a step of w, and an operation one exclusive or.  A
+// chunk that reaches below w0 is written byte by byte, and so is the started
+// chunk at the end (finish): no byte outside [w0, w) is touched, the
+// neighbouring slots belong to other lanes.
 struct OpWriter {
+  static constexpr uint64_t kMatches = 0x4D4D4D4D4D4D4D4Dull;  // 'M'
   unsigned char* out;
   int w, w0;
-  OpChunk c;  // the chunk holding position w: its bytes below w
-  __device__ __forceinline__ unsigned phase() const { return chunk_phase(out + w); }
-  // The chunk [w - 16, w) is complete (w is 16-aligned).
-  __device__ __forceinline__ void flush() {
-    if (w - 16 >= w0) {
-      c.store(out + w - 16);
-    } else {
-      for (int i = w0; i < w; ++i) out[i] = (unsigned char)c.byte_at((unsigned)(i - (w - 16)));
-    }
-    c.clear();
-  }
-  __device__ __forceinline__ void put(unsigned op) {
-    const unsigned d = phase();
-    c.fill(d, d + 1, (op & 0xFFu) * 0x01010101u);
-    ++w;
-    if (d == 15u) flush();
-  }
-  // m copies of op: the rest of the current chunk, then whole chunks, then
-  // the beginning of the last one.
-  __device__ __forceinline__ void run(unsigned op, int m) {
-    if (m <= 0) return;
-    const uint32_t c4 = (op & 0xFFu) * 0x01010101u;
-    const unsigned d = phase();
-    if (d != 0u) {
-      const unsigned take = (unsigned)m < 16u - d ? (unsigned)m : 16u - d;
-      c.fill(d, d + take, c4);
-      w += (int)take;
-      m -= (int)take;
-      if (d + take < 16u) return;
-      flush();
-    }
-    for (; m >= 16; m -= 16, w += 16) *reinterpret_cast<uint4*>(out + w) = make_uint4(c4, c4, c4, c4);
-    if (m > 0) {
-      c.fill(0u, (unsigned)m, c4);
-      w += m;
+  uint64_t lo, hi;
+  __device__ __forceinline__ OpWriter(unsigned char* slot, int begin)
+      : out(slot), w(begin), w0(begin), lo(kMatches), hi(kMatches) {}
+  __device__ __forceinline__ int phase() const { return (int)(reinterpret_cast<uintptr_t>(out + w) & 15u); }
+  __device__ __forceinline__ void bytes(int base, int to) const {
+    for (int i = max(base, w0); i < to; ++i) {
+      const int b = i - base;
+      out[i] = (unsigned char)((b < 8 ? lo : hi) >> (8 * (b & 7)));
     }
   }
-  __device__ __forceinline__ void finish() {
-    const int d = (int)phase();
-    for (int i = max(w - d, w0); i < w; ++i) out[i] = (unsigned char)c.byte_at((unsigned)(i - (w - d)));
-    c.clear();
+  // Moves on by n bytes: what the chunk holds at them, matches beyond it.
+  __device__ __forceinline__ void advance(int n) {
+    int base = w - phase();
+    w += n;
+    if (w - base < 16) return;
+    if (base >= w0) *reinterpret_cast<ulonglong2*>(out + base) = make_ulonglong2(lo, hi);
+    else bytes(base, base + 16);
+    lo = hi = kMatches;
+    for (base += 16; w - base >= 16; base += 16)
+      *reinterpret_cast<ulonglong2*>(out + base) = make_ulonglong2(kMatches, kMatches);
   }
-};
-
-// Backward writer of the walk: bytes written at descending positions below
-// top are combined into aligned 16-byte stores.  A chunk that reaches top
-// (the bytes from top up belong to the trailing gaps or to another slot) is
-// written byte by byte, and so is the partial chunk at the end (finish).
-struct OpWriterBack {
-  unsigned char* out;
-  int p, top;
-  OpChunk c;  // the chunk holding position p: its bytes from p up
-  __device__ __forceinline__ void put(unsigned op) {
-    --p;
-    const unsigned d = chunk_phase(out + p);
-    c.fill(d, d + 1, (op & 0xFFu) * 0x01010101u);
-    if (d == 0u) {
-      if (p + 16 <= top) {
-        c.store(out + p);
-      } else {
-        for (int i = p; i < top; ++i) out[i] = (unsigned char)c.byte_at((unsigned)(i - p));
-      }
-      c.clear();
-    }
+  // One operation, then m matches.
+  __device__ __forceinline__ void put(unsigned op, int m) {
+    const int d = phase();
+    const uint64_t x = (uint64_t)(op ^ 0x4Du) << (8 * (d & 7));
+    lo ^= d < 8 ? x : 0u;
+    hi ^= d < 8 ? 0u : x;
+    advance(1 + m);
   }
-  __device__ __forceinline__ void finish() {
-    const int d = (int)chunk_phase(out + p);
-    if (d != 0) {
-      const int c0 = p - d;
-      for (int i = p; i < min(c0 + 16, top); ++i) out[i] = (unsigned char)c.byte_at((unsigned)(i - c0));
-    }
-    c.clear();
-  }
+  __device__ __forceinline__ void finish() const { bytes(w - phase(), w); }
 };
 
 // One lane per pair, in two passes over the pair's CIGAR slot
@@ -758,9 +707,9 @@ struct OpWriterBack {
 //  1. Walk back from the end cell to the origin over (score, diagonal,
 //     component) with the record bytes (wavefront_backtrace.c:320-529: the
 //     recorded source is the maximum of (offset << 4 | type) the reference
-//     takes).  Each mismatch, insertion or deletion is written backwards at
-//     the end of the slot, its top bit set when the cell it leads into is an
-//     M cell (an X, or the last operation of a gap that closes into M).
+//     takes).  Each mismatch, insertion or deletion goes on a stack in the
+//     end of the slot, marked when the cell it leads into is an M cell (an X,
+//     or the last operation of a gap that closes into M).
 //  2. Replay the operations forward from the origin, extending every M cell
 //     maximally (wavefront_extend_kernels.c:68-123, the same extension the
 //     forward pass made there), and write the full CIGAR into the end of the
@@ -770,6 +719,13 @@ struct OpWriterBack {
 // Near the matrix borders only gaps can reach a cell (offsets of valid M cells
 // are never negative), so walking to score 0 emits the same characters as the
 // reference's shortcut at v == 0 or h == 0.
+//
+// Bound by the chain of operations of one lane: its instructions, with the
+// lanes of a wave on different ones, and the loads of its records.  Hence the
+// stack of four-bit operations and the writer that only steps over matches
+// (150,000 reads of 100-300 bp: 132 us; with the operations kept as bytes and
+// the output filled run by run, 170 us; 20,000 of 500-1,000 bp: 243 and 346
+// us).  Reading the sequences a word ahead of the replay took 153 us.
 //
 // WAVE: the records of the wave family (wfa_wave.hip): no blocks to follow,
 // the word with a cell's byte is found from its step and diagonal, and the
@@ -811,7 +767,7 @@ __device__ __forceinline__ void trace_pair(const BacktraceArgs& a) {
   const int endrec = zd && a.end_rec ? a.end_rec[p] : 0;
   const int vE = zd ? a.end_off[p] - a.end_k[p] : 0, hE = zd ? a.end_off[p] : 0;
   const bool direct = zd && (endrec == 0xFF || vE <= 0 || hE <= 0 || s <= 0);
-  int ntrail_all = 0;
+  int ntrail_all = 0, ntrail_d = 0;
   if (a.endsfree || zd) {
     // Trailing gaps after the end cell (wavefront_backtrace.c:345-355): the
     // pattern's rest as deletions, then the text's rest as insertions.  A
@@ -826,6 +782,7 @@ __device__ __forceinline__ void trace_pair(const BacktraceArgs& a) {
     } else if (!zd || direct) {
       for (int i = 0; i < nd; ++i) out[--pos] = 'D';
       for (int i = 0; i < ni; ++i) out[--pos] = 'I';
+      ntrail_d = nd;
     }
   }
   const int ntrail = cap - pos;
@@ -844,28 +801,35 @@ __device__ __forceinline__ void trace_pair(const BacktraceArgs& a) {
   uint32_t blk = a.last_block[p];
   uint4 hdr = make_uint4(0, 0, 0, kNoBlock);  // WAVE: the units of the phases' records
   if (blk != kNoBlock && blk < a.rec_units) hdr = a.rec_arena[blk];
-  unsigned long long word_at = ~0ull;
+  unsigned long long word_at = ~0ull, base = 0;
   uint32_t word = 0;
-  OpWriterBack bw{out, pos, pos, OpChunk{}};
+  int ph = 0, begin = INT_MAX, k_first = 0;  // WAVE: the phase of the latest step read
+  OpStack walk(out + pos);
   while (s > 0 && !bad && !direct) {
-    if (bw.p <= 0) {
+    if (walk.n >= pos) {
       bad = true;
       break;
     }
     uint32_t rec;
     if constexpr (WAVE) {
       const int i = s - 1;
-      const int ph = (i >= a.wave_last[0] ? 1 : 0) + (i >= a.wave_last[1] ? 1 : 0) + (i >= a.wave_last[2] ? 1 : 0);
-      const int begin = ph == 0 ? 0 : ph == 1 ? a.wave_last[0] : ph == 2 ? a.wave_last[1] : a.wave_last[2];
-      const uint32_t base = ph == 0 ? hdr.x : ph == 1 ? hdr.y : ph == 2 ? hdr.z : hdr.w;
-      const int t = i - begin, kk = k - (a.wave_center - (32 << ph)), c = kk & ((1 << ph) - 1);
+      if (i < begin) {  // the phase of step i
+        ph = (i >= a.wave_last[0] ? 1 : 0) + (i >= a.wave_last[1] ? 1 : 0) + (i >= a.wave_last[2] ? 1 : 0);
+        begin = ph == 0 ? 0 : ph == 1 ? a.wave_last[0] : ph == 2 ? a.wave_last[1] : a.wave_last[2];
+        base = 4ull * (ph == 0 ? hdr.x : ph == 1 ? hdr.y : ph == 2 ? hdr.z : hdr.w);
+        k_first = a.wave_center - (32 << ph);
+      }
+      const int t = i - begin, kk = k - k_first;
       if (blk == kNoBlock || (unsigned)kk >= (64u << ph)) {
         bad = true;
         break;
       }
-      const int group = ph < 3 ? t >> (2 - ph) : 2 * t + (c >> 2);
-      const int byte = ph < 3 ? ((t & ((4 >> ph) - 1)) << ph) + c : c & 3;
-      const unsigned long long at = (unsigned long long)base * 4 + (unsigned)(group * 64 + (kk >> ph));
+      // phases 0 to 2: a word has 4 >> ph steps of the lane's 1 << ph cells;
+      // phase 3: a step has two words of four cells
+      const int sh = ph < 3 ? 2 - ph : 0;
+      const int group = ph < 3 ? t >> sh : 2 * t + ((kk >> 2) & 1);
+      const int byte = ph < 3 ? ((t & ((1 << sh) - 1)) << ph) + (kk & ((1 << ph) - 1)) : kk & 3;
+      const unsigned long long at = base + (unsigned)(group * 64 + (kk >> ph));
       if (at >= a.rec_units * 4) {
         bad = true;
         break;
@@ -904,7 +868,7 @@ __device__ __forceinline__ void trace_pair(const BacktraceArgs& a) {
     if (comp == kM) {
       switch (rec & kRecSrcMask) {
         case kSrcX:
-          bw.put('X' | (mark ? 0x80u : 0u));
+          walk.push(mark ? 4u : 0u);
           ++nx;
           s -= pen.x;
           mark = true;
@@ -919,7 +883,7 @@ __device__ __forceinline__ void trace_pair(const BacktraceArgs& a) {
     const bool ins = comp == kI1 || comp == kI2;
     const bool one = comp == kI1 || comp == kD1;
     const uint32_t ext_bit = comp == kI1 ? kRecI1Ext : comp == kD1 ? kRecD1Ext : comp == kI2 ? kRecI2Ext : kRecD2Ext;
-    bw.put((ins ? 'I' : 'D') | (mark ? 0x80u : 0u));
+    walk.push((ins ? 1u : 2u) | (mark ? 4u : 0u));
     ++nid;
     k += ins ? -1 : 1;
     if (rec & ext_bit) {
@@ -931,18 +895,16 @@ __device__ __forceinline__ void trace_pair(const BacktraceArgs& a) {
       mark = true;
     }
   }
-  bw.finish();
-  pos = bw.p;
+  const int nwalk = walk.n;
   // The walk ends at score 0: at the origin, or (ends-free) at a free
   // beginning cell (v=0, h=k) or (v=-k, h=0) of the score-0 wavefront.
   if (!bad && !direct && (s != 0 || comp != cbeg || (k != 0 && !a.endsfree))) bad = true;
   const int nlead = k < 0 ? -k : k;
-  int start = direct && !bad ? pos : cap;
+  int start = direct && !bad ? pos : cap;  // (the walk's stack lies below pos)
   const long long ppos = a.pat_pos[p], tpos = a.txt_pos[p];
   const uint64_t* P = a.words + ppos / SPW;
   const uint64_t* T = a.words + tpos / SPW;
   const int pb = (int)(ppos % SPW), tb = (int)(tpos % SPW);
-  const int last_walk = cap - ntrail - 1;  // the operation leading into the end cell
   // A z-drop's end cell: the reference writes the matches from the cell's
   // computed offset up to the best cell's offset whatever the bases
   // (wavefront_backtrace.c:77-98); a best offset behind the computed one
@@ -958,16 +920,14 @@ __device__ __forceinline__ void trace_pair(const BacktraceArgs& a) {
       h += m;
     };
     if (cbeg == kM) {
-      if (pos == cap - ntrail) q = h; else dry();
+      if (nwalk == 0) q = h; else dry();
     }
-    for (int i = pos; i < cap - ntrail; ++i) {
-      const unsigned char b = out[i];
-      const unsigned char op = b & 0x7F;
-      if (op == 'X') { ++v; ++h; }
-      else if (op == 'I') ++h;
-      else ++v;
-      if (b & 0x80) {
-        if (i == last_walk) q = h; else dry();
+    for (OpStack st = walk; st.n > 0;) {
+      const uint32_t op = st.pop();
+      v += (op & 3u) != 1u;
+      h += (op & 3u) != 2u;
+      if (op & 4u) {
+        if (st.n == 0) q = h; else dry();  // (the last operation leads into the end cell)
       }
     }
     const int n = a.end_off[p] - q;
@@ -981,64 +941,43 @@ __device__ __forceinline__ void trace_pair(const BacktraceArgs& a) {
     // A z-drop's CIGAR is counted from the dry run instead.
     int len;
     if (zd) {
-      len = zmatches + zrun + (cap - pos) + nlead;
+      len = zmatches + zrun + nwalk + ntrail + nlead;
       if (len > cap) bad = true;
     } else {
       const int rest = cap - 2 * nx - nid - ntrail - nlead;
       if (rest < 0 || (rest & 1)) bad = true;
-      len = bad ? 0 : rest / 2 + (cap - pos) + nlead;
+      len = bad ? 0 : rest / 2 + nwalk + ntrail + nlead;
     }
     start = bad ? cap : cap - len;
-    OpWriter ow{out, start, start, OpChunk{}};
+    OpWriter ow(out, start);
     int v = 0, h = 0;
     if (!bad) {
-      ow.run(k > 0 ? 'I' : 'D', nlead);  // free leading gaps
+      // free leading gaps
+      for (int i = 0; i < nlead; ++i) ow.put(k > 0 ? 'I' : 'D', 0);
       if (k > 0) h = k; else v = -k;
     }
-    auto extend = [&]() {
-      const int h2 = lcp_extend<BITS>(P, pb, T, tb, plen, tlen, h - v, h);
-      const int m = h2 - h;
-      if (ow.w + m > cap) { bad = true; return; }
-      ow.run('M', m);
+    // The matches at (v, h), or a z-drop's last run; bad when the slot cannot hold them.
+    auto matches = [&](bool end, int before) {
+      const int m = end ? zrun : lcp_extend<BITS>(P, pb, T, tb, plen, tlen, h - v, h) - h;
+      if (ow.w + before + m > cap) bad = true;
       v += m;
       h += m;
+      return bad ? 0 : m;
     };
-    auto run_to_end = [&]() {
-      if (ow.w + zrun > cap) { bad = true; return; }
-      ow.run('M', zrun);
-      v += zrun;
-      h += zrun;
-    };
-    if (!bad && cbeg == kM) {
-      if (zd && pos == cap - ntrail) run_to_end(); else extend();
-    }
-    // The operations are read 16 bytes at a time: an aligned 16-byte chunk
-    // that holds a byte of the slot lies in the same page as that byte.
-    // Bytes of the cached chunk below the position read may since have been
-    // overwritten by the writer (which stays below it); they are not read
-    // again.
-    uintptr_t cached = ~(uintptr_t)0;
-    uint4 chunk = make_uint4(0u, 0u, 0u, 0u);
-    for (int i = pos; i < cap && !bad; ++i) {
-      const uintptr_t ad = reinterpret_cast<uintptr_t>(out + i);
-      const unsigned o = (unsigned)(ad & 15u);
-      if ((ad & ~(uintptr_t)15) != cached) {
-        cached = ad & ~(uintptr_t)15;
-        chunk = *reinterpret_cast<const uint4*>(out + (i - (int)o));
-      }
-      const uint32_t lo = (o & 4u) ? chunk.y : chunk.x, hi = (o & 4u) ? chunk.w : chunk.z;
-      const unsigned char b = (unsigned char)(((o & 8u) ? hi : lo) >> (8u * (o & 3u)));
-      const unsigned char op = b & 0x7F;
-      if (ow.w > i) { bad = true; break; }  // inconsistent records: never overrun unread operations
-      ow.put(op);
-      if (op == 'X') { ++v; ++h; }
-      else if (op == 'I') ++h;
-      else ++v;
-      if (b & 0x80) {
-        if (zd && i == last_walk) run_to_end(); else extend();
-      }
+    if (!bad && cbeg == kM) ow.advance(matches(zd && nwalk == 0, 0));
+    while (walk.n > 0 && !bad) {
+      if (ow.w > cap - ntrail - walk.n) { bad = true; break; }  // inconsistent records: never overrun unread operations
+      const uint32_t op = walk.pop();
+      v += (op & 3u) != 1u;
+      h += (op & 3u) != 2u;
+      const int m = (op & 4u) ? matches(zd && walk.n == 0, 1) : 0;
+      ow.put(op_char(op), m);
     }
     ow.finish();
+    // the trailing gaps are in place
+    ow.w += ntrail;
+    v += ntrail_d;
+    h += ntrail - ntrail_d;
     // the end: (plen, tlen), or a z-drop's end cell moved by what it takes back
     if (!bad && (v != (zd ? vE + zback : plen) || h != (zd ? hE + zback : tlen) || ow.w != cap)) bad = true;
   }
@@ -1055,11 +994,11 @@ __device__ __forceinline__ void trace_pair(const BacktraceArgs& a) {
 }
 
 template <int BITS>
-__global__ void __launch_bounds__(256) wfa_backtrace_kernel(BacktraceArgs a) {
+__global__ void __launch_bounds__(64) wfa_backtrace_kernel(BacktraceArgs a) {
   trace_pair<BITS, false>(a);
 }
 template <int BITS>
-__global__ void __launch_bounds__(256) wfa_wave_backtrace_kernel(BacktraceArgs a) {
+__global__ void __launch_bounds__(64) wfa_wave_backtrace_kernel(BacktraceArgs a) {
   trace_pair<BITS, true>(a);
 }
 
@@ -1148,7 +1087,7 @@ hipError_t launch_forward(const ForwardArgs& a, int ncomp, int bits, const Launc
 
 hipError_t launch_backtrace(const BacktraceArgs& a, hipStream_t stream) {
   if (a.n_pairs <= 0) return hipSuccess;
-  const int block = 256;
+  const int block = 64;  // a lane's chain of operations decides: waves spread over as many CUs as there are
   const int grid = (a.n_pairs + block - 1) / block;
   if (a.bits != 2 && a.bits != 8) return hipErrorInvalidValue;
   if (a.wave) {
