@@ -742,7 +742,8 @@ LaunchShape shape_of(Engine* e, const PlanGroup& g, int bits, const Penalties& p
   int per_cu = 0;
   if (g.family == wfa::kWave) {
     shape.lds_bytes = wfa::wave_lds_bytes(g.lmax_words);
-    per_cu = wfa::wave_max_blocks_per_cu(wfa::wave_shape(pen), g.wcap, g.wave_rec, bits, g.wave_ef, shape.lds_bytes);
+    per_cu = wfa::wave_max_blocks_per_cu(wfa::wave_shape(pen), g.wcap, g.wave_rec, bits, g.wave_ef,
+                                         g.wave.cut, shape.lds_bytes);
   } else if (g.family == wfa::kLean) {
     shape.lds_bytes = wfa::lean_lds_bytes(pen, g.wcap, g.lmax_words);
     per_cu = wfa::lean_max_blocks_per_cu(pen, g.wcap, shape.lds_bytes);
@@ -847,6 +848,7 @@ void group_args(wavefront_aligner_t* wf, Engine* e, const JobSet& js, const Plan
     ba.wave = pen.ncomp;
     for (int ph = 0; ph < wfa::kWavePhases; ++ph) ba.wave_last[ph] = grp.wave.last[ph];
     ba.wave_center = grp.wave.center;
+    ba.wave_cut = grp.wave.cut;
   }
   *pba = ba;
 }
@@ -856,7 +858,8 @@ void set_wave(const JobSet& js, PlanGroup& g, const Penalties& pen, int records)
   if (g.family != wfa::kWave) return;
   g.wave_rec = records != 0;
   g.wave_ef = js.ef.on != 0;
-  (void)wfa::wave_phases(wfa::wave_shape(pen), js.ef.on ? js.ef.pbf : 0, js.ef.on ? js.ef.tbf : 0, g.wcap, &g.wave);
+  if (js.heur.cut()) wfa::wave_cut_phases(&g.wave);
+  else (void)wfa::wave_phases(wfa::wave_shape(pen), js.ef.on ? js.ef.pbf : 0, js.ef.on ? js.ef.tbf : 0, g.wcap, &g.wave);
 }
 
 // Forward (and, with records, backtrace) launches of one group, with the
@@ -958,9 +961,16 @@ std::vector<PlanGroup> make_plan(const JobSet& js, const std::vector<int>& ids, 
   const bool tile_ok = js.tiles && js.bits == 2 && !js.cbeg && !js.cend && !js.ef.on && js.heur.cut() == 0 &&
                        wfa::tile_shape(pen) != 0;
   // Pairs of at most 1,024 bases on the wave family where it has an instance:
-  // up to 4 diagonals per lane for the short class, 8 above.
+  // up to 4 diagonals per lane for the short class, 8 above.  With wf-adaptive
+  // alone (gap-affine, 2-bit, end-to-end) too: against the lean family 2.04 and
+  // 1.49 ms for 100,000 reads of 100-300 bp, 1.85 and 1.64 ms for 20,000 of
+  // 500-1,000 bp, 2.51 and 2.44 ms for those at 8-10% errors, whose wavefronts
+  // often leave 64 diagonals.  Bands and drops stay on the lean and ring
+  // families.
   wfa::WaveArgs wa;
-  const bool wave_ok = lt.enabled && js.unlimited && !js.cbeg && !js.cend && js.heur.cut() == 0 &&
+  const bool cut = js.heur.cut() != 0;
+  const bool wave_ok = lt.enabled && js.unlimited && !js.cbeg && !js.cend &&
+                       (!cut || (wfa::wave_cuts(wfa::wave_shape(pen), js.heur) && js.bits == 2 && !js.ef.on)) &&
                        (js.bits == 2 || js.nibbles) && wfa::wave_shape(pen) != 0 &&
                        wfa::wave_phases(wfa::wave_shape(pen), js.ef.on ? js.ef.pbf : 0, js.ef.on ? js.ef.tbf : 0, 4, &wa);
   int wave_words[2] = {0, 0};
@@ -997,7 +1007,7 @@ std::vector<PlanGroup> make_plan(const JobSet& js, const std::vector<int>& ids, 
     PlanGroup g;
     g.family = wfa::kWave;
     g.block = 64;
-    g.wcap = c == 0 ? 4 : 8;
+    g.wcap = cut ? 1 : c == 0 ? 4 : 8;
     g.lmax_words = wave_words[c];
     g.ids = std::move(wave_ids[c]);
     plan.push_back(std::move(g));
@@ -1112,7 +1122,8 @@ int run_jobs(wavefront_aligner_t* wf, Engine* e, const JobSet& js, std::vector<P
         else if (h_status[i] == wfa::kDevArenaFull) arena_full.push_back(i);
       }
       if (!ring_over.empty()) {
-        if (g.family == wfa::kWave && g.wcap < 8) {
+        const bool cut = js.heur.cut() != 0;
+        if (g.family == wfa::kWave && g.wcap < 8 && !cut) {
           PlanGroup h = take_group(e);
           h.family = wfa::kWave;
           h.block = 64;
@@ -1129,7 +1140,7 @@ int run_jobs(wavefront_aligner_t* wf, Engine* e, const JobSet& js, std::vector<P
           PlanGroup h = take_group(e);
           h.family = wfa::kLean;
           h.block = 64;
-          h.wcap = wfa::lean_width(kLeanMaxRing);
+          h.wcap = wfa::lean_width(cut ? lean_tuning().wcap_long : kLeanMaxRing);
           h.lmax_words = (g.lmax_words + 1) / 2;
           h.ids = std::move(ring_over);
           next.push_back(std::move(h));

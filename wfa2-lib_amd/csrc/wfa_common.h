@@ -448,6 +448,20 @@ __device__ __forceinline__ int end_distance(int off, int k, int plen, int tlen, 
   return max(left_v, left_h);
 }
 
+// Minimum over the 64 lanes, uniform: prefix minima within each row of 16
+// lanes by row shifts of 1, 2, 4 and 8 (a lane without a source keeps
+// INT_MAX), then the rows joined by the row broadcasts of lanes 15 and 31;
+// lane 63 ends with the minimum of all.
+__device__ __forceinline__ int wave_min(int v) {
+  v = min(v, __builtin_amdgcn_update_dpp(INT_MAX, v, 0x111, 0xf, 0xf, false));  // row_shr:1
+  v = min(v, __builtin_amdgcn_update_dpp(INT_MAX, v, 0x112, 0xf, 0xf, false));  // row_shr:2
+  v = min(v, __builtin_amdgcn_update_dpp(INT_MAX, v, 0x114, 0xf, 0xf, false));  // row_shr:4
+  v = min(v, __builtin_amdgcn_update_dpp(INT_MAX, v, 0x118, 0xf, 0xf, false));  // row_shr:8
+  v = min(v, __builtin_amdgcn_update_dpp(INT_MAX, v, 0x142, 0xa, 0xf, false));  // row_bcast:15 into rows 1, 3
+  v = min(v, __builtin_amdgcn_update_dpp(INT_MAX, v, 0x143, 0xc, 0xf, false));  // row_bcast:31 into rows 2, 3
+  return __builtin_amdgcn_readlane(v, 63);
+}
+
 // wf-adaptive cut-off (wavefront_heuristic_wfadaptive and its reduce step,
 // wavefront_heuristic.c:190-290) of the extended M wavefront [lo, hi], whose
 // diagonal k holds m[k]: keeps the diagonals whose distance to the end (plain,

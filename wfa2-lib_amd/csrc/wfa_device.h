@@ -104,8 +104,14 @@ struct WaveArgs {
   int last[kWavePhases];       // steps done when each phase ends (its wavefronts fit the wave)
   int center;                  // diagonal of lane 32
   int phase0;                  // phase that holds the score-0 wavefront
+  int cut;                     // with a cut-off: `last` are segments of steps, and a pair's records have
+                               // one or two diagonals per lane, centred per pair
   int lds_words;               // LDS words (32-bit) per sequence
 };
+
+constexpr int kWaveCutSegments = 3;
+// Diagonal of lane 32 of a pair that ends on diagonal kend (WaveArgs::cut).
+__host__ __device__ inline int wave_cut_center(int kend) { return kend / 2; }
 
 struct ForwardArgs {
   int n_pairs;
@@ -180,8 +186,9 @@ struct BacktraceArgs {
   const int* end_off;
   const int* end_rec;          // z-drop: the end cell's record byte (0xFF: no source)
   int wave;                    // records of the wave family: its components (1, 3 or 5), else 0
-  int wave_last[kWavePhases];  // WaveArgs::last and center
+  int wave_last[kWavePhases];  // WaveArgs::last, center and cut
   int wave_center;
+  int wave_cut;
   Penalties pen;
 };
 

@@ -803,7 +803,7 @@ __device__ __forceinline__ void trace_pair(const BacktraceArgs& a) {
   if (blk != kNoBlock && blk < a.rec_units) hdr = a.rec_arena[blk];
   unsigned long long word_at = ~0ull, base = 0;
   uint32_t word = 0;
-  int ph = 0, begin = INT_MAX, k_first = 0;  // WAVE: the phase of the latest step read
+  int ph = 0, wd = 0, begin = INT_MAX, k_first = 0;  // WAVE: the phase of the latest step read
   OpStack walk(out + pos);
   while (s > 0 && !bad && !direct) {
     if (walk.n >= pos) {
@@ -817,19 +817,20 @@ __device__ __forceinline__ void trace_pair(const BacktraceArgs& a) {
         ph = (i >= a.wave_last[0] ? 1 : 0) + (i >= a.wave_last[1] ? 1 : 0) + (i >= a.wave_last[2] ? 1 : 0);
         begin = ph == 0 ? 0 : ph == 1 ? a.wave_last[0] : ph == 2 ? a.wave_last[1] : a.wave_last[2];
         base = 4ull * (ph == 0 ? hdr.x : ph == 1 ? hdr.y : ph == 2 ? hdr.z : hdr.w);
-        k_first = a.wave_center - (32 << ph);
+        wd = a.wave_cut ? (int)hdr.w : ph;
+        k_first = (a.wave_cut ? wave_cut_center(tlen - plen) : a.wave_center) - (32 << wd);
       }
       const int t = i - begin, kk = k - k_first;
-      if (blk == kNoBlock || (unsigned)kk >= (64u << ph)) {
+      if (blk == kNoBlock || (unsigned)kk >= (64u << wd)) {
         bad = true;
         break;
       }
-      // phases 0 to 2: a word has 4 >> ph steps of the lane's 1 << ph cells;
-      // phase 3: a step has two words of four cells
-      const int sh = ph < 3 ? 2 - ph : 0;
-      const int group = ph < 3 ? t >> sh : 2 * t + ((kk >> 2) & 1);
-      const int byte = ph < 3 ? ((t & ((1 << sh) - 1)) << ph) + (kk & ((1 << ph) - 1)) : kk & 3;
-      const unsigned long long at = base + (unsigned)(group * 64 + (kk >> ph));
+      // up to four diagonals per lane: a word has 4 >> wd steps of the lane's
+      // 1 << wd cells; eight: a step has two words of four cells
+      const int sh = wd < 3 ? 2 - wd : 0;
+      const int group = wd < 3 ? t >> sh : 2 * t + ((kk >> 2) & 1);
+      const int byte = wd < 3 ? ((t & ((1 << sh) - 1)) << wd) + (kk & ((1 << wd) - 1)) : kk & 3;
+      const unsigned long long at = base + (unsigned)(group * 64 + (kk >> wd));
       if (at >= a.rec_units * 4) {
         bad = true;
         break;
@@ -843,8 +844,8 @@ __device__ __forceinline__ void trace_pair(const BacktraceArgs& a) {
         // source 4 X, 3 D2, 2 D1, 1 I2, 0 I1 in bits 1..3; flags of I1, D1, I2, D2 from bit 4
         rec = (4u - ((b >> 1) & 7u)) | (((b >> 4) & 15u) << 3);
       } else {
-        // source 2 X, 1 D1, 0 I1 in bits 1..2; flags of I1 and D1 in bits 6 and 7
-        rec = 4u - (b & 6u);
+        // source 3 stale, 2 X, 1 D1, 0 I1 in bits 1..2; flags of I1 and D1 in bits 6 and 7
+        rec = (b & 6u) == 6u ? kRecStale : 4u - (b & 6u);
         if (a.wave == 3) rec |= ((b >> 6) & 3u) << 3;
       }
     } else if (first) {

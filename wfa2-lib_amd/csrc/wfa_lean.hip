@@ -78,20 +78,6 @@ __device__ __forceinline__ int lean_rd_g(const int16_t* ring, const LeanSrc& s, 
   return c == k ? v : (int)kRingNull;
 }
 
-// Minimum over the 64 lanes, uniform: prefix minima within each row of 16
-// lanes by row shifts of 1, 2, 4 and 8 (a lane without a source keeps
-// INT_MAX), then the rows joined by the row broadcasts of lanes 15 and 31;
-// lane 63 ends with the minimum of all.
-__device__ __forceinline__ int wave_min(int v) {
-  v = min(v, __builtin_amdgcn_update_dpp(INT_MAX, v, 0x111, 0xf, 0xf, false));  // row_shr:1
-  v = min(v, __builtin_amdgcn_update_dpp(INT_MAX, v, 0x112, 0xf, 0xf, false));  // row_shr:2
-  v = min(v, __builtin_amdgcn_update_dpp(INT_MAX, v, 0x114, 0xf, 0xf, false));  // row_shr:4
-  v = min(v, __builtin_amdgcn_update_dpp(INT_MAX, v, 0x118, 0xf, 0xf, false));  // row_shr:8
-  v = min(v, __builtin_amdgcn_update_dpp(INT_MAX, v, 0x142, 0xa, 0xf, false));  // row_bcast:15 into rows 1, 3
-  v = min(v, __builtin_amdgcn_update_dpp(INT_MAX, v, 0x143, 0xc, 0xf, false));  // row_bcast:31 into rows 2, 3
-  return __builtin_amdgcn_readlane(v, 63);
-}
-
 // The choices of cell k over clamp-read sources (winning M offset, its
 // source, the gap-extension flags), ties as the compute step breaks them;
 // reads below 0 count as the one NULL offset (the generic kernel's

@@ -46,6 +46,7 @@ __device__ __forceinline__ int first_diagonal(uint32_t bits, int kt) {
   const unsigned long long bal = __ballot(bits != 0);
   if (!bal) return INT_MAX;
   const int l = (int)__builtin_ctzll(bal);
+  if constexpr (N == 1) return kt + l;
   return kt + N * l + (int)__builtin_ctz((unsigned)lane_of((int)bits, l));
 }
 template <int N>
@@ -53,6 +54,7 @@ __device__ __forceinline__ int last_diagonal(uint32_t bits, int kt) {
   const unsigned long long bal = __ballot(bits != 0);
   if (!bal) return INT_MIN;
   const int l = 63 - (int)__builtin_clzll(bal);
+  if constexpr (N == 1) return kt + l;
   return kt + N * l + 31 - (int)__builtin_clz((unsigned)lane_of((int)bits, l));
 }
 

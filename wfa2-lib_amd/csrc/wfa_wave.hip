@@ -366,6 +366,21 @@ __device__ __forceinline__ bool wave_start(WavePair& p, WaveRows<S, N>& w, const
   return b != 0;
 }
 
+// The 2-bit sequences of pair id into LDS.
+__device__ __forceinline__ void stage_sequences(WaveSeqs<2>& q, KernArgs A, int id, uint32_t* seqP, uint32_t* seqT) {
+  const int lane = threadIdx.x & 63;
+  const long long ppos = A->pat_pos[id], tpos = A->txt_pos[id];
+  q.pbit = 2u * (unsigned)(ppos & 31);
+  q.tbit = 2u * (unsigned)(tpos & 31);
+  const uint64_t* gP = A->words + (ppos >> 5);
+  const uint64_t* gT = A->words + (tpos >> 5);
+  const int nwp = ((int)(ppos & 31) + q.plen) / 32 + 2, nwt = ((int)(tpos & 31) + q.tlen) / 32 + 2;
+  uint64_t* dP = reinterpret_cast<uint64_t*>(seqP);
+  uint64_t* dT = reinterpret_cast<uint64_t*>(seqT);
+  for (int x = lane; x < nwp; x += 64) dP[x] = gP[x];
+  for (int x = lane; x < nwt; x += 64) dT[x] = gT[x];
+}
+
 // NMAX: most diagonals per lane (4: pairs up to 254 diagonals, 8: 510).
 // SRC: bits per symbol of the packed sequences in memory.  8-bit symbols that
 // differ in their low four bits are kept as 4-bit ones in LDS.
@@ -402,20 +417,12 @@ __global__ void __launch_bounds__(64, S::NC == 5 ? (NMAX == 8 ? 2 : 3) : (NMAX =
     p.end_k = p.kend;
     p.end_off = p.tlen;
     for (int x = 0; x < kWavePhases; ++x) p.base[x] = 0;
-    const long long ppos = A->pat_pos[id], tpos = A->txt_pos[id];
     WaveSeqs<BITS> q{seqP, seqT, 0u, 0u, p.plen, p.tlen};
     wave_sync();  // the previous pair is done reading the sequences
     if constexpr (SRC == 2) {
-      q.pbit = 2u * (unsigned)(ppos & 31);
-      q.tbit = 2u * (unsigned)(tpos & 31);
-      const uint64_t* gP = A->words + (ppos >> 5);
-      const uint64_t* gT = A->words + (tpos >> 5);
-      const int nwp = ((int)(ppos & 31) + p.plen) / 32 + 2, nwt = ((int)(tpos & 31) + p.tlen) / 32 + 2;
-      uint64_t* dP = reinterpret_cast<uint64_t*>(seqP);
-      uint64_t* dT = reinterpret_cast<uint64_t*>(seqT);
-      for (int x = lane; x < nwp; x += 64) dP[x] = gP[x];
-      for (int x = lane; x < nwt; x += 64) dT[x] = gT[x];
+      stage_sequences(q, A, id, seqP, seqT);
     } else {
+      const long long ppos = A->pat_pos[id], tpos = A->txt_pos[id];
       q.pbit = 4u * (unsigned)(ppos & 7);
       q.tbit = 4u * (unsigned)(tpos & 7);
       // eight bytes to eight nibbles
@@ -487,6 +494,367 @@ __global__ void __launch_bounds__(64, S::NC == 5 ? (NMAX == 8 ? 2 : 3) : (NMAX =
   if (lane == 0 && wg_dsteps) atomicAdd(args_now()->dsteps_total, wg_dsteps);
 }
 
+// A set of the wave's 64 * N diagonals, counted from the first: bit l of w[c]
+// is diagonal N * l + c.
+template <int N>
+struct Diagonals {
+  uint64_t w[N];
+  static __device__ __forceinline__ Diagonals none() {
+    Diagonals r;
+#pragma unroll
+    for (int c = 0; c < N; ++c) r.w[c] = 0;
+    return r;
+  }
+  // (not empty)
+  static __device__ __forceinline__ Diagonals range(int first, int last) {
+    Diagonals r;
+#pragma unroll
+    for (int c = 0; c < N; ++c) {
+      const int f = (first - c + N - 1) / N, l = last < c ? -1 : (last - c) / N;
+      r.w[c] = N == 1 || f <= l ? (~0ull >> (63 - (l - f))) << f : 0ull;
+    }
+    return r;
+  }
+  __device__ __forceinline__ bool any() const {
+    uint64_t r = 0;
+#pragma unroll
+    for (int c = 0; c < N; ++c) r |= w[c];
+    return r != 0;
+  }
+  // (of a set that is not empty)
+  __device__ __forceinline__ int first() const {
+    if constexpr (N == 1) return (int)__builtin_ctzll(w[0]);
+    int r = INT_MAX;
+#pragma unroll
+    for (int c = 0; c < N; ++c) r = min(r, w[c] ? N * (int)__builtin_ctzll(w[c]) + c : INT_MAX);
+    return r;
+  }
+  __device__ __forceinline__ int last() const {
+    if constexpr (N == 1) return 63 - (int)__builtin_clzll(w[0]);
+    int r = -1;
+#pragma unroll
+    for (int c = 0; c < N; ++c) r = max(r, w[c] ? N * (63 - (int)__builtin_clzll(w[c])) + c : -1);
+    return r;
+  }
+  __device__ __forceinline__ Diagonals hull() const { return any() ? range(first(), last()) : none(); }
+  __device__ __forceinline__ Diagonals up() const {  // each diagonal's set bit on the next
+    Diagonals r;
+#pragma unroll
+    for (int c = 0; c < N; ++c) r.w[c] = c ? w[c > 0 ? c - 1 : 0] : w[N - 1] << 1;
+    return r;
+  }
+  __device__ __forceinline__ Diagonals down() const {
+    Diagonals r;
+#pragma unroll
+    for (int c = 0; c < N; ++c) r.w[c] = c + 1 < N ? w[c + 1 < N ? c + 1 : 0] : w[0] >> 1;
+    return r;
+  }
+  __device__ __forceinline__ Diagonals operator|(const Diagonals& o) const {
+    Diagonals r;
+#pragma unroll
+    for (int c = 0; c < N; ++c) r.w[c] = w[c] | o.w[c];
+    return r;
+  }
+  __device__ __forceinline__ Diagonals operator&(const Diagonals& o) const {
+    Diagonals r;
+#pragma unroll
+    for (int c = 0; c < N; ++c) r.w[c] = w[c] & o.w[c];
+    return r;
+  }
+  __device__ __forceinline__ bool edges() const { return ((w[0] & 1ull) | (w[N - 1] >> 63)) != 0; }
+  __device__ __forceinline__ bool mine(int c) const { return (w[c] >> (threadIdx.x & 63)) & 1u; }
+};
+
+// The choices of a lane's cells: their best tagged values, and the record bytes.
+template <class S, int N>
+__device__ __forceinline__ uint32_t cell_choices(const int* mx, const int* mo, const int* i1, const int* d1, int* best) {
+  constexpr int ONE = 1 << S::SH;
+  int a[N], b[N];
+#pragma unroll
+  for (int c = 0; c < N; ++c) {
+    a[c] = max(mo[c], i1[c]);
+    b[c] = max(mo[c], d1[c]);
+  }
+  const int al = from_lower_lane(a[N - 1]), bu = from_upper_lane(b[0]);
+  uint32_t bytes = 0;
+#pragma unroll
+  for (int c = 0; c < N; ++c) {
+    const int ins = (c ? a[c > 0 ? c - 1 : 0] : al) + ONE;
+    const int del = (c + 1 < N ? b[c + 1 < N ? c + 1 : 0] : bu) + 2 * S::kTagD1;
+    best[c] = max(max(ins, del), mx[c] + ONE + 2 * S::kTagX);
+    bytes |= (((uint32_t)best[c] & 63u) | (((uint32_t)ins & 1u) << 6) | (((uint32_t)del & 1u) << 7)) << (8 * c);
+  }
+  return bytes;
+}
+
+// One pair with the wf-adaptive cut-off on N diagonals per lane, the middle
+// between its score-0 and its end diagonal in the middle of the wave.
+// Returns the status; kDevRingOverflow when the pair leaves the wave's
+// diagonals or its steps.
+template <class S, int N, bool REC>
+__device__ __forceinline__ int cut_pair(const WaveSeqs<2>& q, WaveChunk& ch, uint32_t* base, int& steps, int& dsteps) {
+  static_assert(S::NC == 3 && S::DE1 == 1 && S::RM == 4 && N <= 2, "gap-affine");
+  using D = Diagonals<N>;
+  constexpr int G = 4 / N;  // steps per record word
+  KernArgs A = args_now();
+  const int lane = threadIdx.x & 63;
+  const int plen = q.plen, tlen = q.tlen, kend = tlen - plen;
+  const int kt = wave_cut_center(kend) - 32 * N, k0 = kt + N * lane;
+  const int z = -kt, ke = kend - kt;  // diagonal 0 and the end diagonal within the wave
+  steps = dsteps = 0;
+  if (z < 1 || z > 64 * N - 2) return kDevRingOverflow;
+  // rows (newest first) and what the cut-off left of them
+  WaveRows<S, N> w;
+  D rm[S::RM], ri = D::none(), rd = D::none();
+  int h0 = 0, n0 = 0;
+  do {
+    const int r = min(plen, tlen) - h0;
+    n0 = r > 0 ? uniform(q.run(h0, h0, r)) : 0;
+    h0 += n0;
+  } while (n0 == WaveSeqs<2>::kSpan);
+  if (kend == 0 && h0 >= tlen) return kDevCompleted;
+#pragma unroll
+  for (int r = 0; r < S::RM; ++r) {
+    rm[r] = r ? D::none() : D::range(z, z);
+#pragma unroll
+    for (int c = 0; c < N; ++c) w.m[r][c] = r == 0 && k0 + c == 0 ? h0 << S::SH : kNullTagged;
+  }
+  uint32_t endm = 0;
+#pragma unroll
+  for (int c = 0; c < N; ++c) {
+    w.i1[0][c] = w.d1[0][c] = kNullTagged;
+    endm |= k0 + c == kend ? 1u << c : 0u;
+  }
+  int wait = A->heur.steps - 1;
+  if (wait <= 0 && A->heur.min_len <= 1) wait = A->heur.steps;  // (a single diagonal is never cut)
+  StepCells<N> cell;
+  cell.rec[0] = 0;
+  uint32_t* rec = nullptr;
+  int seg = -1, first = 0, last = 0, i = 0;
+  bool probe = false;  // the last step's I1 or D1 was emptied: its cells are in pi, pd
+  int pi[N], pd[N];
+  int status = kDevRingOverflow;
+  for (;;) {
+    if (i == last) {  // the next segment of records
+      if (++seg == kWaveCutSegments) {
+        steps = i;
+        return kDevRingOverflow;
+      }
+      KernArgs B = args_now();
+      first = last;
+      last = B->wave.last[seg];
+      if constexpr (REC) {
+        const uint32_t units = (uint32_t)((last - first) / G) * 16u;
+        if (!reserve_records(ch, units)) return kDevArenaFull;
+#pragma unroll
+        for (int x = 0; x < kWaveCutSegments; ++x) base[x] = x == seg ? ch.cur : base[x];
+        rec = reinterpret_cast<uint32_t*>(B->rec_arena + ch.cur) + lane;
+        ch.cur += units;  // (what is not used goes back at the end)
+      }
+    }
+    // wavefront_compute_limits_input (wavefront_compute.c:40-86)
+    const D mo = rm[S::DO1 - 1];
+    const D reach = rm[S::DX - 1] | mo.up() | mo.down() | ri.up() | rd.down();
+    D in = D::none();
+    if (reach.any()) {
+      int lo = reach.first(), hi = reach.last();
+      if (lo > z || hi < z) {
+        // a null source still contributes the limits (1, -1), shifted as its gap moves it
+        if (!rm[S::DX - 1].any()) { lo = min(lo, z + 1); hi = max(hi, z - 1); }
+        if (!mo.any()) { lo = min(lo, z); hi = max(hi, z); }
+        if (!ri.any()) { lo = min(lo, z + 2); hi = max(hi, z); }
+        if (!rd.any()) { lo = min(lo, z); hi = max(hi, z - 2); }
+      }
+      in = D::range(lo, hi);
+      dsteps += hi - lo + 1;
+    }
+    int chosen[N], probed[N], m[N];
+    uint32_t bytes = 0;
+    if (REC && probe) {
+      (void)cell_choices<S, N>(w.m[S::DX - 1], w.m[S::DO1 - 1], w.i1[0], w.d1[0], chosen);
+      bytes = cell_choices<S, N>(w.m[S::DX - 1], w.m[S::DO1 - 1], pi, pd, probed);
+    }
+    wave_cells<S, N, 2>(w.m[S::DX - 1], w.m[S::DO1 - 1], w.i1[0], w.d1[0], nullptr, nullptr, nullptr, m, k0, q, cell);
+    if (REC && probe) {
+      probe = false;
+#pragma unroll
+      for (int c = 0; c < N; ++c)  // (source 3: a trace through the cell would take operations back)
+        if ((probed[c] >= 0) & ((probed[c] >> S::SH) > max(chosen[c], m[c]) >> S::SH)) bytes |= 6u << (8 * c);
+      cell.rec[0] = (cell.rec[0] & ((1u << (32 - 8 * N)) - 1u)) | (bytes << (32 - 8 * N));
+    }
+    D bm, bi, bd;
+    bool out = false, fin = false;
+#pragma unroll
+    for (int c = 0; c < N; ++c) {
+      const bool mine = in.mine(c);
+      m[c] = mine ? m[c] : kNullTagged;
+      w.i1[0][c] = mine ? w.i1[0][c] : kNullTagged;
+      w.d1[0][c] = mine ? w.d1[0][c] : kNullTagged;
+      bm.w[c] = __ballot(m[c] >= 0);
+      bi.w[c] = __ballot(w.i1[0][c] >= 0);
+      bd.w[c] = __ballot(w.d1[0][c] >= 0);
+      out |= cell.oob[c] & mine;
+      fin |= (((endm >> c) & 1u) != 0) & (m[c] >= (tlen << S::SH));
+    }
+#pragma unroll
+    for (int r = S::RM - 1; r > 0; --r) {
+      rm[r] = rm[r - 1];
+#pragma unroll
+      for (int c = 0; c < N; ++c) w.m[r][c] = w.m[r - 1][c];
+    }
+#pragma unroll
+    for (int c = 0; c < N; ++c) w.m[0][c] = m[c];
+    ++i;
+    if constexpr (REC) {
+      if (((i - first) & (G - 1)) == 0) {
+        *rec = cell.rec[0];
+        rec += 64;
+      }
+    }
+    if (__ballot(out)) {
+      // gap cells outside the matrix: not in the trimmed ranges, and NULL
+      // beyond them (wavefront_compute.c:498-613)
+#pragma unroll
+      for (int c = 0; c < N; ++c) {
+        bi.w[c] = __ballot(in_bounds(w.i1[0][c] >> S::SH, k0 + c, plen, tlen));
+        bd.w[c] = __ballot(in_bounds(w.d1[0][c] >> S::SH, k0 + c, plen, tlen));
+      }
+      const D hi = bi.hull(), hd = bd.hull();
+#pragma unroll
+      for (int c = 0; c < N; ++c) {
+        w.i1[0][c] = hi.mine(c) ? w.i1[0][c] : kNullTagged;
+        w.d1[0][c] = hd.mine(c) ? w.d1[0][c] : kNullTagged;
+      }
+    }
+    if (__ballot(fin)) {
+      status = kDevCompleted;
+      break;
+    }
+    if ((bm | bi | bd).edges()) break;  // (the outermost diagonals have no neighbour)
+    rm[0] = bm;
+    ri = bi;
+    rd = bd;
+    if (bm.any() && --wait <= 0) {
+      KernArgs B = args_now();
+      const int lo = bm.first(), hi = bm.last();
+      if (hi - lo + 1 >= B->heur.min_len) {
+        wait = B->heur.steps;
+        int d[N], dmin = kNullDistance;
+#pragma unroll
+        for (int c = 0; c < N; ++c) {
+          const int h = m[c] >> S::SH;
+          d[c] = m[c] >= 0 ? max(plen - (h - (k0 + c)), tlen - h) : kNullDistance;
+          dmin = min(dmin, d[c]);
+        }
+        dmin = min(wave_min(dmin), max(plen, tlen));
+        D keep;
+#pragma unroll
+        for (int c = 0; c < N; ++c) keep.w[c] = __ballot(d[c] - dmin <= B->heur.thr);
+        keep = keep & D::range(lo, hi);
+        const int top = min(ke, hi);
+        const int clo = lo >= top ? lo : keep.any() ? min(keep.first(), top) : top;
+        const int bottom = max(ke, clo);
+        const int chi = hi <= bottom ? hi : keep.any() ? max(keep.last(), bottom) : bottom;
+        if (clo != lo || chi != hi) {
+          const D cut = D::range(clo, chi);  // (never empty)
+          rm[0] = cut;
+          ri = bi.hull() & cut;
+          rd = bd.hull() & cut;
+          const bool no_i = !ri.any(), no_d = !rd.any();
+          if ((bi.any() && no_i) || (bd.any() && no_d)) {
+            probe = true;
+#pragma unroll
+            for (int c = 0; c < N; ++c) {
+              pi[c] = w.i1[0][c];
+              pd[c] = w.d1[0][c];
+              w.i1[0][c] = no_i ? kNullTagged : w.i1[0][c];
+              w.d1[0][c] = no_d ? kNullTagged : w.d1[0][c];
+            }
+          }
+        }
+      }
+    }
+  }
+  if constexpr (REC) {
+    // the started word, its steps moved down to their places; the unused rest
+    // of the segment goes back
+    const int done = i - first, rest = done & (G - 1);
+    if (rest) *rec = cell.rec[0] >> (8 * N * (G - rest));
+    ch.cur -= (uint32_t)((last - first) / G - (done + G - 1) / G) * 16u;
+  }
+  steps = i;
+  return status;
+}
+
+// wf-adaptive (wavefront_heuristic.c:190-290): the cut-off keeps a wavefront
+// some tens of diagonals wide, so a lane holds one diagonal throughout; a pair
+// that leaves the wave's 64 diagonals starts again with two per lane (and,
+// leaving those too, goes to the lean kernel).  A step computes [lo, hi] from
+// the ranges the cut-off left of its sources; cells outside are NULL, cells
+// the cut-off dropped are still read (their wavefronts hold them).  Ranges are
+// lane masks: a source one diagonal off is a shift, the limits are the ends of
+// the union, and the computed range masks lanes as it is.  A gap range that
+// the cut-off empties is not read by the next step, but the reference's
+// backtrace probes its cells: that step's records are the choices with them.
+//
+// Records lie in up to three segments of steps (WaveArgs::last), reserved as
+// the pair reaches them: short pairs take only the first.
+//
+// Bound by the instructions of a step, about 85 on the vector and 100 on the
+// scalar side (100,000 reads of 100-300 bp, cut-off (10, 50, 1): 1.00 ms; the
+// lean kernel, with a ring in LDS and clamped reads, 1.48 ms; the same loop
+// with ranges as pairs of limits, 1.03 ms beside 0.34 ms and two more launches
+// for the 0.3% of the pairs that leave 64 diagonals).
+template <class S, bool REC>
+__global__ void __launch_bounds__(64, 7) wfa_wave_cut_kernel(ForwardArgs a) {
+  extern __shared__ __align__(16) unsigned char smem[];
+  uint32_t* seqP = reinterpret_cast<uint32_t*>(smem);
+  uint32_t* seqT = seqP + a.wave.lds_words;
+  const int lane = threadIdx.x;
+  WaveChunk ch{0, 0};
+  unsigned long long wg_dsteps = 0;
+  bool q_first = true;
+  for (;;) {
+    KernArgs A = args_now();
+    int qv = 0;
+    if (!q_first && lane == 0) qv = (int)atomicAdd(work_queue(A->queue, A->queues), 1u);
+    const int qi = work_item(A->queues, q_first, lane_of(qv, 0));
+    q_first = false;
+    if (qi >= A->n_pairs) break;
+    const int id = uniform(A->order ? A->order[qi] : qi);
+    WaveSeqs<2> q{seqP, seqT, 0u, 0u, uniform(A->plen[id]), uniform(A->tlen[id])};
+    wave_sync();  // the previous pair is done reading the sequences
+    stage_sequences(q, A, id, seqP, seqT);
+    wave_sync();
+    int status = kDevArenaFull, steps = 0, dsteps = 0, wide = 0;
+    uint32_t header = kNoBlock, base[kWaveCutSegments] = {0, 0, 0};
+    if (!REC || reserve_records(ch, 1)) {
+      if constexpr (REC) header = ch.cur++;
+      status = cut_pair<S, 1, REC>(q, ch, base, steps, dsteps);
+      if (status == kDevRingOverflow) {
+        wide = 1;
+        status = cut_pair<S, 2, REC>(q, ch, base, steps, dsteps);
+      }
+    }
+    KernArgs B = args_now();
+    const bool good = status == kDevCompleted;
+    if (lane == 0) {
+      B->out_status[id] = status;
+      B->out_score[id] = steps * B->pen.g;
+      B->out_last_block[id] = header;
+      B->out_dsteps[id] = good ? (long long)dsteps : 0;
+      if (REC && good) B->rec_arena[header] = make_uint4(base[0], base[1], base[2], (uint32_t)wide);
+      if (B->out_end_k) {
+        B->out_end_k[id] = q.tlen - q.plen;
+        B->out_end_off[id] = q.tlen;
+      }
+      if (!good) atomicAdd(B->retry_count, 1u);
+    }
+    wg_dsteps += good ? (unsigned long long)dsteps : 0ull;
+  }
+  if (lane == 0 && wg_dsteps) atomicAdd(args_now()->dsteps_total, wg_dsteps);
+}
+
 template <class S>
 bool wave_matches(const Penalties& p) {
   if (p.g <= 0 || p.ncomp != S::NC) return false;
@@ -520,6 +888,11 @@ const void* select_wave(int shape, int nmax, bool rec, int bits, bool ef) {
     case 5: return wave_fn_of<ShapeLinear>(nmax, rec, bits, ef);
   }
   return nullptr;
+}
+
+const void* select_wave_cut(bool rec) {
+  return rec ? reinterpret_cast<const void*>(&wfa_wave_cut_kernel<ShapeAffine, true>)
+             : reinterpret_cast<const void*>(&wfa_wave_cut_kernel<ShapeAffine, false>);
 }
 
 }  // namespace
@@ -559,8 +932,21 @@ bool wave_phases(int shape, int pbf, int tbf, int nmax, WaveArgs* w) {
 
 size_t wave_lds_bytes(int lds_words) { return (size_t)2 * lds_words * sizeof(uint32_t); }
 
-int wave_max_blocks_per_cu(int shape, int nmax, bool rec, int bits, bool ef, size_t lds) {
-  const void* f = select_wave(shape, nmax, rec, bits, ef);
+bool wave_cuts(int shape, const HeurArgs& h) {
+  return shape == 1 && h.wfadaptive == 1 && !h.xdrop && !h.zdrop && !h.banded;
+}
+
+void wave_cut_phases(WaveArgs* w) {
+  *w = WaveArgs{};
+  w->cut = 1;
+  w->last[0] = 48;
+  w->last[1] = 176;
+  w->last[2] = w->last[3] = kWaveSteps;
+  static_assert(kWaveCutSegments == 3 && kWaveSteps % 4 == 0, "segments");
+}
+
+int wave_max_blocks_per_cu(int shape, int nmax, bool rec, int bits, bool ef, bool cut, size_t lds) {
+  const void* f = cut ? select_wave_cut(rec) : select_wave(shape, nmax, rec, bits, ef);
   int n = 0;
   if (!f || hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, f, 64, lds) != hipSuccess) return 0;
   return n;
@@ -568,7 +954,8 @@ int wave_max_blocks_per_cu(int shape, int nmax, bool rec, int bits, bool ef, siz
 
 hipError_t launch_forward_wave(const ForwardArgs& a, int shape, int nmax, int bits, const LaunchShape& ls,
                                hipStream_t stream) {
-  const void* f = select_wave(shape, nmax, a.records != 0, bits, a.endsfree != 0);
+  const void* f = a.wave.cut ? select_wave_cut(a.records != 0)
+                             : select_wave(shape, nmax, a.records != 0, bits, a.endsfree != 0);
   if (!f || ls.block != 64) return hipErrorInvalidValue;
   void* args[] = {const_cast<ForwardArgs*>(&a)};
   return hipLaunchKernel(f, dim3(ls.grid), dim3(64), args, ls.lds_bytes, stream);
