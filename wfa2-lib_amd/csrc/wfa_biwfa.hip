@@ -545,7 +545,6 @@ __device__ int side_extend0(Side<NC, CUT>& sd, int plen, int tlen, int wcap, con
 template <int NC, int BLOCK, bool CUT>
 __device__ void side_resume(Side<NC, CUT>& sd, const int* rows, int par, int ib, int g, int plen, int tlen, int wcap,
                             int R, BlockRed<BLOCK>& red) {
-  constexpr int SH = 3;  // bits below the offset in the tiles' rows
   const int pitch = tile_pitch(plen, tlen), kpad = tile_kpad(plen), lane = threadIdx.x & 63;
   const int kmin = max(-plen, -ib), kmax = min(tlen, ib);  // a step reaches one diagonal further
   for (int age = kBiTileAges - 1; age >= 0; --age) {
@@ -557,7 +556,7 @@ __device__ void side_resume(Side<NC, CUT>& sd, const int* rows, int par, int ib,
       int first = INT_MAX, last = INT_MIN;
       for (int k = kmin + (int)threadIdx.x; k <= kmax; k += BLOCK) {
         const int v = row[k];
-        if (v >= 0 && in_bounds(v >> SH, k, plen, tlen)) {
+        if (v >= 0 && in_bounds(v, k, plen, tlen)) {
           first = min(first, k);
           last = max(last, k);
         }
@@ -574,7 +573,7 @@ __device__ void side_resume(Side<NC, CUT>& sd, const int* rows, int par, int ib,
       int* out = sd.ring + (slot * NC + c) * wcap - alo;
       for (int k = lo[c] + (int)threadIdx.x; k <= hi[c]; k += BLOCK) {
         const int v = row[k];
-        out[k] = v < 0 ? kOffsetNull : v >> SH;
+        out[k] = v < 0 ? kOffsetNull : v;
       }
     }
     if (lane == slot) {

@@ -9,7 +9,8 @@
 // outside a wavefront's range hold NULL by themselves, because everything
 // they are computed from does.
 //
-// Values are kept as (offset << SH) | source << 1 | flag.  One maximum over
+// Values are kept as (offset << SH) | source << 1 | flag (ScoreOnly shapes:
+// as offsets).  One maximum over
 // the candidates then takes the largest offset with the reference's
 // tie-breaks (M > D2 > D1 > I2 > I1, extension before opening,
 // wavefront_backtrace.c:64-219): the source codes rise in that order below
@@ -96,6 +97,7 @@ template <int N>
 struct StepCells {
   int h[N];        // extended M offset (meaningless where !ok)
   bool ok[N];      // valid M cell
+  int rem[N];      // symbols left to the nearer border after the extension
   bool oob[N];     // a path reaches the cell, but outside the matrix
   // Record bytes, shifted in from the top: after four cells (of one step, or
   // with N < 4 of consecutive steps) a word holds them in order.
@@ -129,7 +131,6 @@ __device__ __forceinline__ void wave_cells(const int* mx, const int* mo, int* i1
     b2u = from_upper_lane(b2[0]);
   }
   uint32_t full = 0;  // cells whose run fills the window
-  int rem[N];
 #pragma unroll
   for (int c = 0; c < N; ++c) {
     const int ins1 = (c ? a1[c > 0 ? c - 1 : 0] : a1l) + ONE;
@@ -143,12 +144,12 @@ __device__ __forceinline__ void wave_cells(const int* mx, const int* mo, int* i1
       best = max(max(best, ins2), del2);
     }
     if constexpr (S::NC > 1) {
-      i1[c] = (ins1 & ~(ONE - 1)) | 1;
-      d1[c] = (del1 & ~(ONE - 1)) | 1;
+      i1[c] = S::kTags ? (ins1 & ~(ONE - 1)) | 1 : ins1;
+      d1[c] = S::kTags ? (del1 & ~(ONE - 1)) | 1 : del1;
     }
     if constexpr (S::NC == 5) {
-      i2[c] = (ins2 & ~(ONE - 1)) | 1;
-      d2[c] = (del2 & ~(ONE - 1)) | 1;
+      i2[c] = S::kTags ? (ins2 & ~(ONE - 1)) | 1 : ins2;
+      d2[c] = S::kTags ? (del2 & ~(ONE - 1)) | 1 : del2;
     }
     // record byte: NC == 5: source and flag of the best (4 bits), then the
     // flags of I1, D1, I2, D2; NC == 3: 6 bits of the best (source in bits
@@ -176,7 +177,7 @@ __device__ __forceinline__ void wave_cells(const int* mx, const int* mo, int* i1
     out.ok[c] = ok;
     out.oob[c] = !ok & (best >= 0);
     out.h[c] = o + n;
-    rem[c] = r - n;
+    out.rem[c] = r - n;
     full |= (ok & (n == SPAN) & (r > SPAN)) ? 1u << c : 0u;
   }
   // long runs (rare away from the main diagonal): more windows, cell by cell
@@ -185,7 +186,7 @@ __device__ __forceinline__ void wave_cells(const int* mx, const int* mo, int* i1
     for (int c = 0; c < N; ++c) {
       bool more = (full >> c) & 1u;
       if (__ballot(more)) {
-        int h = out.h[c], r = rem[c];
+        int h = out.h[c], r = out.rem[c];
         while (more) {
           const int n = q.run(h, h - (k0 + c), r);
           h += n;
@@ -193,6 +194,7 @@ __device__ __forceinline__ void wave_cells(const int* mx, const int* mo, int* i1
           more = (n == SPAN) & (r > 0);
         }
         out.h[c] = h;
+        out.rem[c] = r;
       }
     }
   }

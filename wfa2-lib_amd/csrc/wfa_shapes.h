@@ -8,12 +8,21 @@ namespace wfa {
 // Distances between wavefronts in steps (score / g), known at compile time.
 template <int NC_, int DX_, int DO1_, int DE1_, int DO2_, int DE2_>
 struct SlotShape {
+  using Slots = SlotShape;
   static constexpr int NC = NC_, DX = DX_, DO1 = DO1_, DE1 = DE1_, DO2 = DO2_, DE2 = DE2_;
   static constexpr int RM = DX > DO1 ? DX : DO1;  // M rows kept in registers (the second gap's come from memory)
   static constexpr int SH = NC == 5 ? 4 : 3;      // bits below the offset
   static constexpr bool kMismatch = DX > 0;       // (indel distance has no mismatches)
+  static constexpr bool kTags = true;             // ... which hold a cell's source
   static constexpr int kTagX = NC == 5 ? 4 : 2, kTagD2 = 3, kTagD1 = NC == 5 ? 2 : 1, kTagI2 = 1;
   static constexpr int kGapRows = 2 * DE1 + (NC == 5 ? 2 * DE2 : 0);
+};
+// The shape without records: values are plain offsets, which saves the tags'
+// masking (150,000 reads of 100-300 bp, score only: 0.574 -> 0.533 ms).
+template <class S>
+struct ScoreOnly : S {
+  static constexpr bool kTags = false;
+  static constexpr int SH = 0, kTagX = 0, kTagD2 = 0, kTagD1 = 0, kTagI2 = 0;
 };
 using Shape2p = SlotShape<5, 4, 8, 2, 25, 1>;  // gap-affine-2p (x 4, o1 6, e1 2, o2 24, e2 1) and its multiples
 using ShapeAffine = SlotShape<3, 2, 4, 1, 0, 1>;  // gap-affine (x 4, o 6, e 2) and its multiples

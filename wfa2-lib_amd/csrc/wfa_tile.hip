@@ -865,8 +865,10 @@ __device__ __forceinline__ BiSide bi_side(const BiTileArgs& a, int prob, int sid
   return s;
 }
 
+// Steps per block, and the halo: 64 pairs of 20-60 kbp take 63.4 ms with 16,
+// 60.3 with 24, 60.2 with 32 (and more for the breakpoint kernel to do again).
 struct BiGeom {
-  static constexpr int N = 4, T = 16, H = 16, U = 64 * N - 2 * H;
+  static constexpr int N = 4, T = 24, H = 24, U = 64 * N - 2 * H;
 };
 
 // One block of T steps of both sides of every active sub-problem, score only:
@@ -876,14 +878,15 @@ struct BiGeom {
 // takes over from the rows at the block's start, which sit in the other half.
 //
 // Bound by the vector units and, while few tiles are alive, by the latency of
-// a step (131 vector instructions for a lane's four cells, 33 a cell): a
-// launch costs 5.5 us for its loads and 0.85 us (one wave per SIMD) to 1.5 us
+// a step: a launch costs 5.5 us for its loads and 0.85 us (one wave per SIMD) to 1.5 us
 // (four) per step.  One workgroup or team per search instead pays a barrier
 // and a trip to its ring in HBM per step, and the longest search decides: 64
-// pairs of 20-60 kbp took 482 ms that way, 67 ms in tiles (45 ms here, 14 ms
-// in the breakpoint kernel's last block and overlap scans).
+// pairs of 20-60 kbp took 482 ms that way, 60 ms in tiles (40 ms here, 14 ms
+// in the breakpoint kernel's last block and overlap scans).  Plain offsets
+// instead of tagged ones, and the furthest antidiagonal taken only where it
+// can be: 66.6 -> 63.8 ms, 24 steps a launch instead of 16: 60.3 ms.
 __global__ void __launch_bounds__(64 * kTileWaves) bi_tile_kernel(BiTileArgs a) {
-  using S = ShapeAffine;
+  using S = ScoreOnly<ShapeAffine>;
   constexpr int N = BiGeom::N, T = BiGeom::T, H = BiGeom::H, U = BiGeom::U;
   extern __shared__ __align__(16) unsigned char smem[];
   __shared__ int far_lds[kTileWaves];
@@ -942,8 +945,16 @@ __global__ void __launch_bounds__(64 * kTileWaves) bi_tile_kernel(BiTileArgs a) 
       StepCells<N> cell;
       for (uint32_t& r : cell.rec) r = 0;
       wave_step<S, N, PH, 2>(w, nullptr, k0, q, cell);
+      // The furthest antidiagonal: along a diagonal M gains at least one cell
+      // every DX steps, so the block's last DX steps have it, or a step with a
+      // cell on a border (what a border cuts off lies behind such a cell).
+      int rem = cell.rem[0];
 #pragma unroll
-      for (int c = 0; c < N; ++c) far = (cell.ok[c] & own) ? max(far, 2 * cell.h[c] - (k0 + c)) : far;
+      for (int c = 1; c < N; ++c) rem = min(rem, cell.rem[c]);
+      if (t >= T - S::DX || __ballot(rem <= 0)) {
+#pragma unroll
+        for (int c = 0; c < N; ++c) far = (cell.ok[c] & own) ? max(far, 2 * cell.h[c] - (k0 + c)) : far;
+      }
       if (ends) {
         bool out = false;
 #pragma unroll
@@ -987,7 +998,6 @@ __global__ void __launch_bounds__(64 * kTileWaves) bi_tile_kernel(BiTileArgs a) 
 
 // Score 0 of both sides, and the first active list.
 __global__ void __launch_bounds__(64) bi_tile_init_kernel(BiTileArgs a, int* act, int* n_act) {
-  using S = ShapeAffine;
   const int x = blockIdx.x * 64 + threadIdx.x;
   if (x == 0) *n_act = a.n;
   if (x >= 2 * a.n) return;
@@ -1003,7 +1013,7 @@ __global__ void __launch_bounds__(64) bi_tile_init_kernel(BiTileArgs a, int* act
     h = lcp_extend<2>(sd.words + (sd.ppos >> 5), (int)(sd.ppos & 31), sd.words + (sd.tpos >> 5), (int)(sd.tpos & 31),
                       sd.plen, sd.tlen, 0, 0);
   a.state[a.st_off[prob] + ((long long)side * kBiTileRows + bi_row(1, sd.begin, 0)) * pitch + tile_kpad(sd.plen)] =
-      (h << S::SH) | (sd.begin == kM ? 0 : 1);
+      h;
   // (an end reached at score 0: found again by the breakpoint kernel)
   const bool end0 = sd.begin == kM && sd.end == kM && sd.plen == sd.tlen && h >= sd.tlen;
   a.far[2 * prob + side] = a.far[2 * a.n + 2 * prob + side] = end0 ? sd.plen + sd.tlen : 2 * h;

@@ -198,8 +198,8 @@ __device__ __forceinline__ void wave_phase(WavePair& p, WaveChunk& ch, WaveRows<
       KernArgs B = args_now();
       if (!p.exact) {
         p.exact = true;
-        p.hist_m = wave_table<S>.hist_m[i - 1];
-        p.hist_gap = wave_table<S>.hist_gap[i - 1];
+        p.hist_m = wave_table<typename S::Slots>.hist_m[i - 1];
+        p.hist_gap = wave_table<typename S::Slots>.hist_gap[i - 1];
       }
       uint32_t okm = 0, reach = 0;
 #pragma unroll
@@ -226,7 +226,7 @@ __device__ __forceinline__ void wave_phase(WavePair& p, WaveChunk& ch, WaveRows<
           if (null_gap(kD2, S::DE2)) { lo = min(lo, 0); hi = max(hi, -2); }
         }
       }
-      const int tlo = wave_table<S>.lo[i - 1], thi = wave_table<S>.hi[i - 1];
+      const int tlo = wave_table<typename S::Slots>.lo[i - 1], thi = wave_table<typename S::Slots>.hi[i - 1];
       p.dev += (some ? hi - lo + 1 : 0) - (tlo <= thi ? thi - tlo + 1 + (EF ? B->pbf + B->tbf : 0) : 0);
       p.hist_m = (p.hist_m << 1) | (__ballot(okm != 0) ? 1u : 0u);
       p.hist_gap <<= 4;
@@ -476,7 +476,7 @@ __global__ void __launch_bounds__(64, S::NC == 5 ? (NMAX == 8 ? 2 : 3) : (NMAX =
     if (p.status == 1) p.status = kDevRingOverflow;  // wider than the wave holds
     KernArgs B = args_now();
     const bool good = p.status == kDevCompleted;
-    const int ds = good ? wave_table<S>.dsteps[p.i] + p.dev + (EF ? wave_table<S>.nonnull[p.i] * (B->pbf + B->tbf) : 0) : 0;
+    const int ds = good ? wave_table<typename S::Slots>.dsteps[p.i] + p.dev + (EF ? wave_table<typename S::Slots>.nonnull[p.i] * (B->pbf + B->tbf) : 0) : 0;
     if (lane == 0) {
       B->out_status[id] = p.status;
       B->out_score[id] = p.i * B->pen.g;
@@ -870,9 +870,9 @@ template <class S, int SRC, bool EF>
 const void* wave_fn(int nmax, bool rec) {
   if (nmax <= 4)
     return rec ? reinterpret_cast<const void*>(&wfa_wave_kernel<S, 4, SRC, true, EF>)
-               : reinterpret_cast<const void*>(&wfa_wave_kernel<S, 4, SRC, false, EF>);
+               : reinterpret_cast<const void*>(&wfa_wave_kernel<ScoreOnly<S>, 4, SRC, false, EF>);
   return rec ? reinterpret_cast<const void*>(&wfa_wave_kernel<S, 8, SRC, true, EF>)
-             : reinterpret_cast<const void*>(&wfa_wave_kernel<S, 8, SRC, false, EF>);
+             : reinterpret_cast<const void*>(&wfa_wave_kernel<ScoreOnly<S>, 8, SRC, false, EF>);
 }
 template <class S>
 const void* wave_fn_of(int nmax, bool rec, int bits, bool ef) {
@@ -892,7 +892,7 @@ const void* select_wave(int shape, int nmax, bool rec, int bits, bool ef) {
 
 const void* select_wave_cut(bool rec) {
   return rec ? reinterpret_cast<const void*>(&wfa_wave_cut_kernel<ShapeAffine, true>)
-             : reinterpret_cast<const void*>(&wfa_wave_cut_kernel<ShapeAffine, false>);
+             : reinterpret_cast<const void*>(&wfa_wave_cut_kernel<ScoreOnly<ShapeAffine>, false>);
 }
 
 }  // namespace
