@@ -104,6 +104,7 @@ PlanGroup& PlanGroup::operator=(PlanGroup&& o) noexcept {
   wave = o.wave;
   wave_rec = o.wave_rec;
   wave_ef = o.wave_ef;
+  wave_wide = o.wave_wide;
   ids = std::move(o.ids);
   d_ids = std::move(o.d_ids);
   ids_on_device = o.ids_on_device;
@@ -864,8 +865,10 @@ void set_wave(const JobSet& js, PlanGroup& g, const Penalties& pen, int records)
 
 // Forward (and, with records, backtrace) launches of one group, with the
 // group's events around them when it has events.
+// `wide`: a second forward launch for the pairs that outgrow the first.
 hipError_t launch_group(const PlanGroup& grp, const LaunchShape& shape, const ForwardArgs& args,
-                        const BacktraceArgs& ba, int ncomp, int bits, int records, hipStream_t st) {
+                        const BacktraceArgs& ba, int ncomp, int bits, int records, hipStream_t st,
+                        const ForwardArgs* wide = nullptr, const LaunchShape* wide_shape = nullptr) {
   if (grp.ev[0]) (void)hipEventRecord(grp.ev[0], st);
   ForwardArgs fa = args;
   fa.queues = shape.grid >= 64 * wfa::kMaxQueues ? wfa::kMaxQueues : 1;
@@ -873,6 +876,8 @@ hipError_t launch_group(const PlanGroup& grp, const LaunchShape& shape, const Fo
                        ? wfa::launch_forward_wave(fa, wfa::wave_shape(fa.pen), grp.wcap, bits, shape, st)
                    : grp.family == wfa::kLean ? wfa::launch_forward_lean(fa, shape, st)
                                               : wfa::launch_forward(fa, ncomp, bits, shape, st);
+  if (err == hipSuccess && wide)
+    err = wfa::launch_forward_wave(*wide, wfa::wave_shape(fa.pen), 8, bits, *wide_shape, st);
   if (err != hipSuccess) return err;
   if (grp.ev[1]) (void)hipEventRecord(grp.ev[1], st);
   if (records) {
@@ -881,6 +886,17 @@ hipError_t launch_group(const PlanGroup& grp, const LaunchShape& shape, const Fo
   }
   if (grp.ev[2]) (void)hipEventRecord(grp.ev[2], st);
   return hipSuccess;
+}
+
+// Below this many pairs the second launch is not worth its few microseconds.
+constexpr int kWideFollowMin = 2048;
+// Arena for the second launch's chunks: some 150 KB for each of up to 1,000
+// workgroups at a time.
+constexpr double kWideRecordBytes = 160e6;
+
+bool wide_follows(const Engine* e, const JobSet& js, const PlanGroup& g, const Penalties& pen) {
+  return g.family == wfa::kWave && g.wcap == 4 && !e->na && (int)g.ids.size() >= kWideFollowMin && !js.heur.cut() &&
+         (pen.ncomp == 5 || js.ef.on);
 }
 
 // Enqueues forward + backtrace of one group on the aligner's stream; with
@@ -910,7 +926,40 @@ int enqueue_group(wavefront_aligner_t* wf, Engine* e, const JobSet& js, PlanGrou
   BacktraceArgs ba;
   group_args(wf, e, js, grp, pen, records, ident, &fa, &ba);
   if (!fresh && !hip_ok(wfa::launch_reset_counters(counters_of(e), 0, st), "reset")) return WF_STATUS_OOM;
-  if (!hip_ok(launch_group(grp, shape, fa, ba, pen.ncomp, js.bits, records, st), "forward/backtrace launch"))
+  // Pairs that outgrow 4 diagonals per lane go on with 8 in a launch of its own
+  // right behind, before the one backtrace of all: some always do with a
+  // second gap or free ends, and a round of their own (status, order, launch,
+  // backtrace, all waiting for a few pairs) took longer: 50,000 reads of
+  // 100-300 bp under gap-affine-2p 1.59 -> 1.37 ms, 100,000 with free ends
+  // (and one length class instead of two) 1.42 -> 1.26 ms.
+  ForwardArgs wide;
+  LaunchShape wide_shape;
+  grp.wave_wide = wide_follows(e, js, grp, pen) && e->over.ensure((size_t)n * 4);
+  if (grp.wave_wide) {
+    PlanGroup g8;
+    g8.family = wfa::kWave;
+    g8.block = 64;
+    g8.wcap = 8;
+    g8.lmax_words = grp.lmax_words;
+    g8.max_grid = grp.max_grid;
+    set_wave(js, g8, pen, records);
+    g8.ids.swap(grp.ids);
+    wide_shape = shape_of(e, g8, js.bits, pen, 0);
+    g8.ids.swap(grp.ids);
+    fa.over_ids = e->over.as<int>();
+    fa.over_n = &counters_of(e)->over;
+    wide = fa;
+    wide.over_ids = nullptr;
+    wide.order = e->over.as<int>();
+    wide.n_over = fa.over_n;
+    wide.queue = &counters_of(e)->over_queue;
+    wide.queues = 1;
+    wide.wave = g8.wave;
+    wide.wave.lds_words = grp.lmax_words;
+    for (int ph = 0; ph < wfa::kWavePhases; ++ph) ba.wave_last[ph] = g8.wave.last[ph];  // (the same but the last)
+  }
+  if (!hip_ok(launch_group(grp, shape, fa, ba, pen.ncomp, js.bits, records, st, grp.wave_wide ? &wide : nullptr,
+                           &wide_shape), "forward/backtrace launch"))
     return WF_STATUS_OOM;
   return WF_STATUS_OK;
 }
@@ -974,11 +1023,13 @@ std::vector<PlanGroup> make_plan(const JobSet& js, const std::vector<int>& ids, 
                        (js.bits == 2 || js.nibbles) && wfa::wave_shape(pen) != 0 &&
                        wfa::wave_phases(wfa::wave_shape(pen), js.ef.on ? js.ef.pbf : 0, js.ef.on ? js.ef.tbf : 0, 4, &wa);
   int wave_words[2] = {0, 0};
+  const int wave_free = js.ef.on ? std::max(js.ef.pbf + js.ef.pef, js.ef.tbf + js.ef.tef) : 0;
   for (int i : ids) {
     const int L = std::max(js.h_plen[i], js.h_tlen[i]);
     // (with a second gap, pairs of the longer class outgrow a wave: tiles)
     if (wave_ok && L <= (ncomp == 5 && tile_ok ? lt.short_len : kLeanMaxLen)) {
-      const int c = L <= lt.short_len ? 0 : 1;
+      // (free ends add symbols, not errors)
+      const int c = L - wave_free <= lt.short_len ? 0 : 1;
       wave_ids[c].push_back(i);
       wave_words[c] = std::max(wave_words[c], js.bits == 2 ? 2 * (L / 32 + 3) : L / 8 + 3);
       continue;
@@ -1070,6 +1121,7 @@ int run_jobs(wavefront_aligner_t* wf, Engine* e, const JobSet& js, std::vector<P
         set_wave(js, g, pen, records);
         if (g.family != wfa::kTile)  // and the record chunk of every workgroup
           g.est_rec_bytes += (double)shape_of(e, g, js.bits, pen, js.heur.cut()).grid * wfa::kChunkUnits * 16;
+        if (wide_follows(e, js, g, pen)) g.est_rec_bytes += kWideRecordBytes;
       }
       want += g.est_rec_bytes;
     }
@@ -1123,7 +1175,7 @@ int run_jobs(wavefront_aligner_t* wf, Engine* e, const JobSet& js, std::vector<P
       }
       if (!ring_over.empty()) {
         const bool cut = js.heur.cut() != 0;
-        if (g.family == wfa::kWave && g.wcap < 8 && !cut) {
+        if (g.family == wfa::kWave && g.wcap < 8 && !g.wave_wide && !cut) {
           PlanGroup h = take_group(e);
           h.family = wfa::kWave;
           h.block = 64;

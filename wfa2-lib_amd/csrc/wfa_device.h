@@ -116,6 +116,9 @@ __host__ __device__ inline int wave_cut_center(int kend) { return kend / 2; }
 struct ForwardArgs {
   int n_pairs;
   const int* order;            // processing order (pair ids), longest first
+  const unsigned int* n_over;  // wave family: where set, the number of pairs in `order`
+  int* over_ids;               // wave family: where set, pairs that outgrow the wave are noted here,
+  unsigned int* over_n;        // ... counted here, and not in retry_count
   const int* plen;
   const int* tlen;
   const uint64_t* words;       // packed sequences
@@ -215,12 +218,12 @@ hipError_t launch_backtrace(const BacktraceArgs& a, hipStream_t stream);
 // Device counters of one run: the totals (64 bytes, copied to the host) and
 // the work queues of the current launch.
 struct Counters {
-  unsigned int pad1;
+  unsigned int over;             // pairs that outgrew the first kernel of their group (ForwardArgs::over_ids)
   unsigned int retry;            // pairs to re-run (ring overflow / arena full)
   unsigned long long rec_top;    // record arena bump pointer (16-byte units)
   unsigned long long dsteps;     // diagonal-steps of the pairs that finished
   unsigned int fail;             // pairs that finished with a status other than completed
-  unsigned int pad0;
+  unsigned int over_queue;       // work queue of the kernel that takes them
   unsigned long long pad[12];
   unsigned int queue[kMaxQueues * kQueueStride];
 };

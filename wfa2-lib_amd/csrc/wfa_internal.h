@@ -102,6 +102,7 @@ struct PlanGroup {
   int lclass = -1;             // lean family: length class (0 short, 1 long)
   wfa::WaveArgs wave{};        // wave family (wcap: most diagonals per lane): phases, set before a launch
   bool wave_rec = false, wave_ef = false;  // ... and its kernel instance
+  bool wave_wide = false;      // ... and whether the pairs that outgrew it ran on 8 diagonals per lane already
   hipEvent_t ev[3] = {nullptr, nullptr, nullptr};
   PlanGroup() = default;
   PlanGroup(const PlanGroup&) = delete;
@@ -121,6 +122,7 @@ struct Engine {
   DevBuf rec;
   DevBuf ring;
   DevBuf counters;
+  DevBuf over;  // ids of a group's pairs that outgrow its first kernel
   size_t rec_bytes = 0;     // record arena size for the next run (grows on demand)
   size_t rec_cap = 0;       // largest record arena this engine may allocate
   bool ok = false;

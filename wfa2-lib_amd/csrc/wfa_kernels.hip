@@ -1007,6 +1007,8 @@ __global__ void wfa_reset_kernel(Counters* c, int all) {
   if (threadIdx.x < kMaxQueues) c->queue[threadIdx.x * kQueueStride] = 0u;
   if (threadIdx.x == 0) {
     c->rec_top = 0ull;
+    c->over = 0u;
+    c->over_queue = 0u;
     if (all >= 1) c->retry = 0u;
     if (all >= 2) { c->dsteps = 0ull; c->fail = 0u; }
   }

@@ -402,7 +402,7 @@ __global__ void __launch_bounds__(64, S::NC == 5 ? (NMAX == 8 ? 2 : 3) : (NMAX =
     if (!q_first && lane == 0) qv = (int)atomicAdd(work_queue(A->queue, A->queues), 1u);
     const int qi = work_item(A->queues, q_first, lane_of(qv, 0));
     q_first = false;
-    if (qi >= A->n_pairs) break;
+    if (qi >= (A->n_over ? uniform((int)*A->n_over) : A->n_pairs)) break;
     const int id = A->order ? A->order[qi] : qi;
     WavePair p;
     p.plen = A->plen[id];
@@ -487,7 +487,10 @@ __global__ void __launch_bounds__(64, S::NC == 5 ? (NMAX == 8 ? 2 : 3) : (NMAX =
         B->out_end_k[id] = p.end_k;
         B->out_end_off[id] = p.end_off;
       }
-      if (!good) atomicAdd(B->retry_count, 1u);
+      if (!good) {
+        if (p.status == kDevRingOverflow && B->over_ids) B->over_ids[atomicAdd(B->over_n, 1u)] = id;
+        else atomicAdd(B->retry_count, 1u);
+      }
     }
     wg_dsteps += (unsigned long long)ds;
   }
