@@ -829,6 +829,7 @@ void group_args(wavefront_aligner_t* wf, Engine* e, const JobSet& js, const Plan
   ba.ops = js.ops;
   ba.ops_off = js.ops_off;
   ba.ops_begin = js.ops_begin;
+  ba.run_counts = js.run_counts;
   ba.fail_count = &c->fail;
   ba.comp_end_p = js.cend;
   ba.comp_begin_p = js.cbeg;
@@ -1145,6 +1146,7 @@ int run_jobs(wavefront_aligner_t* wf, Engine* e, const JobSet& js, std::vector<P
                                             : enqueue_group(wf, e, js, g, pen, records, fresh);
       if (rc != WF_STATUS_OK) return rc;
       if (!g.ids.empty()) fresh = false;
+      tot->uncounted = tot->uncounted || g.family == wfa::kTile;
       ++tot->launches;
     }
     if (!hip_ok(hipMemcpyAsync(&host_c, e->counters.p, wfa::kCounterTotals, hipMemcpyDeviceToHost, st), "counters") ||
@@ -1326,6 +1328,7 @@ wfa_host::JobSet wfa_device_batch_t::jobs() const {
   js.ops = d_ops.as<char>();
   js.ops_off = d_ops_off.as<int64_t>();
   js.ops_begin = d_ops_begin.as<int>();
+  js.run_counts = counting ? d_run_counts.as<long long>() : nullptr;
   js.end_k = d_end_k.as<int>();
   js.end_off = d_end_off.as<int>();
   js.end_rec = d_end_rec.as<int>();
@@ -1847,6 +1850,8 @@ int batch_run(wavefront_aligner_t* wf, wfa_device_batch_t* b, Engine* e) {
   RunTotals tot;
   int rc;
   b->bi_mode = wf->memory_mode == wavefront_memory_ultralow;
+  b->counted = false;
+  b->counting = records && !b->bi_mode && !e->na && b->d_run_counts.ensure(((size_t)b->n + 1) * 8);
   if (b->bi_mode) {
     rc = bialign_run(wf, e, b, &tot);
     if (rc == WF_STATUS_OOM) return rc;
@@ -1886,6 +1891,7 @@ int batch_run(wavefront_aligner_t* wf, wfa_device_batch_t* b, Engine* e) {
   b->stats.record_arena_bytes = (int64_t)e->rec.cap;
   b->have_results = true;
   b->host_results = false;
+  b->counted = b->counting && !tot.uncounted;
   if (tot.fail == 0) return WF_STATUS_ALG_COMPLETED;
   if (e->na) {
     // statuses through pageable host memory (no pinned staging), settled,
@@ -2155,6 +2161,7 @@ int plain_run(wavefront_aligner_t* wf, Engine* e, wfa_device_batch_t* b, const w
   b->heur = heuristic_of(wf);
   b->stats = wfa_run_stats_t{};
   b->bi_mode = false;
+  b->counting = b->counted = false;
   b->unlimited = b->tiles = unlimited_steps(wf);
   b->first_fail = WF_STATUS_ALG_COMPLETED;
   hipStream_t st = e->stream;
@@ -2293,18 +2300,20 @@ int make_runs(wavefront_aligner_t* wf, Engine* e, wfa_device_batch_t* b) {
   a.plen = b->d_plen.as<int>();
   a.tlen = b->d_tlen.as<int>();
   a.status = b->d_status.as<int>();
-  if (!b->d_run_counts.ensure((size_t)n * 8) || !b->d_run_off.ensure(((size_t)n + 1) * 8)) return WF_STATUS_OOM;
+  if (!b->d_run_counts.ensure(((size_t)n + 1) * 8) || !b->d_run_off.ensure(((size_t)n + 1) * 8)) return WF_STATUS_OOM;
   a.counts = b->d_run_counts.as<long long>();
   a.offsets = b->d_run_off.as<long long>();
   size_t temp = 0;
-  if (!hip_ok(wfa::launch_cigar_runs_count(a, nullptr, &temp, st), "scan size") ||
+  if (!hip_ok(wfa::launch_cigar_runs_count(a, false, nullptr, &temp, st), "scan size") ||
       !b->d_scan_temp.ensure(std::max<size_t>(temp, 256)))
     return WF_STATUS_OOM;
   temp = b->d_scan_temp.cap;
   // The results come down with the run offsets, and are unpacked while the
   // runs are written and copied: 150,000 reads of 100-300 bp 1.82 -> 1.44 ms.
   const bool res = !b->host_results;
-  if (!hip_ok(wfa::launch_cigar_runs_count(a, b->d_scan_temp.p, &temp, st), "run count") ||
+  // (counted by the backtrace, except for tiles and BiWFA: without the pass
+  // over the operations 150,000 reads of 100-300 bp take 1.35 ms, not 1.42)
+  if (!hip_ok(wfa::launch_cigar_runs_count(a, !b->counted, b->d_scan_temp.p, &temp, st), "run count") ||
       !hip_ok(hipMemcpyAsync(b->h_run_off.p, b->d_run_off.p, ((size_t)n + 1) * 8, hipMemcpyDeviceToHost, st),
               "run offsets") ||
       (res && !queue_results(e, b)) || !hip_ok(hipStreamSynchronize(st), "run offsets"))

@@ -5,10 +5,10 @@
 // matches, 8 (X), 1 (I), 2 (D).  A 100-300 bp read at a few percent error
 // has a few dozen runs, so the runs are 4-10 times smaller than the bytes.
 //
-// Two passes, one wave per pair: count the runs (a run starts at the first
-// byte and wherever a byte differs from the one before it: one ballot per 64
-// bytes), an inclusive scan of the counts (hipcub), then write each run at
-// its pair's offset.
+// The lane-per-pair backtrace counts the runs itself; otherwise two passes,
+// one wave per pair: count the runs (a run starts at the first byte and
+// wherever a byte differs from the one before it: one ballot per 64 bytes), a
+// scan of the counts (hipcub), then write each run at its pair's offset.
 #include <hipcub/hipcub.hpp>
 
 #include "wfa_device.h"
@@ -32,7 +32,6 @@ __device__ __forceinline__ void cigar_span(const CigarRunsArgs& a, int p, long l
 __global__ void __launch_bounds__(64 * kRunsWaves) cigar_count_kernel(CigarRunsArgs a) {
   const int lane = threadIdx.x & 63;
   const int p = blockIdx.x * kRunsWaves + (threadIdx.x >> 6);
-  if (p == 0 && lane == 0) a.offsets[0] = 0;
   if (p >= a.n) return;
   long long begin, end;
   cigar_span(a, p, &begin, &end);
@@ -83,17 +82,19 @@ __global__ void __launch_bounds__(64 * kRunsWaves) cigar_write_kernel(CigarRunsA
 
 }  // namespace
 
-hipError_t launch_cigar_runs_count(const CigarRunsArgs& a, void* temp, size_t* temp_bytes, hipStream_t stream) {
+hipError_t launch_cigar_runs_count(const CigarRunsArgs& a, bool count, void* temp, size_t* temp_bytes, hipStream_t stream) {
   if (temp == nullptr) {
     // scan storage query only
-    return hipcub::DeviceScan::InclusiveSum(nullptr, *temp_bytes, a.counts, a.offsets + 1, a.n, stream);
+    return hipcub::DeviceScan::ExclusiveSum(nullptr, *temp_bytes, a.counts, a.offsets, a.n + 1, stream);
   }
   if (a.n <= 0) return hipSuccess;
-  const int grid = (a.n + kRunsWaves - 1) / kRunsWaves;
-  hipLaunchKernelGGL(cigar_count_kernel, dim3(grid), dim3(64 * kRunsWaves), 0, stream, a);
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return e;
-  return hipcub::DeviceScan::InclusiveSum(temp, *temp_bytes, a.counts, a.offsets + 1, a.n, stream);
+  if (count) {
+    const int grid = (a.n + kRunsWaves - 1) / kRunsWaves;
+    hipLaunchKernelGGL(cigar_count_kernel, dim3(grid), dim3(64 * kRunsWaves), 0, stream, a);
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+  }
+  return hipcub::DeviceScan::ExclusiveSum(temp, *temp_bytes, a.counts, a.offsets, a.n + 1, stream);
 }
 
 hipError_t launch_cigar_runs_write(const CigarRunsArgs& a, hipStream_t stream) {

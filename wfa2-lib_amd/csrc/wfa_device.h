@@ -176,6 +176,7 @@ struct BacktraceArgs {
   char* ops;                   // operations arena
   const int64_t* ops_off;      // slot of pair i: ops[ops_off[i] .. +plen+tlen)
   int* ops_begin;              // CIGAR = ops[ops_off + ops_begin .. ops_off + plen + tlen)
+  long long* run_counts;       // where set: runs of equal operations of the CIGAR, 0 for a failed pair
   unsigned int* fail_count;    // incremented for a pair whose trace is inconsistent
   const signed char* comp_end_p;  // per-pair end component (null: comp_end)
   const signed char* comp_begin_p; // per-pair begin component (null: comp_begin)
@@ -330,12 +331,12 @@ struct CigarRunsArgs {
   const int* plen;
   const int* tlen;
   const int* status;           // null: every pair has its CIGAR
-  long long* counts;           // runs per pair
+  long long* counts;           // runs per pair (room for n + 1)
   long long* offsets;          // n + 1 entries: offsets[i] = runs before pair i
   uint32_t* runs;
 };
-// Counting pass and scan (temp == null: only sets *temp_bytes, the scan's storage).
-hipError_t launch_cigar_runs_count(const CigarRunsArgs& a, void* temp, size_t* temp_bytes, hipStream_t stream);
+// Counting pass (unless the counts are there) and scan (temp == null: only sets *temp_bytes, the scan's storage).
+hipError_t launch_cigar_runs_count(const CigarRunsArgs& a, bool count, void* temp, size_t* temp_bytes, hipStream_t stream);
 hipError_t launch_cigar_runs_write(const CigarRunsArgs& a, hipStream_t stream);
 
 // Lean family: whether the penalties' slot structure has an instance, its

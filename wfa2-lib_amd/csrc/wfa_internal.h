@@ -237,6 +237,7 @@ struct JobSet {
   char* ops = nullptr;
   const int64_t* ops_off = nullptr;
   int* ops_begin = nullptr;
+  long long* run_counts = nullptr;  // where set, the backtrace counts the runs of each CIGAR
   int* end_k = nullptr;        // end cell (diagonal, offset) of each completed job
   int* end_off = nullptr;
   int* end_rec = nullptr;      // z-drop: record byte of the end cell (0xFF: no source)
@@ -253,6 +254,7 @@ wfa::HeurArgs heuristic_of(const wavefront_aligner_t* wf);
 struct RunTotals {
   double forward_ms = 0;
   double backtrace_ms = 0;
+  bool uncounted = false;      // some pairs' backtrace does not count runs
   int launches = 0;
   unsigned long long dsteps = 0;
   unsigned int fail = 0;
@@ -323,6 +325,7 @@ struct wfa_device_batch_t {
             size_t* upload_bytes = nullptr);
   const char* h_ops = nullptr;             // a host copy of the operations (single-pair graph), or null
   // run-length CIGARs of the last run (wfa_device_batch_download_runs), made on first request
+  bool counting = false, counted = false;  // the run / the last run leaves d_run_counts
   wfa_host::DevBuf d_run_counts, d_run_off, d_runs, d_scan_temp;
   bool runs_ready = false;
   long long total_runs = 0;

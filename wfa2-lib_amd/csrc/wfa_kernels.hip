@@ -743,7 +743,11 @@ __device__ __forceinline__ void trace_pair(const BacktraceArgs& a) {
   // A z-dropped pair is traced from the best cell it saw, at the score it
   // dropped at (wavefront_unialign.c:175-200), like an ends-free end cell.
   const bool zd = a.status[p] == kDevZdropped;
-  if (a.status[p] != kDevCompleted && !zd) { a.ops_begin[p] = cap; return; }
+  if (a.status[p] != kDevCompleted && !zd) {
+    a.ops_begin[p] = cap;
+    if (a.run_counts) a.run_counts[p] = 0;
+    return;
+  }
   Penalties pen = a.pen;
   const int cbeg = a.comp_begin_p ? (int)a.comp_begin_p[p] : a.comp_begin;
   int comp = a.comp_end_p ? (int)a.comp_end_p[p] : a.comp_end;
@@ -936,6 +940,7 @@ __device__ __forceinline__ void trace_pair(const BacktraceArgs& a) {
     zback = n < 0 ? -n : 0;
     if (zback > ntrail_all) stale = bad = true;  // would take back past the trailing gaps
   }
+  int runs = 0;
   if (!bad && !direct) {
     // 2M + 2X + I + D = plen + tlen: the match count follows, and with it
     // the CIGAR's length and start (rest >= 0 keeps start in [0, pos - nlead]).
@@ -965,7 +970,14 @@ __device__ __forceinline__ void trace_pair(const BacktraceArgs& a) {
       h += m;
       return bad ? 0 : m;
     };
-    if (!bad && cbeg == kM) ow.advance(matches(zd && nwalk == 0, 0));
+    uint32_t prev = nlead == 0 ? 4u : k > 0 ? 1u : 2u;  // operation of the last run (3: M)
+    runs = nlead > 0;
+    if (!bad && cbeg == kM) {
+      const int m = matches(zd && nwalk == 0, 0);
+      ow.advance(m);
+      runs += m > 0;
+      prev = m > 0 ? 3u : prev;
+    }
     while (walk.n > 0 && !bad) {
       if (ow.w > cap - ntrail - walk.n) { bad = true; break; }  // inconsistent records: never overrun unread operations
       const uint32_t op = walk.pop();
@@ -973,8 +985,15 @@ __device__ __forceinline__ void trace_pair(const BacktraceArgs& a) {
       h += (op & 3u) != 2u;
       const int m = (op & 4u) ? matches(zd && walk.n == 0, 1) : 0;
       ow.put(op_char(op), m);
+      runs += ((op & 3u) != prev) + (m > 0);
+      prev = m > 0 ? 3u : op & 3u;
     }
     ow.finish();
+    if (ntrail_d > 0) {
+      runs += prev != 2u;
+      prev = 2u;
+    }
+    runs += ntrail > ntrail_d && prev != 1u;
     // the trailing gaps are in place
     ow.w += ntrail;
     v += ntrail_d;
@@ -992,6 +1011,7 @@ __device__ __forceinline__ void trace_pair(const BacktraceArgs& a) {
     atomicAdd(a.fail_count, 1u);
   }
   a.ops_begin[p] = start;
+  if (a.run_counts) a.run_counts[p] = bad ? 0 : runs;
 }
 
 template <int BITS>
