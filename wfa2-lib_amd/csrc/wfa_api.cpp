@@ -894,6 +894,9 @@ constexpr int kWideFollowMin = 2048;
 // Arena for the second launch's chunks: some 150 KB for each of up to 1,000
 // workgroups at a time.
 constexpr double kWideRecordBytes = 160e6;
+// ... and per pair of the longer class under two gap costs, half of which
+// write 90 KB on 8 diagonals per lane at 10% errors.
+constexpr double kWidePairBytes = 48e3;
 
 bool wide_follows(const Engine* e, const JobSet& js, const PlanGroup& g, const Penalties& pen) {
   return g.family == wfa::kWave && g.wcap == 4 && !e->na && (int)g.ids.size() >= kWideFollowMin && !js.heur.cut() &&
@@ -1027,10 +1030,13 @@ std::vector<PlanGroup> make_plan(const JobSet& js, const std::vector<int>& ids, 
   const int wave_free = js.ef.on ? std::max(js.ef.pbf + js.ef.pef, js.ef.tbf + js.ef.tef) : 0;
   for (int i : ids) {
     const int L = std::max(js.h_plen[i], js.h_tlen[i]);
-    // (with a second gap, pairs of the longer class outgrow a wave: tiles)
-    if (wave_ok && L <= (ncomp == 5 && tile_ok ? lt.short_len : kLeanMaxLen)) {
-      // (free ends add symbols, not errors)
-      const int c = L - wave_free <= lt.short_len ? 0 : 1;
+    if (wave_ok && L <= kLeanMaxLen) {
+      // (free ends add symbols, not errors; with a second gap 8 diagonals per
+      // lane leave two waves per SIMD, so all pairs start with 4: 20,000 pairs
+      // of 500-1,000 bp at 0-3% errors 5.9 -> 1.1 ms against tiles at once,
+      // 30,000 of 330-350 bp at 0-10% 7.9 -> 2.2 ms; 6,000 of 950-1,000 bp at
+      // 0-10%, half of which go on to tiles, 5.5 -> 6.6 ms)
+      const int c = ncomp == 5 || L - wave_free <= lt.short_len ? 0 : 1;
       wave_ids[c].push_back(i);
       wave_words[c] = std::max(wave_words[c], js.bits == 2 ? 2 * (L / 32 + 3) : L / 8 + 3);
       continue;
@@ -1117,6 +1123,7 @@ int run_jobs(wavefront_aligner_t* wf, Engine* e, const JobSet& js, std::vector<P
         for (int i : g.ids) {
           const double L = std::max(js.h_plen[i], js.h_tlen[i]);
           w += L * L * per_l2 + 8 * L;
+          if (g.family == wfa::kWave && pen.ncomp == 5 && L > lean_tuning().short_len) w += kWidePairBytes;
         }
         g.est_rec_bytes = w;
         set_wave(js, g, pen, records);
