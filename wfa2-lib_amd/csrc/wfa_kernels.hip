@@ -633,6 +633,90 @@ __global__ void __launch_bounds__(BLOCK, BLOCK == 1024 ? 4 : 1) wfa_forward_kern
   if (tid == 0 && wg_dsteps) atomicAdd(a.dsteps_total, wg_dsteps);
 }
 
+// Sixteen bytes of a CIGAR slot gathered in registers before one aligned
+// 16-byte store (one lane per pair: a store of a wave touches 64 different
+// lines).  A chunk starts out as matches, so setting a byte, once, is one
+// exclusive or, and a match is there already.
+struct OpChunk {
+  static constexpr uint64_t kMatches = 0x4D4D4D4D4D4D4D4Dull;  // 'M'
+  uint64_t lo = kMatches, hi = kMatches;
+  __device__ __forceinline__ void set(int b, unsigned op) {
+    const uint64_t x = (uint64_t)((op ^ 0x4Du) & 0xFFu) << (8 * (b & 7));
+    lo ^= b < 8 ? x : 0u;
+    hi ^= b < 8 ? 0u : x;
+  }
+  __device__ __forceinline__ void store(unsigned char* at) const {
+    *reinterpret_cast<uint4*>(at) = make_uint4((uint32_t)lo, (uint32_t)(lo >> 32), (uint32_t)hi, (uint32_t)(hi >> 32));
+  }
+  // Bytes [from, to) of the chunk whose byte 0 is at `at`, one by one.
+  __device__ __forceinline__ void bytes(unsigned char* at, int from, int to) const {
+    for (int b = from; b < to; ++b) at[b] = (unsigned char)((b < 8 ? lo : hi) >> (8 * (b & 7)));
+  }
+  __device__ __forceinline__ void clear() { lo = hi = kMatches; }
+};
+
+__device__ __forceinline__ int chunk_phase(const unsigned char* at) {
+  return (int)(reinterpret_cast<uintptr_t>(at) & 15u);
+}
+
+// Forward writer of the replay: consecutive bytes from position w0 of a slot.
+// A run of matches is nothing but a step of w.  A chunk that reaches below w0
+// is written byte by byte, and so is the started chunk at the end (finish): no
+// byte outside [w0, w) is touched, the neighbouring slots belong to other
+// lanes.
+struct OpWriter {
+  unsigned char* out;
+  int w, w0;
+  OpChunk c;  // the chunk holding position w: its bytes below w, matches above
+  // Moves on by n bytes: what the chunk holds at them, matches beyond it.
+  __device__ __forceinline__ void advance(int n) {
+    int base = w - chunk_phase(out + w);
+    w += n;
+    if (w - base < 16) return;
+    if (base >= w0) c.store(out + base);
+    else c.bytes(out + base, w0 - base, 16);
+    c.clear();
+    for (base += 16; w - base >= 16; base += 16) c.store(out + base);
+  }
+  // One operation, then m matches.
+  __device__ __forceinline__ void put(unsigned op, int m = 0) {
+    c.set(chunk_phase(out + w), op);
+    advance(1 + m);
+  }
+  __device__ __forceinline__ void run(unsigned op, int m) {
+    if (op == 'M') advance(m);
+    else
+      for (int i = 0; i < m; ++i) put(op);
+  }
+  __device__ __forceinline__ void finish() const {
+    const int d = chunk_phase(out + w), base = w - d;
+    c.bytes(out + base, max(w0 - base, 0), d);
+  }
+};
+
+// Backward writer: bytes at descending positions below top.  A chunk that
+// reaches top (the bytes from top up belong to another slot) is written byte
+// by byte, and so is the started chunk at the end (finish).
+struct OpWriterBack {
+  unsigned char* out;
+  int p, top;
+  OpChunk c;  // the chunk holding position p: its bytes from p up
+  __device__ __forceinline__ void put(unsigned op) {
+    --p;
+    const int d = chunk_phase(out + p);
+    c.set(d, op);
+    if (d == 0) {
+      if (p + 16 <= top) c.store(out + p);
+      else c.bytes(out + p, 0, top - p);
+      c.clear();
+    }
+  }
+  __device__ __forceinline__ void finish() const {
+    const int d = chunk_phase(out + p), base = p - d;
+    if (d != 0) c.bytes(out + base, d, min(16, top - base));
+  }
+};
+
 // Operations of the walk, the last one on top: four bits each (0 X, 1 I, 2 D;
 // 4: it leads into an M cell), eight to a word.  Full words grow downwards
 // from the end of the slot's free part; the started word stays in a register.
@@ -659,48 +743,6 @@ struct OpStack {
 };
 
 __device__ __forceinline__ unsigned op_char(uint32_t op) { return (0x00444958u >> (8u * (op & 3u))) & 0xFFu; }
-
-// Forward writer of the replay from position w0 of a slot, in aligned 16-byte
-// stores (one lane per pair: a store of a wave touches 64 different lines).  The chunk holding position w starts out as matches, so a run of
-// matches is nothing but a step of w, and an operation one exclusive or.  A
-// chunk that reaches below w0 is written byte by byte, and so is the started
-// chunk at the end (finish): no byte outside [w0, w) is touched, the
-// neighbouring slots belong to other lanes.
-struct OpWriter {
-  static constexpr uint64_t kMatches = 0x4D4D4D4D4D4D4D4Dull;  // 'M'
-  unsigned char* out;
-  int w, w0;
-  uint64_t lo, hi;
-  __device__ __forceinline__ OpWriter(unsigned char* slot, int begin)
-      : out(slot), w(begin), w0(begin), lo(kMatches), hi(kMatches) {}
-  __device__ __forceinline__ int phase() const { return (int)(reinterpret_cast<uintptr_t>(out + w) & 15u); }
-  __device__ __forceinline__ void bytes(int base, int to) const {
-    for (int i = max(base, w0); i < to; ++i) {
-      const int b = i - base;
-      out[i] = (unsigned char)((b < 8 ? lo : hi) >> (8 * (b & 7)));
-    }
-  }
-  // Moves on by n bytes: what the chunk holds at them, matches beyond it.
-  __device__ __forceinline__ void advance(int n) {
-    int base = w - phase();
-    w += n;
-    if (w - base < 16) return;
-    if (base >= w0) *reinterpret_cast<ulonglong2*>(out + base) = make_ulonglong2(lo, hi);
-    else bytes(base, base + 16);
-    lo = hi = kMatches;
-    for (base += 16; w - base >= 16; base += 16)
-      *reinterpret_cast<ulonglong2*>(out + base) = make_ulonglong2(kMatches, kMatches);
-  }
-  // One operation, then m matches.
-  __device__ __forceinline__ void put(unsigned op, int m) {
-    const int d = phase();
-    const uint64_t x = (uint64_t)(op ^ 0x4Du) << (8 * (d & 7));
-    lo ^= d < 8 ? x : 0u;
-    hi ^= d < 8 ? 0u : x;
-    advance(1 + m);
-  }
-  __device__ __forceinline__ void finish() const { bytes(w - phase(), w); }
-};
 
 // One lane per pair, in two passes over the pair's CIGAR slot
 // ops[0 .. plen+tlen):
@@ -784,8 +826,11 @@ __device__ __forceinline__ void trace_pair(const BacktraceArgs& a) {
     if (nd < 0 || ni < 0 || nd + ni > cap) {
       bad = true;
     } else if (!zd || direct) {
-      for (int i = 0; i < nd; ++i) out[--pos] = 'D';
-      for (int i = 0; i < ni; ++i) out[--pos] = 'I';
+      OpWriterBack bw{out, pos, pos, OpChunk{}};
+      for (int i = 0; i < nd; ++i) bw.put('D');
+      for (int i = 0; i < ni; ++i) bw.put('I');
+      bw.finish();
+      pos = bw.p;
       ntrail_d = nd;
     }
   }
@@ -796,9 +841,12 @@ __device__ __forceinline__ void trace_pair(const BacktraceArgs& a) {
     if (vE < 0 || hE < 0 || vE + hE - m > pos) {
       bad = true;
     } else {
-      for (int i = 0; i < m; ++i) out[--pos] = 'M';
-      for (int i = 0; i < vE - m; ++i) out[--pos] = 'D';
-      for (int i = 0; i < hE - m; ++i) out[--pos] = 'I';
+      OpWriterBack bw{out, pos, pos, OpChunk{}};
+      for (int i = 0; i < m; ++i) bw.put('M');
+      for (int i = 0; i < vE - m; ++i) bw.put('D');
+      for (int i = 0; i < hE - m; ++i) bw.put('I');
+      bw.finish();
+      pos = bw.p;
     }
   }
   bool mark = comp == kM;  // the next operation written leads into an M cell
@@ -955,11 +1003,11 @@ __device__ __forceinline__ void trace_pair(const BacktraceArgs& a) {
       len = bad ? 0 : rest / 2 + nwalk + ntrail + nlead;
     }
     start = bad ? cap : cap - len;
-    OpWriter ow(out, start);
+    OpWriter ow{out, start, start, OpChunk{}};
     int v = 0, h = 0;
     if (!bad) {
       // free leading gaps
-      for (int i = 0; i < nlead; ++i) ow.put(k > 0 ? 'I' : 'D', 0);
+      ow.run(k > 0 ? 'I' : 'D', nlead);
       if (k > 0) h = k; else v = -k;
     }
     // The matches at (v, h), or a z-drop's last run; bad when the slot cannot hold them.
