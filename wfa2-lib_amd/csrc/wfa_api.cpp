@@ -1871,12 +1871,17 @@ int batch_run(wavefront_aligner_t* wf, wfa_device_batch_t* b, Engine* e) {
     give_back_groups(e, plan);
     if (rc != WF_STATUS_OK) return rc;
   } else {
-    const std::vector<int> key = {pen.metric, pen.x, pen.o1, pen.e1, pen.o2, pen.e2, b->bits, b->ef.on,
-                                  b->heur.cut(), records, b->unlimited};
+    // The tuner's choices hold for the kernel instance (cut()); the plan also
+    // for what make_plan chose the families by: a change of strategy between
+    // two runs of the batch plans again.
+    const std::vector<int> conf = {pen.metric, pen.x, pen.o1, pen.e1, pen.o2, pen.e2, b->bits, b->ef.on,
+                                   b->heur.cut(), records, b->unlimited};
+    std::vector<int> key = conf;
+    key.insert(key.end(), {b->heur.wfadaptive, b->heur.xdrop, b->heur.zdrop, b->heur.banded});
     if (b->plan_key != key) {
       std::vector<PlanGroup> plan = make_plan(b->jobs(), b->sorted, pen);
       std::vector<TuneTrial> trials;
-      if (env_on("WFA_AUTOTUNE", true)) tune_plan(e, b->jobs(), key, plan, &trials);
+      if (env_on("WFA_AUTOTUNE", true)) tune_plan(e, b->jobs(), conf, plan, &trials);
       if (!trials.empty()) {
         // measure the candidates on their slices (aligning those pairs)
         rc = run_trials(wf, e, b->jobs(), records, trials, &tot);

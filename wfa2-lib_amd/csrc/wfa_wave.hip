@@ -957,6 +957,8 @@ int wave_max_blocks_per_cu(int shape, int nmax, bool rec, int bits, bool ef, boo
 
 hipError_t launch_forward_wave(const ForwardArgs& a, int shape, int nmax, int bits, const LaunchShape& ls,
                                hipStream_t stream) {
+  // a cut-off that the kernel does not do, or one where none is asked for
+  if ((a.wave.cut != 0) != (a.heur.cut() != 0) || (a.wave.cut && !wave_cuts(shape, a.heur))) return hipErrorInvalidValue;
   const void* f = a.wave.cut ? select_wave_cut(a.records != 0)
                              : select_wave(shape, nmax, a.records != 0, bits, a.endsfree != 0);
   if (!f || ls.block != 64) return hipErrorInvalidValue;
