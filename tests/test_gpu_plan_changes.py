@@ -28,11 +28,11 @@ def pairs(seed):
                                       a.texts() + b.texts() + s.texts())
 
 
-def check(al, db, ps, label, **kw):
+def check(al, db, ps, label, metric="affine", pen=PEN, **kw):
     say(label)
     db.run()
     got = db.download()
-    ref = O.oracle_align(O.Conf("affine", PEN, "high", **kw), O.Pairs(ps.patterns(), ps.texts()))
+    ref = O.oracle_align(O.Conf(metric, pen, "high", **kw), O.Pairs(ps.patterns(), ps.texts()))
     stale = np.asarray(ref.stale[:ps.n], dtype=bool)
     assert [i for i in range(ps.n) if got.status[i] == wfa_amd.WF_STATUS_UNSUPPORTED] == list(np.flatnonzero(stale)), label
     bad = [i for i in range(ps.n) if not stale[i] and
@@ -64,3 +64,29 @@ def test_heuristics_changed_between_runs():
     check(al, db, ps, "wf-adaptive, other limits", heuristic=(4, 10, 30, 2))
     L.wavefront_aligner_set_heuristic_none(al.wf)
     check(al, db, ps, "none")
+
+
+@pytest.mark.parametrize("metric,pen", [("affine", PEN), ("affine2p", (0, 4, 6, 2, 24, 1)), ("linear", (0, 4, 2))],
+                         ids=["affine", "affine2p", "linear"])
+def test_free_ends_changed_between_runs(metric, pen):
+    """Free ends whose score-0 wavefront fits a wave at 1, 4 and 8 diagonals
+    per lane and not at all (a pair starts on 4 at most), grown and shrunk."""
+    rng = np.random.default_rng(612)
+    base = np.frombuffer(b"ACGT", dtype=np.uint8)
+    P, T = [], []
+    for i in range(48):
+        t = base[rng.integers(0, 4, int(rng.integers(640, 900)))]
+        at = int(rng.integers(0, len(t) - 300)) if i % 3 else 250
+        p = t[at:at + int(rng.integers(200, 300))].copy()
+        p[rng.integers(0, len(p), 8)] = base[rng.integers(0, 4, 8)]
+        P.append(base[rng.integers(0, 4, 180 if i % 2 else 1)].tobytes() + p.tobytes())
+        T.append(t.tobytes())
+    ps = datagen.PairSet.from_lists(P, T)
+    al = wfa_amd.Aligner(metric=metric, penalties=pen)
+    L = wfa_amd.lib()
+    db = al.upload(ps)
+    for free in ((0, 0, 30, 30), (0, 0, 300, 100), (0, 0, 600, 200), (100, 0, 140, 20), (150, 0, 150, 0), (0, 10, 30, 0)):
+        L.wavefront_aligner_set_alignment_free_ends(al.wf, *free)
+        check(al, db, ps, "%s %s" % (metric, free), metric, pen, ends_free=free)
+    L.wavefront_aligner_set_alignment_end_to_end(al.wf)
+    check(al, db, ps, "%s end to end" % metric, metric, pen)

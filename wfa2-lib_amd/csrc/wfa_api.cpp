@@ -855,7 +855,8 @@ void group_args(wavefront_aligner_t* wf, Engine* e, const JobSet& js, const Plan
   *pba = ba;
 }
 
-// The kernel and phases of a wave group.
+// The kernel and phases of a wave group (of a score-0 wavefront that does not
+// fit the wave, which make_plan keeps out: phases that the launch refuses).
 void set_wave(const JobSet& js, PlanGroup& g, const Penalties& pen, int records) {
   if (g.family != wfa::kWave) return;
   g.wave_rec = records != 0;
@@ -1872,12 +1873,13 @@ int batch_run(wavefront_aligner_t* wf, wfa_device_batch_t* b, Engine* e) {
     if (rc != WF_STATUS_OK) return rc;
   } else {
     // The tuner's choices hold for the kernel instance (cut()); the plan also
-    // for what make_plan chose the families by: a change of strategy between
-    // two runs of the batch plans again.
+    // for what make_plan chose the families by: a change of strategy or of the
+    // free ends between two runs of the batch plans again.
     const std::vector<int> conf = {pen.metric, pen.x, pen.o1, pen.e1, pen.o2, pen.e2, b->bits, b->ef.on,
                                    b->heur.cut(), records, b->unlimited};
     std::vector<int> key = conf;
-    key.insert(key.end(), {b->heur.wfadaptive, b->heur.xdrop, b->heur.zdrop, b->heur.banded});
+    key.insert(key.end(), {b->heur.wfadaptive, b->heur.xdrop, b->heur.zdrop, b->heur.banded, b->ef.pbf,
+                           b->ef.pef, b->ef.tbf, b->ef.tef});
     if (b->plan_key != key) {
       std::vector<PlanGroup> plan = make_plan(b->jobs(), b->sorted, pen);
       std::vector<TuneTrial> trials;

@@ -959,6 +959,8 @@ hipError_t launch_forward_wave(const ForwardArgs& a, int shape, int nmax, int bi
                                hipStream_t stream) {
   // a cut-off that the kernel does not do, or one where none is asked for
   if ((a.wave.cut != 0) != (a.heur.cut() != 0) || (a.wave.cut && !wave_cuts(shape, a.heur))) return hipErrorInvalidValue;
+  // a score-0 wavefront that needs more than the 4 diagonals per lane a pair starts with at most
+  if (!a.wave.cut && (a.wave.phase0 < 0 || a.wave.phase0 > 2)) return hipErrorInvalidValue;
   const void* f = a.wave.cut ? select_wave_cut(a.records != 0)
                              : select_wave(shape, nmax, a.records != 0, bits, a.endsfree != 0);
   if (!f || ls.block != 64) return hipErrorInvalidValue;
