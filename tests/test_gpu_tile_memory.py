@@ -1,0 +1,78 @@
+"""Device memory of the tile family (wfa_tile.hip, wfa_tile_run.cpp)."""
+import ctypes
+import sys
+
+import numpy as np
+import pytest
+
+import oracle as O
+import wfa_amd
+from wfa_amd import datagen
+
+pytestmark = pytest.mark.gpu
+
+PEN = (0, 4, 6, 2, 24, 1)
+BASES = np.frombuffer(b"ACGT", dtype=np.uint8)
+
+
+def say(msg):
+    print(msg, flush=True)
+    sys.stdout.flush()
+
+
+def free_device_bytes():
+    hip = ctypes.CDLL("libamdhip64.so")
+    free, total = ctypes.c_size_t(0), ctypes.c_size_t(0)
+    assert hip.hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+    return free.value
+
+
+def mutate(rng, t, e):
+    u = rng.random(len(t))
+    out = t.copy()
+    sub = u < e / 3
+    out[sub] = BASES[rng.integers(0, 4, int(sub.sum()))]
+    reps = np.ones(len(t), dtype=np.int64)
+    reps[(u >= e / 3) & (u < 2 * e / 3)] = 2
+    reps[(u >= 2 * e / 3) & (u < e)] = 0
+    return np.repeat(out, reps).tobytes()
+
+
+def pair(rng, n, e):
+    t = BASES[rng.integers(0, 4, n)]
+    return mutate(rng, t, e), t.tobytes()
+
+
+def assert_same(got, ref, ids):
+    bad = [i for x, i in enumerate(ids) if got.status[i] != ref.status[x] or got.score[i] != ref.score[x] or
+           got.ops(i) != ref.ops(x)]
+    assert not bad, (bad[:10], got.status[bad[0]], got.score[bad[0]])
+
+
+def test_one_long_pair_among_many_reads(monkeypatch):
+    """100,000 reads and one pair of 30 kbp: beside what the reads take, the
+    pair takes its 62 rows of 61,000 diagonals (15 MB), a table of 5,000
+    blocks and its sequences and CIGAR, not a table for every read (2 GB)."""
+    monkeypatch.setenv("WFA_RECORD_ARENA_MB", "256")
+    rng = np.random.default_rng(5)
+    reads = datagen.generate(1, 91, 100000)
+    P, T = reads.patterns(), reads.texts()
+    long_p, long_t = pair(rng, 30000, 0.003)
+    used = []
+    for extra in (0, 1):
+        ps = datagen.PairSet.from_lists(P + [long_p] * extra, T + [long_t] * extra)
+        al = wfa_amd.Aligner(metric="affine2p", penalties=PEN)
+        db = al.upload(ps)
+        before = free_device_bytes()
+        assert db.run() == 0
+        used.append(before - free_device_bytes())
+        say("%d pairs: %.0f MB" % (ps.n, used[-1] / 1e6))
+        if extra:
+            got = db.download()
+            ids = list(range(0, reads.n, 997)) + [reads.n]
+            ref = O.oracle_align(O.Conf("affine2p", PEN, "high"),
+                                 O.Pairs([ps.pattern(i) for i in ids], [ps.text(i) for i in ids]))
+            assert_same(got, ref, ids)
+        db.free()
+        al.close()
+    assert used[1] - used[0] < 128e6

@@ -249,7 +249,7 @@ bool bi_fast_forward(Engine* e, const std::vector<wfa::BiProblem>& probs, wfa::B
     }
     const int slot = chunk & 1;
     if (!hip_ok(wfa::launch_tile_compact(act[which], n_act + which, f.done, nullptr, blk, act[which ^ 1],
-                                         n_act + (which ^ 1), const_cast<int*>(h_n) + slot, st), "bi tile compact") ||
+                                         n_act + (which ^ 1), nullptr, const_cast<int*>(h_n) + slot, st), "bi tile compact") ||
         !hip_ok(hipEventRecord(t.ev[slot], st), "bi tile event"))
       return false;
     which ^= 1;

@@ -151,8 +151,9 @@ struct Engine {
   struct TileState {
     int shape = 0;
     std::vector<int> lo, hi;          // hull of the ranges up to each step
-    DevBuf d_range, d_dsteps, d_job_range, d_dev, d_ends, d_flags, d_dsum, d_step_state, d_step_off, d_step0, d_step_act, d_off, d_pitch, d_jobs, d_marks, d_act, d_info, d_tab;
+    DevBuf d_range, d_dsteps, d_job_range, d_dev, d_ends, d_flags, d_dsum, d_step_state, d_step_off, d_step0, d_step_act, d_up, d_jobs, d_marks, d_act, d_tab;
     HostBuf h_n;                      // jobs left, written by the device
+    HostBuf h_up;                     // what goes up for a pass
     hipEvent_t ev[5] = {nullptr, nullptr, nullptr, nullptr, nullptr};
   } tile;
   // BiWFA sub-problems in tiles (wfa_bialign.cpp): range tables and buffers.

@@ -26,17 +26,33 @@ struct TileRange {
   int left, right, min_lo, max_hi;
 };
 
-struct TileArgs {
-  const int* act;              // active jobs
-  const int* n_act;
+// A job of a pass.  Everything the tiles keep of a job is found by its slot in
+// the pass, not by its id in the batch: the buffers are as large as the pass,
+// however many other pairs the batch has.
+struct TileJob {
+  int64_t ppos, tpos;          // its sequences (symbols)
+  int64_t st_off;              // first int of its state
+  int plen, tlen;
+  int pitch;                   // ints per state row
+  int id;
+};
+struct TileSeqs {              // of the batch, by id
   const int* plen;
   const int* tlen;
-  const uint64_t* words;
   const int64_t* pat_pos;
   const int64_t* txt_pos;
+};
+struct TileSlot {              // what the host says of a job
+  int64_t st_off;
+  int id, pad;
+};
+
+struct TileArgs {
+  const int* act;              // slots of the active jobs
+  const int* n_act;
+  TileJob* jobs;
+  const uint64_t* words;
   int* state;                  // rows of every job
-  const int64_t* st_off;       // first int of a job's state
-  const int* st_pitch;         // ints per row
   int* done;                   // step at which the job reached its end (INT_MAX: not yet)
   int* irr;                    // first step whose end left its tile (INT_MAX: none)
   TileRange* range;            // per job, of the last four blocks
@@ -65,14 +81,10 @@ constexpr int kTileStepEnds = 12, kTileStepFlags = 32;
 struct StepArgs {
   const int* act;
   const int* n_act;
-  const int* plen;
-  const int* tlen;
+  const TileJob* jobs;
   const uint64_t* words;
-  const int64_t* pat_pos;
-  const int64_t* txt_pos;
   int* state;
-  const int64_t* st_off;       // first int of a job's rows
-  const int* st_pitch;
+  const int64_t* st_off;       // first int of a job's rows here
   int* done;
   int* ends;                   // per job, ring of 4 steps: kTileStepEnds ends of the components
   int* flags;                  // per job, ring of kTileStepFlags steps: which components have a valid cell
@@ -88,9 +100,7 @@ struct StepArgs {
 
 struct TileFinishArgs {
   int n;
-  const int* jobs;             // null: 0..n-1
-  const int* plen;
-  const int* tlen;
+  const TileJob* jobs;
   const int* done;
   const int* irr;
   const long long* dsteps_upto;
@@ -114,9 +124,7 @@ struct TileFinishArgs {
 };
 
 struct TileTraceArgs {
-  const int* jobs;
-  const int* plen;
-  const int* tlen;
+  const TileJob* jobs;
   int* status;
   const int* score;
   const uint4* rec;
@@ -124,8 +132,6 @@ struct TileTraceArgs {
   int tab_stride;
   const TileBlockInfo* blocks;
   const uint64_t* words;
-  const int64_t* pat_pos;
-  const int64_t* txt_pos;
   char* ops;
   const int64_t* ops_off;
   int* ops_begin;
@@ -181,12 +187,17 @@ int bi_tile_useful();          // diagonals per tile
 hipError_t launch_bi_tile_init(const BiTileArgs& a, int* act, int* n_act, hipStream_t st);
 hipError_t launch_bi_tile_block(const BiTileArgs& a, int problems, int tiles, hipStream_t st);
 hipError_t launch_tile_fill(int* state, long long ints, hipStream_t st);
-hipError_t launch_tile_init(int shape, const TileArgs& a, int n, const int* jobs, int* act, int* n_act, hipStream_t st);
+// The jobs of a pass from their slots, their score-0 rows and marks, the first
+// active list (act, n_act) and the count of lost jobs.
+hipError_t launch_tile_init(int shape, const TileArgs& a, int n, const TileSlot* slots, const TileSeqs& seqs, int* act,
+                            int* n_act, int* lost, hipStream_t st);
 hipError_t launch_tile_block(int shape, bool records, const TileArgs& a, int jobs, hipStream_t st);
 hipError_t launch_tile_step_init(int shape, const StepArgs& a, const TileArgs& t, int n, int max_pitch, hipStream_t st);
 hipError_t launch_tile_step(int shape, bool records, const StepArgs& a, int t, int jobs, int max_width, hipStream_t st);
+// host_n[0]: the jobs left, host_n[kTileHostLost]: the jobs lost so far (with irr).
+constexpr int kTileHostLost = 4;
 hipError_t launch_tile_compact(const int* act, const int* n_act, const int* done, const int* irr, int ib, int* act2,
-                               int* n_act2, int* host_n, hipStream_t st);
+                               int* n_act2, int* lost, int* host_n, hipStream_t st);
 hipError_t launch_tile_finish(int shape, const TileFinishArgs& a, hipStream_t st);
 hipError_t launch_tile_backtrace(int shape, const TileTraceArgs& a, int n, hipStream_t st);
 

@@ -109,8 +109,9 @@ __global__ void __launch_bounds__(64 * kTileWaves) wfa_tile_kernel(TileArgs a) {
   const int tiles = (right - left + U - 1) / U;
   const int quads = (right - left) / 4;  // tiles of equal width, in units of four diagonals
   if ((int)blockIdx.x * kTileWaves >= tiles) return;
-  const int plen = a.plen[job], tlen = a.tlen[job];
-  const long long ppos = a.pat_pos[job], tpos = a.txt_pos[job];
+  const TileJob jb = a.jobs[job];
+  const int plen = jb.plen, tlen = jb.tlen;
+  const long long ppos = jb.ppos, tpos = jb.tpos;
   uint64_t* seqP = reinterpret_cast<uint64_t*>(smem);
   uint64_t* seqT = seqP + a.lmax_words;
   {
@@ -133,8 +134,8 @@ __global__ void __launch_bounds__(64 * kTileWaves) wfa_tile_kernel(TileArgs a) {
   const int kend = tlen - plen;
   const bool has_end = kend >= first && kend < past;
   const bool low = tile == 0, high = past == right;
-  const int pitch = a.st_pitch[job];
-  int* st = a.state + a.st_off[job] + (k0 + tile_kpad(plen));
+  const int pitch = jb.pitch;
+  int* st = a.state + jb.st_off + (k0 + tile_kpad(plen));
   auto mrow = [&](int slot) { return st + (long long)slot * pitch; };
   auto grow = [&](int par, int row) { return st + (long long)(G::MS + par * S::kGapRows + row) * pitch; };
   // Rows were written over the diagonals of their block: beyond them the
@@ -349,17 +350,23 @@ __global__ void __launch_bounds__(256) tile_fill_kernel(int4* p, long long n4) {
 // Score 0 of every job (M holds offset 0 at k = 0, extended;
 // wavefront_aligner.c:252-380), its marks, and the first active list.
 template <class S>
-__global__ void __launch_bounds__(64) tile_init_kernel(TileArgs a, int n, const int* jobs, int* act, int* n_act) {
-  const int j = blockIdx.x * 64 + threadIdx.x;
-  if (j == 0) *n_act = n;
-  if (j >= n) return;
-  const int job = jobs ? jobs[j] : j;
-  act[j] = job;
-  const int plen = a.plen[job], tlen = a.tlen[job];
-  const long long ppos = a.pat_pos[job], tpos = a.txt_pos[job];
+__global__ void __launch_bounds__(64) tile_init_kernel(TileArgs a, int n, const TileSlot* slots, TileSeqs seqs, int* act,
+                                                       int* n_act, int* lost) {
+  const int job = blockIdx.x * 64 + threadIdx.x;
+  if (job == 0) {
+    *n_act = n;
+    *lost = 0;
+  }
+  if (job >= n) return;
+  act[job] = job;
+  const TileSlot sl = slots[job];
+  const int plen = seqs.plen[sl.id], tlen = seqs.tlen[sl.id];
+  const long long ppos = seqs.pat_pos[sl.id], tpos = seqs.txt_pos[sl.id];
+  const int pitch = tile_pitch(plen, tlen);
+  a.jobs[job] = TileJob{ppos, tpos, sl.st_off, plen, tlen, pitch, sl.id};
   const int h = lcp_extend<2>(a.words + (ppos >> 5), (int)(ppos & 31), a.words + (tpos >> 5), (int)(tpos & 31), plen,
                               tlen, 0, 0);
-  a.state[a.st_off[job] + (long long)m_slot<S>(-1, -1) * a.st_pitch[job] + tile_kpad(plen)] = h << S::SH;
+  a.state[sl.st_off + (long long)m_slot<S>(-1, -1) * pitch + tile_kpad(plen)] = h << S::SH;
   a.done[job] = (plen == tlen && h >= tlen) ? -1 : INT_MAX;
   a.irr[job] = INT_MAX;
   a.exact_lo[job] = a.exact_hi[job] = a.stepped[job] = 0;
@@ -419,9 +426,10 @@ __global__ void __launch_bounds__(256) tile_step_init_kernel(StepArgs a, TileArg
   constexpr int T = TileGeom<S>::T, MT = TileGeom<S>::MS;
   const int job = a.act[blockIdx.y];
   const int ib = tl.irr[job] / T * T, blk = ib / T;
-  const int pitch = tl.st_pitch[job], kpad = tile_kpad(tl.plen[job]);
+  const TileJob jb = tl.jobs[job];
+  const int pitch = jb.pitch, kpad = tile_kpad(jb.plen);
   const TileRange r1 = tl.range[4 * job + ((blk + 3) & 3)], r2 = tl.range[4 * job + ((blk + 2) & 3)];
-  const int* from = tl.state + tl.st_off[job];
+  const int* from = tl.state + jb.st_off;
   int* to = a.state + a.st_off[job];
   const int x = blockIdx.x * 256 + threadIdx.x;
   int* flags = a.flags + (long long)job * kStepFlags;
@@ -510,13 +518,14 @@ __global__ void __launch_bounds__(64 * kStepWaves) tile_step_kernel(StepArgs a, 
     }
     if (REC && i % T == 0) a.rec_tab[(long long)job * a.tab_stride + i / T] = a.rec_unit0 + blockIdx.y * a.rec_job_units;
   }
-  const int plen = a.plen[job], tlen = a.tlen[job];
+  const TileJob jb = a.jobs[job];
+  const int plen = jb.plen, tlen = jb.tlen;
   const int base = (-plen - 2) & ~3;
   const int first = base + ((int)blockIdx.x * kStepWaves + wid) * (62 * N);
   if (base + (int)blockIdx.x * kStepWaves * (62 * N) > tlen + 1) return;
   const int k0 = first + N * (lane - 1);
   const bool own = lane >= 1 && lane < 63;
-  const int pitch = a.st_pitch[job];
+  const int pitch = jb.pitch;
   const bool some = first <= tlen + 1;  // a wave past the last diagonal has nothing to do
   int rng[kStepEnds];
 #pragma unroll
@@ -541,7 +550,7 @@ __global__ void __launch_bounds__(64 * kStepWaves) tile_step_kernel(StepArgs a, 
       load_gap(i2, kI2, i - S::DE2, e2);
       load_gap(d2, kD2, i - S::DE2, e2);
     }
-    const long long ppos = a.pat_pos[job], tpos = a.txt_pos[job];
+    const long long ppos = jb.ppos, tpos = jb.tpos;
     const WaveSeqs<2> q{reinterpret_cast<const uint32_t*>(a.words + (ppos >> 5)),
                      reinterpret_cast<const uint32_t*>(a.words + (tpos >> 5)), 2u * (unsigned)(ppos & 31),
                      2u * (unsigned)(tpos & 31), plen, tlen};
@@ -601,14 +610,15 @@ __global__ void __launch_bounds__(64 * kStepWaves) tile_step_kernel(StepArgs a, 
 }
 
 // Drops the jobs marked before step ib from the active list (one workgroup;
-// the order stays) and tells the host how many are left.
+// the order stays) and tells the host how many are left, and how many were
+// lost so far (their end left its tile).
 __global__ void __launch_bounds__(1024) tile_compact_kernel(const int* act, const int* n_act, const int* done,
                                                             const int* irr, int ib, int* act2, int* n_act2,
-                                                            int* host_n) {
+                                                            int* lost, int* host_n) {
   __shared__ int wave_n[16];
-  __shared__ int total;
+  __shared__ int total, gone;
   const int n = *n_act, lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-  if (threadIdx.x == 0) total = 0;
+  if (threadIdx.x == 0) total = gone = 0;
   __syncthreads();
   for (int b = 0; b < n; b += 1024) {
     const int j = b + (int)threadIdx.x;
@@ -617,6 +627,7 @@ __global__ void __launch_bounds__(1024) tile_compact_kernel(const int* act, cons
     if (j < n) {
       job = act[j];
       keep = done[job] >= ib && (!irr || irr[job] >= ib);
+      if (irr && irr[job] < ib && irr[job] < done[job]) atomicAdd(&gone, 1);
     }
     const unsigned long long bal = __ballot(keep);
     if (lane == 0) wave_n[wid] = (int)__popcll(bal);
@@ -631,7 +642,8 @@ __global__ void __launch_bounds__(1024) tile_compact_kernel(const int* act, cons
   }
   if (threadIdx.x == 0) {
     *n_act2 = total;
-    *host_n = total;
+    host_n[0] = total;
+    if (irr) host_n[kTileHostLost] = *lost += gone;
   }
 }
 
@@ -643,7 +655,7 @@ __global__ void __launch_bounds__(256) tile_finish_kernel(TileFinishArgs a) {
   unsigned long long ds = 0;
   unsigned retry = 0;
   if (j < a.n) {
-    const int job = a.jobs ? a.jobs[j] : j;
+    const int job = j, id = a.jobs[j].id;
     const int d = a.done[job], r = a.irr[job];
     const bool good = d != INT_MAX && r >= d;
     const int status = good ? (int)kDevCompleted : r != INT_MAX ? (int)kDevRingOverflow : (int)kDevArenaFull;
@@ -663,13 +675,13 @@ __global__ void __launch_bounds__(256) tile_finish_kernel(TileFinishArgs a) {
     } else {
       retry = 1;
     }
-    a.out_status[job] = status;
-    a.out_score[job] = good ? (d + 1) * a.g : 0;
-    a.out_dsteps[job] = (long long)ds;
-    a.out_last_block[job] = kNoBlock;
+    a.out_status[id] = status;
+    a.out_score[id] = good ? (d + 1) * a.g : 0;
+    a.out_dsteps[id] = (long long)ds;
+    a.out_last_block[id] = kNoBlock;
     if (a.out_end_k) {
-      a.out_end_k[job] = a.tlen[job] - a.plen[job];
-      a.out_end_off[job] = a.tlen[job];
+      a.out_end_k[id] = a.jobs[j].tlen - a.jobs[j].plen;
+      a.out_end_off[id] = a.jobs[j].tlen;
     }
   }
   for (int o = 32; o > 0; o >>= 1) {
@@ -697,14 +709,15 @@ __global__ void __launch_bounds__(64) tile_backtrace_kernel(TileTraceArgs a) {
   __shared__ __align__(16) uint32_t win[64 * 4];
   __shared__ int win_k[64];
   const int lane = threadIdx.x;
-  const int job = a.jobs ? a.jobs[blockIdx.x] : (int)blockIdx.x;
-  const int plen = a.plen[job], tlen = a.tlen[job], cap = plen + tlen;
-  if (a.status[job] != kDevCompleted) {
-    if (lane == 0) a.ops_begin[job] = cap;
+  const int job = (int)blockIdx.x;
+  const TileJob jb = a.jobs[job];
+  const int plen = jb.plen, tlen = jb.tlen, cap = plen + tlen;
+  if (a.status[jb.id] != kDevCompleted) {
+    if (lane == 0) a.ops_begin[jb.id] = cap;
     return;
   }
-  unsigned char* out = reinterpret_cast<unsigned char*>(a.ops + a.ops_off[job]);
-  int i = a.score[job] / a.g - 1;  // row of the end cell
+  unsigned char* out = reinterpret_cast<unsigned char*>(a.ops + a.ops_off[jb.id]);
+  int i = a.score[jb.id] / a.g - 1;  // row of the end cell
   int k = tlen - plen, comp = kM, n = 0, nx = 0;
   bool mark = true, bad = false;
   int win_i = INT_MIN;             // row of lane 0's window line
@@ -782,7 +795,7 @@ __global__ void __launch_bounds__(64) tile_backtrace_kernel(TileTraceArgs a) {
   if (rest < 0 || (rest & 1)) bad = true;
   const int start = bad ? cap : pos - rest / 2;
   if (!bad) {
-    const long long ppos = a.pat_pos[job], tpos = a.txt_pos[job];
+    const long long ppos = jb.ppos, tpos = jb.tpos;
     const uint32_t* P = reinterpret_cast<const uint32_t*>(a.words + (ppos >> 5));
     const uint32_t* Q = reinterpret_cast<const uint32_t*>(a.words + (tpos >> 5));
     const unsigned pbit = 2u * (unsigned)(ppos & 31), tbit = 2u * (unsigned)(tpos & 31);
@@ -832,10 +845,10 @@ __global__ void __launch_bounds__(64) tile_backtrace_kernel(TileTraceArgs a) {
   }
   if (lane == 0) {
     if (bad) {
-      a.status[job] = kDevBadTrace;
+      a.status[jb.id] = kDevBadTrace;
       atomicAdd(a.fail_count, 1u);
     }
-    a.ops_begin[job] = bad ? cap : start;
+    a.ops_begin[jb.id] = bad ? cap : start;
   }
 }
 
@@ -1074,10 +1087,11 @@ hipError_t launch_tile_fill(int* state, long long ints, hipStream_t st) {
   return hipGetLastError();
 }
 
-hipError_t launch_tile_init(int shape, const TileArgs& a, int n, const int* jobs, int* act, int* n_act,
-                            hipStream_t st) {
-  if (shape == 2) hipLaunchKernelGGL(tile_init_kernel<Shape2p>, dim3((n + 63) / 64), dim3(64), 0, st, a, n, jobs, act, n_act);
-  else hipLaunchKernelGGL(tile_init_kernel<ShapeAffine>, dim3((n + 63) / 64), dim3(64), 0, st, a, n, jobs, act, n_act);
+hipError_t launch_tile_init(int shape, const TileArgs& a, int n, const TileSlot* slots, const TileSeqs& seqs, int* act,
+                            int* n_act, int* lost, hipStream_t st) {
+  const dim3 grid((n + 63) / 64), block(64);
+  if (shape == 2) hipLaunchKernelGGL(tile_init_kernel<Shape2p>, grid, block, 0, st, a, n, slots, seqs, act, n_act, lost);
+  else hipLaunchKernelGGL(tile_init_kernel<ShapeAffine>, grid, block, 0, st, a, n, slots, seqs, act, n_act, lost);
   return hipGetLastError();
 }
 
@@ -1116,8 +1130,8 @@ hipError_t launch_tile_step(int shape, bool records, const StepArgs& a, int t, i
 }
 
 hipError_t launch_tile_compact(const int* act, const int* n_act, const int* done, const int* irr, int ib, int* act2,
-                               int* n_act2, int* host_n, hipStream_t st) {
-  hipLaunchKernelGGL(tile_compact_kernel, dim3(1), dim3(1024), 0, st, act, n_act, done, irr, ib, act2, n_act2, host_n);
+                               int* n_act2, int* lost, int* host_n, hipStream_t st) {
+  hipLaunchKernelGGL(tile_compact_kernel, dim3(1), dim3(1024), 0, st, act, n_act, done, irr, ib, act2, n_act2, lost, host_n);
   return hipGetLastError();
 }
 

@@ -11,7 +11,8 @@
 namespace wfa_host {
 namespace {
 
-// State rows of the jobs that run at once.
+// State rows of the jobs that run at once.  All other buffers of a pass are
+// per job of the pass too (wfa::TileJob).
 constexpr size_t kTileStateBytes = size_t(24) << 30;
 constexpr int kTileMaxJobs = 32768;  // grid y
 // Records a long pair is planned with: 1-20 kbp pairs of 1-15% error write
@@ -76,43 +77,45 @@ bool tile_fits(int plen, int tlen) {
 // The jobs whose ends moved past their end tiles, one step per launch from
 // the start of the block that found it, all of them side by side.  `unit`:
 // record units taken so far.  Jobs left when the records run out stay
-// unfinished (they are re-run with the records free again).
+// unfinished (they are re-run with the records free again).  Jobs are slots of
+// the pass, `ids` their pairs.
 int run_steps(Engine* e, const JobSet& js, int shape, const wfa::TileGeometry& g, const wfa::TileArgs& a,
               const int* ids, int n_pass, const std::vector<wfa::TileBlockInfo>& info, int records,
               uint64_t rec_units, uint64_t* unit) {
   Engine::TileState& t = e->tile;
   hipStream_t st = e->stream;
   const int T = g.steps;
-  std::vector<int> marks(2 * (size_t)js.n);
+  std::vector<int> marks(2 * (size_t)n_pass);
   if (!hip_ok(hipMemcpyAsync(marks.data(), a.done, marks.size() * 4, hipMemcpyDeviceToHost, st), "tile marks") ||
       !hip_ok(hipStreamSynchronize(st), "tile marks"))
     return WF_STATUS_OOM;
   const int* done = marks.data();
-  const int* irr = done + js.n;
+  const int* irr = done + n_pass;
   std::vector<int> jobs;
   for (int x = 0; x < n_pass; ++x)
-    if (irr[ids[x]] != INT_MAX && irr[ids[x]] < done[ids[x]]) jobs.push_back(ids[x]);
-  const bool ok = t.d_ends.ensure((size_t)js.n * 4 * wfa::kTileStepEnds * 4) &&
-                  t.d_flags.ensure((size_t)js.n * wfa::kTileStepFlags * 4) && t.d_dsum.ensure((size_t)js.n * 8);
+    if (irr[x] != INT_MAX && irr[x] < done[x]) jobs.push_back(x);
+  const bool ok = jobs.empty() || (t.d_ends.ensure((size_t)n_pass * 4 * wfa::kTileStepEnds * 4) &&
+                                   t.d_flags.ensure((size_t)n_pass * wfa::kTileStepFlags * 4) &&
+                                   t.d_dsum.ensure((size_t)n_pass * 8) && t.d_step0.ensure((size_t)n_pass * 4) &&
+                                   t.d_step_off.ensure((size_t)n_pass * 8));
   if (!ok) return WF_STATUS_OOM;
   // as many at once as their rows' memory allows
   for (size_t first = 0; first < jobs.size();) {
-    std::vector<int64_t> off(js.n, 0);
+    std::vector<int64_t> off(n_pass, 0);
     int64_t ints = 0;
     int n = 0, max_pitch = 0, max_width = 0;
     while (first + n < jobs.size()) {
-      const int i = jobs[first + n], pitch = wfa::tile_pitch(js.h_plen[i], js.h_tlen[i]);
+      const int x = jobs[first + n], i = ids[x], pitch = wfa::tile_pitch(js.h_plen[i], js.h_tlen[i]);
       const int64_t need = (int64_t)pitch * g.step_rows;
       if (n > 0 && (size_t)(ints + need) * 4 > kTileStateBytes) break;
-      off[i] = ints;
+      off[x] = ints;
       ints += need;
       max_pitch = std::max(max_pitch, pitch);
       max_width = std::max(max_width, js.h_plen[i] + js.h_tlen[i] + 4);
       ++n;
     }
     const int* sel = jobs.data() + first;
-    if (!t.d_step_state.ensure((size_t)ints * 4) || !t.d_step_off.ensure((size_t)js.n * 8) ||
-        !t.d_step0.ensure((size_t)js.n * 4) || !t.d_step_act.ensure((size_t)2 * n * 4 + 64)) {
+    if (!t.d_step_state.ensure((size_t)ints * 4) || !t.d_step_act.ensure((size_t)2 * n * 4 + 64)) {
       fprintf(stderr, "[WFA] cannot allocate %zu MB of wavefront rows\n", (size_t)ints >> 18);
       return WF_STATUS_OOM;
     }
@@ -121,14 +124,10 @@ int run_steps(Engine* e, const JobSet& js, int shape, const wfa::TileGeometry& g
     wfa::StepArgs s{};
     s.act = act[0];
     s.n_act = n_act;
-    s.plen = js.plen;
-    s.tlen = js.tlen;
+    s.jobs = a.jobs;
     s.words = js.words;
-    s.pat_pos = js.ppos;
-    s.txt_pos = js.tpos;
     s.state = t.d_step_state.as<int>();
     s.st_off = t.d_step_off.as<int64_t>();
-    s.st_pitch = a.st_pitch;
     s.done = a.done;
     s.ends = t.d_ends.as<int>();
     s.flags = t.d_flags.as<int>();
@@ -137,9 +136,9 @@ int run_steps(Engine* e, const JobSet& js, int shape, const wfa::TileGeometry& g
     s.rec = a.rec;
     s.rec_tab = a.rec_tab;
     s.tab_stride = a.tab_stride;
-    s.blocks = t.d_info.as<wfa::TileBlockInfo>();
+    s.blocks = t.d_up.as<wfa::TileBlockInfo>();
     volatile int* h_n = t.h_n.as<int>() + 8;
-    if (!hip_ok(hipMemcpyAsync(t.d_step_off.p, off.data(), (size_t)js.n * 8, hipMemcpyHostToDevice, st), "steps") ||
+    if (!hip_ok(hipMemcpyAsync(t.d_step_off.p, off.data(), (size_t)n_pass * 8, hipMemcpyHostToDevice, st), "steps") ||
         !hip_ok(hipMemcpyAsync(act[0], sel, (size_t)n * 4, hipMemcpyHostToDevice, st), "steps") ||
         !hip_ok(hipMemcpyAsync(n_act, &n, 4, hipMemcpyHostToDevice, st), "steps") ||
         !hip_ok(wfa::launch_tile_step_init(shape, s, a, n, max_pitch, st), "step init"))
@@ -167,7 +166,8 @@ int run_steps(Engine* e, const JobSet& js, int shape, const wfa::TileGeometry& g
           return WF_STATUS_OOM;
       const int slot = b & 1;
       if (!hip_ok(wfa::launch_tile_compact(act[which], n_act + which, a.done, nullptr, INT_MAX, act[which ^ 1],
-                                           n_act + (which ^ 1), const_cast<int*>(h_n) + slot, st), "tile compact") ||
+                                           n_act + (which ^ 1), nullptr, const_cast<int*>(h_n) + slot, st),
+                  "tile compact") ||
           !hip_ok(hipEventRecord(t.ev[3 + slot], st), "tile event"))
         return WF_STATUS_OOM;
       which ^= 1;
@@ -219,18 +219,6 @@ int run_tile_group(Engine* e, const JobSet& js, const PlanGroup& grp, const wfa:
     tiles[b] = (hi0 - lo0 + 1 + 2 * T + 8) / g.useful + 1;
   }
   const int n_all = (int)grp.ids.size();
-  std::vector<int64_t> st_off(js.n, 0);
-  std::vector<int> st_pitch(js.n, 0);
-  if (!t.d_off.ensure((size_t)js.n * 8) || !t.d_pitch.ensure((size_t)js.n * 4) || !t.d_jobs.ensure((size_t)n_all * 4) ||
-      !t.d_marks.ensure((size_t)js.n * 5 * 4) ||
-      !t.d_job_range.ensure((size_t)js.n * 4 * sizeof(wfa::TileRange)) || !t.d_dev.ensure((size_t)js.n * 4 * T * 8) || !t.d_act.ensure((size_t)2 * n_all * 4 + 64) ||
-      !t.d_info.ensure((size_t)max_blocks * sizeof(wfa::TileBlockInfo)) ||
-      (records && !t.d_tab.ensure((size_t)js.n * max_blocks * 4))) {
-    fprintf(stderr, "[WFA] cannot allocate the tile buffers of %d pairs\n", n_all);
-    return WF_STATUS_OOM;
-  }
-  if (!hip_ok(hipMemcpyAsync(t.d_info.p, info.data(), info.size() * sizeof(info[0]), hipMemcpyHostToDevice, st), "tiles"))
-    return WF_STATUS_OOM;
   const uint64_t rec_units = records ? std::min<uint64_t>(e->rec.cap / 16, 0xFFFFFFF0ull) : 0;
 
   for (int first = 0; first < n_all;) {
@@ -238,6 +226,7 @@ int run_tile_group(Engine* e, const JobSet& js, const PlanGroup& grp, const wfa:
     int64_t ints = 0;
     double rec_plan = 0;
     int n = 0, lw = 0;
+    std::vector<wfa::TileSlot> slots;
     while (first + n < n_all && n < kTileMaxJobs) {
       const int i = grp.ids[first + n];
       const int pitch = wfa::tile_pitch(js.h_plen[i], js.h_tlen[i]);
@@ -246,44 +235,44 @@ int run_tile_group(Engine* e, const JobSet& js, const PlanGroup& grp, const wfa:
       if (n > 0 && ((size_t)(ints + need) * 4 > kTileStateBytes || grp.max_grid == n ||
                     (records && rec_plan + L * L * kTileRecordShareOfL2 > (double)rec_units * 16)))
         break;
-      st_off[i] = ints;
-      st_pitch[i] = pitch;
+      slots.push_back(wfa::TileSlot{ints, i, 0});
       ints += need;
       rec_plan += L * L * kTileRecordShareOfL2;
       lw = std::max(lw, (int)L / 32 + 3);
       ++n;
     }
-    if (!e->ring.ensure((size_t)ints * 4)) {
+    const size_t nn = (size_t)n, up_info = (size_t)max_blocks * sizeof(wfa::TileBlockInfo);
+    const size_t up = up_info + nn * sizeof(wfa::TileSlot);
+    if (!e->ring.ensure((size_t)ints * 4) || !t.d_up.ensure(up) || !t.h_up.ensure(up) ||
+        !t.d_jobs.ensure(nn * sizeof(wfa::TileJob)) || !t.d_marks.ensure(nn * 5 * 4) ||
+        !t.d_job_range.ensure(nn * 4 * sizeof(wfa::TileRange)) || !t.d_dev.ensure(nn * 4 * T * 8) ||
+        !t.d_act.ensure(2 * nn * 4 + 64) || (records && !t.d_tab.ensure(nn * max_blocks * 4))) {
       fprintf(stderr, "[WFA] cannot allocate %zu MB of wavefront rows\n", (size_t)ints >> 18);
       return WF_STATUS_OOM;
     }
+    // block infos and slots go up in one copy
     const int* ids = grp.ids.data() + first;
-    if (!hip_ok(hipMemcpyAsync(t.d_off.p, st_off.data(), (size_t)js.n * 8, hipMemcpyHostToDevice, st), "tiles") ||
-        !hip_ok(hipMemcpyAsync(t.d_pitch.p, st_pitch.data(), (size_t)js.n * 4, hipMemcpyHostToDevice, st), "tiles") ||
-        !hip_ok(hipMemcpyAsync(t.d_jobs.p, ids, (size_t)n * 4, hipMemcpyHostToDevice, st), "tiles"))
-      return WF_STATUS_OOM;
+    memcpy(t.h_up.p, info.data(), up_info);
+    memcpy(t.h_up.as<char>() + up_info, slots.data(), nn * sizeof(wfa::TileSlot));
+    if (!hip_ok(hipMemcpyAsync(t.d_up.p, t.h_up.p, up, hipMemcpyHostToDevice, st), "tiles")) return WF_STATUS_OOM;
     int* marks = t.d_marks.as<int>();
-    int* act[2] = {t.d_act.as<int>() + 16, t.d_act.as<int>() + 16 + n_all};
-    int* n_act = t.d_act.as<int>();  // counts of the two lists
+    int* n_act = t.d_act.as<int>();  // counts of the two lists, and of the jobs lost
+    int* act[2] = {n_act + 16, n_act + 16 + n};
+    int* lost = n_act + 2;
     wfa::TileArgs a{};
     a.act = act[0];
     a.n_act = n_act;
-    a.plen = js.plen;
-    a.tlen = js.tlen;
+    a.jobs = t.d_jobs.as<wfa::TileJob>();
     a.words = js.words;
-    a.pat_pos = js.ppos;
-    a.txt_pos = js.tpos;
     a.state = e->ring.as<int>();
-    a.st_off = t.d_off.as<int64_t>();
-    a.st_pitch = t.d_pitch.as<int>();
     a.done = marks;
-    a.irr = marks + js.n;
+    a.irr = marks + nn;
     a.range = t.d_job_range.as<wfa::TileRange>();
     a.m_range = t.d_range.as<int2>();
-    a.exact_lo = marks + 2 * (size_t)js.n;
-    a.exact_hi = marks + 3 * (size_t)js.n;
-    a.stepped = marks + 4 * (size_t)js.n;
-    for (int x = 0; x < 4; ++x) a.dev[x / 2][x % 2] = t.d_dev.as<long long>() + (size_t)js.n * T * x;
+    a.exact_lo = marks + 2 * nn;
+    a.exact_hi = marks + 3 * nn;
+    a.stepped = marks + 4 * nn;
+    for (int x = 0; x < 4; ++x) a.dev[x / 2][x % 2] = t.d_dev.as<long long>() + nn * T * x;
     a.dsteps_upto = t.d_dsteps.as<long long>();
     a.rec = e->rec.as<uint4>();
     a.rec_tab = t.d_tab.as<uint32_t>();
@@ -291,7 +280,9 @@ int run_tile_group(Engine* e, const JobSet& js, const PlanGroup& grp, const wfa:
     a.lmax_words = lw;
     (void)hipEventRecord(t.ev[0], st);
     if (!hip_ok(wfa::launch_tile_fill(a.state, ints, st), "tile fill") ||
-        !hip_ok(wfa::launch_tile_init(shape, a, n, t.d_jobs.as<int>(), act[0], n_act, st), "tile init"))
+        !hip_ok(wfa::launch_tile_init(shape, a, n, reinterpret_cast<wfa::TileSlot*>(t.d_up.as<char>() + up_info),
+                                      wfa::TileSeqs{js.plen, js.tlen, js.ppos, js.tpos}, act[0], n_act, lost, st),
+                "tile init"))
       return WF_STATUS_OOM;
     int known = n, which = 0, chunk = 0;
     uint64_t unit = 0;
@@ -318,7 +309,7 @@ int run_tile_group(Engine* e, const JobSet& js, const PlanGroup& grp, const wfa:
       // so that the device always has launches queued
       const int slot = chunk & 1;
       if (!hip_ok(wfa::launch_tile_compact(act[which], n_act + which, a.done, a.irr, b * T, act[which ^ 1],
-                                           n_act + (which ^ 1), const_cast<int*>(h_n) + slot, st), "tile compact") ||
+                                           n_act + (which ^ 1), lost, const_cast<int*>(h_n) + slot, st), "tile compact") ||
           !hip_ok(hipEventRecord(t.ev[3 + slot], st), "tile event"))
         return WF_STATUS_OOM;
       which ^= 1;
@@ -334,9 +325,7 @@ int run_tile_group(Engine* e, const JobSet& js, const PlanGroup& grp, const wfa:
     }
     wfa::TileFinishArgs f{};
     f.n = n;
-    f.jobs = t.d_jobs.as<int>();
-    f.plen = js.plen;
-    f.tlen = js.tlen;
+    f.jobs = a.jobs;
     f.done = a.done;
     f.irr = a.irr;
     f.exact_lo = a.exact_lo;
@@ -361,18 +350,14 @@ int run_tile_group(Engine* e, const JobSet& js, const PlanGroup& grp, const wfa:
     (void)hipEventRecord(t.ev[1], st);
     if (records) {
       wfa::TileTraceArgs ta{};
-      ta.jobs = t.d_jobs.as<int>();
-      ta.plen = js.plen;
-      ta.tlen = js.tlen;
+      ta.jobs = a.jobs;
       ta.status = js.status;
       ta.score = js.score;
       ta.rec = a.rec;
       ta.rec_tab = a.rec_tab;
       ta.tab_stride = a.tab_stride;
-      ta.blocks = t.d_info.as<wfa::TileBlockInfo>();
+      ta.blocks = t.d_up.as<wfa::TileBlockInfo>();
       ta.words = js.words;
-      ta.pat_pos = js.ppos;
-      ta.txt_pos = js.tpos;
       ta.ops = js.ops;
       ta.ops_off = js.ops_off;
       ta.ops_begin = js.ops_begin;
