@@ -76,3 +76,40 @@ def test_one_long_pair_among_many_reads(monkeypatch):
         db.free()
         al.close()
     assert used[1] - used[0] < 128e6
+
+
+def check(metric, pen, ps, **kw):
+    al = wfa_amd.Aligner(metric=metric, penalties=pen, **kw)
+    db = al.upload(ps)
+    ref = O.oracle_align(O.Conf(metric, pen, kw.get("memory", "high")), O.Pairs(ps.patterns(), ps.texts()))
+    assert db.run() == 0
+    assert_same(db.download(), ref, range(ps.n))
+    return al, db, ref
+
+
+@pytest.mark.parametrize("metric,pen", [("affine2p", PEN), ("affine", (0, 4, 6, 2))], ids=["affine2p", "affine"])
+def test_little_memory_for_rows(monkeypatch, metric, pen):
+    """1 MB of rows (affine2p takes 0.8 MB for a pair of 1,100 bp, affine 0.15
+    MB): a pass for every pair or few of them, one of 9 kbp and one of 17 kbp
+    that do not fit at all, and pairs that change over to single steps."""
+    monkeypatch.setenv("WFA_ROWS_MB", "1")
+    rng = np.random.default_rng(6)
+    pairs = [pair(rng, n, 0.04) for n in (1100, 1290, 9000, 1150, 1030, 17000, 1200, 1250)]
+    sk = datagen.skewed(8, 2, tlen=(300, 600), insert=(900, 1100))
+    ps = datagen.PairSet.from_lists([p for p, _ in pairs] + sk.patterns(), [t for _, t in pairs] + sk.texts())
+    al, db, ref = check(metric, pen, ps)
+    assert db.stats().diagonal_steps == int(ref.dsteps.sum())
+    say("%s: %d launches" % (metric, db.stats().forward_launches))
+    assert db.stats().forward_launches >= 4
+    assert db.run() == 0  # the statuses of the first run are there now
+    assert_same(db.download(), ref, range(ps.n))
+
+
+def test_little_memory_for_biwfa_rows(monkeypatch):
+    """1 MB of rows: sub-problems of up to 1,700 symbols a side in tiles, a
+    few at a time, larger ones without."""
+    monkeypatch.setenv("WFA_ROWS_MB", "1")
+    rng = np.random.default_rng(7)
+    pairs = [pair(rng, n, 0.06) for n in (1100, 6000, 700, 2500, 1300, 900)]
+    check("affine", (0, 4, 6, 2), datagen.PairSet.from_lists([p for p, _ in pairs], [t for _, t in pairs]),
+          memory="ultralow")

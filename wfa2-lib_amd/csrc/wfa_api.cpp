@@ -246,6 +246,10 @@ bool engine_init(Engine* e) {
   if (env) cap = std::min<size_t>(strtoull(env, nullptr, 10) << 20, kMaxArenaBytes);
   if (e->rec_cap) cap = std::min(cap, e->rec_cap);  // a cap set before the first run
   e->rec_cap = std::max<size_t>(cap, 64ull << 20);
+  // Wavefront rows of the tiles, per buffer: WFA_ROWS_MB bounds them.
+  const char* rows = getenv("WFA_ROWS_MB");
+  const size_t rows_cap = rows ? strtoull(rows, nullptr, 10) << 20 : 0;
+  if (rows_cap) e->rows_cap = e->rows_cap ? std::min(e->rows_cap, rows_cap) : rows_cap;
   // The arena starts at 64 MB; each run grows it to its pairs' estimate.
   e->rec_bytes = std::min<size_t>(64ull << 20, e->rec_cap);
   e->ok = true;
@@ -1149,8 +1153,9 @@ int run_jobs(wavefront_aligner_t* wf, Engine* e, const JobSet& js, std::vector<P
     // the reset before the first round clears every counter
     if (round > 0 && !hip_ok(wfa::launch_reset_counters(counters_of(e), 1, st), "reset")) return WF_STATUS_OOM;
     bool fresh = true;
+    std::vector<int> ring_ids;  // jobs whose rows do not fit the tiles' memory
     for (PlanGroup& g : *pending) {
-      const int rc = g.family == wfa::kTile ? run_tile_group(e, js, g, pen, records, tot)
+      const int rc = g.family == wfa::kTile ? run_tile_group(e, js, g, pen, records, tot, &ring_ids)
                                             : enqueue_group(wf, e, js, g, pen, records, fresh);
       if (rc != WF_STATUS_OK) return rc;
       if (!g.ids.empty()) fresh = false;
@@ -1168,7 +1173,7 @@ int run_jobs(wavefront_aligner_t* wf, Engine* e, const JobSet& js, std::vector<P
       tot->forward_ms += f;
       tot->backtrace_ms += t;
     }
-    if (host_c.retry == 0) break;
+    if (host_c.retry == 0 && ring_ids.empty()) break;
     // Some jobs overflowed the LDS ring or the record arena: re-run only them.
     h_status.resize(js.n);
     // copies on the aligner's stream, never the null stream (which would wait
@@ -1176,6 +1181,7 @@ int run_jobs(wavefront_aligner_t* wf, Engine* e, const JobSet& js, std::vector<P
     if (!hip_ok(hipMemcpyAsync(h_status.data(), js.status, (size_t)js.n * 4, hipMemcpyDeviceToHost, st), "status") ||
         !hip_ok(hipStreamSynchronize(st), "status"))
       return WF_STATUS_OOM;
+    for (int i : ring_ids) h_status[i] = wfa::kDevCompleted;  // (not run yet: what is there is an earlier run's)
     std::vector<PlanGroup> next;
     for (PlanGroup& g : *pending) {
       std::vector<int> ring_over, arena_full;
@@ -1255,6 +1261,7 @@ int run_jobs(wavefront_aligner_t* wf, Engine* e, const JobSet& js, std::vector<P
         }
       }
     }
+    if (!ring_ids.empty()) next.push_back(make_large(e, js, std::move(ring_ids)));
     give_back_groups(e, retry_groups);
     retry_groups = std::move(next);
     pending = &retry_groups;

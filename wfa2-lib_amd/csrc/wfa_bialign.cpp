@@ -185,8 +185,8 @@ bool bi_table(Engine* e, int steps) {
 
 // Advances the sub-problems probs[0..n) (already in d_probs) in tiles until
 // the block in which phase 1 ends, and sets a's resume fields; without memory
-// for their rows the search runs from the start.
-bool bi_fast_forward(Engine* e, const std::vector<wfa::BiProblem>& probs, wfa::BiArgs& a) {
+// for their rows (which grow up to max_bytes) the search runs from the start.
+bool bi_fast_forward(Engine* e, const std::vector<wfa::BiProblem>& probs, size_t max_bytes, wfa::BiArgs& a) {
   Engine::BiTiles& t = e->bi_tiles;
   const int n = (int)probs.size(), T = wfa::bi_tile_steps(), U = wfa::bi_tile_useful();
   hipStream_t st = e->stream;
@@ -206,7 +206,7 @@ bool bi_fast_forward(Engine* e, const std::vector<wfa::BiProblem>& probs, wfa::B
   }
   const int max_blocks = max_steps / T + 2;  // (a search not done by then starts over: wfa_breakpoint_kernel)
   if (!bi_table(e, (max_blocks + 1) * T)) return false;
-  if (!t.h_n.ensure(4096) || !t.d_state.ensure((size_t)ints * 4) || !t.d_off.ensure((size_t)n * 8) ||
+  if (!t.h_n.ensure(4096) || !t.d_state.ensure((size_t)ints * 4, std::max(max_bytes, (size_t)ints * 4)) || !t.d_off.ensure((size_t)n * 8) ||
       !t.d_marks.ensure((size_t)n * 5 * 4) || !t.d_act.ensure((size_t)2 * n * 4 + 64))
     return true;
   for (auto& ev : t.ev)
@@ -291,19 +291,28 @@ bool run_breakpoints(wavefront_aligner_t* wf, Engine* e, wfa_device_batch_t* b, 
   // large sub-problems in tiles: as many at once as their rows' memory allows
   std::vector<std::vector<int>> runs(groups, groups + 3);
   std::vector<int> run_block = {64, 256, 1024};
+  size_t rows_bytes = kBiTileStateBytes;
   if (tiles_ok) {
+    auto rows_of = [&](int i) {
+      const wfa::BiProblem& p = nodes[i].prob;
+      return (size_t)2 * wfa::kBiTileRows * wfa::tile_pitch(p.pe - p.pb, p.te - p.tb) * 4;
+    };
+    size_t want = 0;
+    for (size_t i = 0; i < nodes.size(); ++i) want += rows_of((int)i);
+    rows_bytes = rows_limit(e, want, kBiTileStateBytes, e->bi_tiles.d_state.cap);
     for (int gi = 0; gi < 3; ++gi) {
       int64_t bytes = INT64_MAX;
       std::vector<int> rest;
       for (int i : groups[gi]) {
         const wfa::BiProblem& p = nodes[i].prob;
         const int pl = p.pe - p.pb, tl = p.te - p.tb;
-        if (pl + tl < kBiTileMinSize || 2 * (size_t)(std::max(pl, tl) / 32 + 4) * 8 > wfa::kTileSeqLdsBytes) {
+        const int64_t need = (int64_t)rows_of(i);
+        if (pl + tl < kBiTileMinSize || 2 * (size_t)(std::max(pl, tl) / 32 + 4) * 8 > wfa::kTileSeqLdsBytes ||
+            (e->rows_cap && (size_t)need > e->rows_cap)) {
           rest.push_back(i);
           continue;
         }
-        const int64_t need = (int64_t)2 * wfa::kBiTileRows * wfa::tile_pitch(pl, tl) * 4;
-        if (bytes > (int64_t)kBiTileStateBytes - need || runs.back().size() >= kBiTileMaxProblems) {
+        if (bytes > (int64_t)rows_bytes - need || runs.back().size() >= kBiTileMaxProblems) {
           runs.emplace_back();
           run_block.push_back(run_block[gi]);
           bytes = 0;
@@ -398,7 +407,7 @@ bool run_breakpoints(wavefront_aligner_t* wf, Engine* e, wfa_device_batch_t* b, 
                 (!paired || hip_ok(hipMemsetAsync(a.mail, 0, probs.size() * 4 * sizeof(unsigned long long), st),
                                    "mailboxes"));
       (void)hipEventRecord(e0, st);
-      if (ok && tile && !bi_fast_forward(e, probs, a)) return false;
+      if (ok && tile && !bi_fast_forward(e, probs, rows_bytes, a)) return false;
       ok = ok && hip_ok(paired ? wfa::launch_breakpoint_pair(a, ncomp, b->bits, block, st)
                                : wfa::launch_breakpoint(a, ncomp, b->bits, block, grid, st),
                         "breakpoint launch");

@@ -125,6 +125,7 @@ struct Engine {
   DevBuf over;  // ids of a group's pairs that outgrow its first kernel
   size_t rec_bytes = 0;     // record arena size for the next run (grows on demand)
   size_t rec_cap = 0;       // largest record arena this engine may allocate
+  size_t rows_cap = 0;      // most bytes of wavefront rows per buffer of the tiles (0: what is free decides)
   bool ok = false;
   // Stream on a hardware queue of its own: HIP spreads ordinary streams over a
   // few shared queues, on which kernels of different streams run in order;
@@ -151,7 +152,7 @@ struct Engine {
   struct TileState {
     int shape = 0;
     std::vector<int> lo, hi;          // hull of the ranges up to each step
-    DevBuf d_range, d_dsteps, d_job_range, d_dev, d_ends, d_flags, d_dsum, d_step_state, d_step_off, d_step0, d_step_act, d_up, d_jobs, d_marks, d_act, d_tab;
+    DevBuf d_state, d_range, d_dsteps, d_job_range, d_dev, d_ends, d_flags, d_dsum, d_step_state, d_step_off, d_step0, d_step_act, d_up, d_jobs, d_marks, d_act, d_tab;
     HostBuf h_n;                      // jobs left, written by the device
     HostBuf h_up;                     // what goes up for a pass
     hipEvent_t ev[5] = {nullptr, nullptr, nullptr, nullptr, nullptr};
@@ -272,8 +273,13 @@ int run_jobs(wavefront_aligner_t* wf, Engine* e, const JobSet& js, std::vector<P
 // Long pairs in tiles (wfa_tile_run.cpp).
 bool tile_table(Engine* e, int shape, int steps);
 bool tile_fits(int plen, int tlen);
+// Bytes of wavefront rows to take at once of the `want` that all jobs together
+// need: no more than `most` and the engine's cap, and where the buffer (`held`
+// bytes) would have to grow, a quarter of the memory that is free.
+size_t rows_limit(const Engine* e, size_t want, size_t most, size_t held);
+// Jobs whose rows do not fit are left to the HBM-ring family (`ring`).
 int run_tile_group(Engine* e, const JobSet& js, const PlanGroup& grp, const wfa::Penalties& pen, int records,
-                   RunTotals* tot);
+                   RunTotals* tot, std::vector<int>* ring);
 
 }  // namespace wfa_host
 

@@ -11,8 +11,7 @@
 namespace wfa_host {
 namespace {
 
-// State rows of the jobs that run at once.  All other buffers of a pass are
-// per job of the pass too (wfa::TileJob).
+// Buffers of the jobs that run at once (wfa::TileJob), at most.
 constexpr size_t kTileStateBytes = size_t(24) << 30;
 constexpr int kTileMaxJobs = 32768;  // grid y
 // Records a long pair is planned with: 1-20 kbp pairs of 1-15% error write
@@ -68,6 +67,15 @@ bool tile_table(Engine* e, int shape, int steps) {
   return true;
 }
 
+size_t rows_limit(const Engine* e, size_t want, size_t most, size_t held) {
+  if (e->rows_cap) most = std::min(most, e->rows_cap);
+  if (std::min(want, most) <= held) return most;
+  // (two such buffers, and room for other aligners)
+  size_t free_b = 0, total_b = 0;
+  if (hipMemGetInfo(&free_b, &total_b) != hipSuccess) return most;
+  return std::min(most, std::max(held, (held + free_b) / 4));
+}
+
 // Whether a job of these lengths can run in tiles: its sequences in LDS.
 bool tile_fits(int plen, int tlen) {
   const int lw = std::max(plen, tlen) / 32 + 3;
@@ -77,10 +85,11 @@ bool tile_fits(int plen, int tlen) {
 // The jobs whose ends moved past their end tiles, one step per launch from
 // the start of the block that found it, all of them side by side.  `unit`:
 // record units taken so far.  Jobs left when the records run out stay
-// unfinished (they are re-run with the records free again).  Jobs are slots of
-// the pass, `ids` their pairs.
+// unfinished (they are re-run with the records free again), and so do jobs
+// whose rows do not fit (they go to the HBM-ring family).  Jobs are slots of
+// the pass.
 int run_steps(Engine* e, const JobSet& js, int shape, const wfa::TileGeometry& g, const wfa::TileArgs& a,
-              const int* ids, int n_pass, const std::vector<wfa::TileBlockInfo>& info, int records,
+              const std::vector<wfa::TileSlot>& slots, int n_pass, const std::vector<wfa::TileBlockInfo>& info, int records,
               uint64_t rec_units, uint64_t* unit) {
   Engine::TileState& t = e->tile;
   hipStream_t st = e->stream;
@@ -98,26 +107,34 @@ int run_steps(Engine* e, const JobSet& js, int shape, const wfa::TileGeometry& g
                                    t.d_flags.ensure((size_t)n_pass * wfa::kTileStepFlags * 4) &&
                                    t.d_dsum.ensure((size_t)n_pass * 8) && t.d_step0.ensure((size_t)n_pass * 4) &&
                                    t.d_step_off.ensure((size_t)n_pass * 8));
-  if (!ok) return WF_STATUS_OOM;
+  if (!ok) return WF_STATUS_OK;
+  auto rows_of = [&](int x) {
+    return (size_t)wfa::tile_pitch(js.h_plen[slots[x].id], js.h_tlen[slots[x].id]) * g.step_rows * 4;
+  };
+  size_t want = 0;
+  for (int x : jobs) want += rows_of(x);
+  size_t limit = rows_limit(e, want, kTileStateBytes, t.d_step_state.cap);
   // as many at once as their rows' memory allows
   for (size_t first = 0; first < jobs.size();) {
     std::vector<int64_t> off(n_pass, 0);
     int64_t ints = 0;
     int n = 0, max_pitch = 0, max_width = 0;
     while (first + n < jobs.size()) {
-      const int x = jobs[first + n], i = ids[x], pitch = wfa::tile_pitch(js.h_plen[i], js.h_tlen[i]);
-      const int64_t need = (int64_t)pitch * g.step_rows;
-      if (n > 0 && (size_t)(ints + need) * 4 > kTileStateBytes) break;
+      const int x = jobs[first + n], i = slots[x].id;
+      const size_t need = rows_of(x);
+      if (n > 0 && (size_t)ints * 4 + need > limit) break;
       off[x] = ints;
-      ints += need;
-      max_pitch = std::max(max_pitch, pitch);
+      ints += need / 4;
+      max_pitch = std::max(max_pitch, wfa::tile_pitch(js.h_plen[i], js.h_tlen[i]));
       max_width = std::max(max_width, js.h_plen[i] + js.h_tlen[i] + 4);
       ++n;
     }
     const int* sel = jobs.data() + first;
-    if (!t.d_step_state.ensure((size_t)ints * 4) || !t.d_step_act.ensure((size_t)2 * n * 4 + 64)) {
-      fprintf(stderr, "[WFA] cannot allocate %zu MB of wavefront rows\n", (size_t)ints >> 18);
-      return WF_STATUS_OOM;
+    if (!t.d_step_state.ensure((size_t)ints * 4, std::max(limit, (size_t)ints * 4)) ||
+        !t.d_step_act.ensure((size_t)2 * n * 4 + 64)) {
+      limit = (size_t)ints * 2;  // fewer at once, or without this one
+      if (n == 1) ++first;
+      continue;
     }
     int* n_act = t.d_step_act.as<int>();
     int* act[2] = {n_act + 16, n_act + 16 + n};
@@ -185,7 +202,7 @@ int run_steps(Engine* e, const JobSet& js, int shape, const wfa::TileGeometry& g
 // Aligns the jobs of a tile group; statuses, scores and CIGARs stay on the
 // device, and jobs to be re-run are counted in the run counters.
 int run_tile_group(Engine* e, const JobSet& js, const PlanGroup& grp, const wfa::Penalties& pen, int records,
-                   RunTotals* tot) {
+                   RunTotals* tot, std::vector<int>* ring) {
   Engine::TileState& t = e->tile;
   const int shape = wfa::tile_shape(pen);
   const wfa::TileGeometry g = wfa::tile_geometry(shape);
@@ -221,37 +238,58 @@ int run_tile_group(Engine* e, const JobSet& js, const PlanGroup& grp, const wfa:
   const int n_all = (int)grp.ids.size();
   const uint64_t rec_units = records ? std::min<uint64_t>(e->rec.cap / 16, 0xFFFFFFF0ull) : 0;
 
+  // device bytes of a job: its rows, its blocks' records, and what the kernels keep of it
+  auto rows_of = [&](int i) { return (size_t)wfa::tile_pitch(js.h_plen[i], js.h_tlen[i]) * g.state_rows * 4; };
+  const size_t tab_bytes = (records ? (size_t)max_blocks * 4 : 0) + (size_t)4 * T * 8 + sizeof(wfa::TileJob) +
+                           sizeof(wfa::TileSlot) + 4 * sizeof(wfa::TileRange) + 7 * 4;
+  size_t want = 0;
+  for (int i : grp.ids) want += rows_of(i) + tab_bytes;
+  size_t limit = rows_limit(e, want, kTileStateBytes, t.d_state.cap);
+  bool some = false;  // a pass has run
+
   for (int first = 0; first < n_all;) {
-    // the jobs of one pass: their state rows and planned records fit
+    // the jobs of one pass: their buffers and planned records fit
+    size_t bytes = 0;
     int64_t ints = 0;
     double rec_plan = 0;
-    int n = 0, lw = 0;
+    int n = 0, lw = 0, taken = 0;
     std::vector<wfa::TileSlot> slots;
-    while (first + n < n_all && n < kTileMaxJobs) {
-      const int i = grp.ids[first + n];
-      const int pitch = wfa::tile_pitch(js.h_plen[i], js.h_tlen[i]);
-      const int64_t need = (int64_t)pitch * g.state_rows;
+    for (; first + taken < n_all && n < kTileMaxJobs; ++taken) {
+      const int i = grp.ids[first + taken];
+      const size_t need = rows_of(i) + tab_bytes;
       const double L = std::max(js.h_plen[i], js.h_tlen[i]);
-      if (n > 0 && ((size_t)(ints + need) * 4 > kTileStateBytes || grp.max_grid == n ||
+      if (e->rows_cap && need > e->rows_cap) {
+        ring->push_back(i);
+        continue;
+      }
+      if (n > 0 && (bytes + need > limit || grp.max_grid == n ||
                     (records && rec_plan + L * L * kTileRecordShareOfL2 > (double)rec_units * 16)))
         break;
       slots.push_back(wfa::TileSlot{ints, i, 0});
-      ints += need;
+      bytes += need;
+      ints += (int64_t)(rows_of(i) / 4);
       rec_plan += L * L * kTileRecordShareOfL2;
       lw = std::max(lw, (int)L / 32 + 3);
       ++n;
     }
+    if (n == 0) break;
     const size_t nn = (size_t)n, up_info = (size_t)max_blocks * sizeof(wfa::TileBlockInfo);
     const size_t up = up_info + nn * sizeof(wfa::TileSlot);
-    if (!e->ring.ensure((size_t)ints * 4) || !t.d_up.ensure(up) || !t.h_up.ensure(up) ||
-        !t.d_jobs.ensure(nn * sizeof(wfa::TileJob)) || !t.d_marks.ensure(nn * 5 * 4) ||
+    if (!t.d_state.ensure((size_t)ints * 4, std::max(limit, (size_t)ints * 4)) || !t.d_up.ensure(up) ||
+        !t.h_up.ensure(up) || !t.d_jobs.ensure(nn * sizeof(wfa::TileJob)) || !t.d_marks.ensure(nn * 5 * 4) ||
         !t.d_job_range.ensure(nn * 4 * sizeof(wfa::TileRange)) || !t.d_dev.ensure(nn * 4 * T * 8) ||
         !t.d_act.ensure(2 * nn * 4 + 64) || (records && !t.d_tab.ensure(nn * max_blocks * 4))) {
-      fprintf(stderr, "[WFA] cannot allocate %zu MB of wavefront rows\n", (size_t)ints >> 18);
-      return WF_STATUS_OOM;
+      // fewer at once, or without this one
+      limit = bytes / 2;
+      if (n == 1) {
+        ring->push_back(slots[0].id);
+        first += taken;
+      } else {
+        ring->resize(ring->size() - (size_t)(taken - n));
+      }
+      continue;
     }
     // block infos and slots go up in one copy
-    const int* ids = grp.ids.data() + first;
     memcpy(t.h_up.p, info.data(), up_info);
     memcpy(t.h_up.as<char>() + up_info, slots.data(), nn * sizeof(wfa::TileSlot));
     if (!hip_ok(hipMemcpyAsync(t.d_up.p, t.h_up.p, up, hipMemcpyHostToDevice, st), "tiles")) return WF_STATUS_OOM;
@@ -264,7 +302,7 @@ int run_tile_group(Engine* e, const JobSet& js, const PlanGroup& grp, const wfa:
     a.n_act = n_act;
     a.jobs = t.d_jobs.as<wfa::TileJob>();
     a.words = js.words;
-    a.state = e->ring.as<int>();
+    a.state = t.d_state.as<int>();
     a.done = marks;
     a.irr = marks + nn;
     a.range = t.d_job_range.as<wfa::TileRange>();
@@ -320,7 +358,7 @@ int run_tile_group(Engine* e, const JobSet& js, const PlanGroup& grp, const wfa:
       ++chunk;
     }
     if (!full) {
-      const int rc = run_steps(e, js, shape, g, a, ids, n, info, records, rec_units, &unit);
+      const int rc = run_steps(e, js, shape, g, a, slots, n, info, records, rec_units, &unit);
       if (rc != WF_STATUS_OK) return rc;
     }
     wfa::TileFinishArgs f{};
@@ -373,8 +411,9 @@ int run_tile_group(Engine* e, const JobSet& js, const PlanGroup& grp, const wfa:
     (void)hipEventElapsedTime(&bms, t.ev[1], t.ev[2]);
     tot->forward_ms += fms;
     tot->backtrace_ms += bms;
-    if (first > 0) ++tot->launches;  // a further pass (the caller counts one)
-    first += n;
+    if (some) ++tot->launches;  // a further pass (the caller counts one)
+    some = true;
+    first += taken;
   }
   return WF_STATUS_OK;
 }
