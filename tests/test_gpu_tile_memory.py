@@ -113,3 +113,30 @@ def test_little_memory_for_biwfa_rows(monkeypatch):
     pairs = [pair(rng, n, 0.06) for n in (1100, 6000, 700, 2500, 1300, 900)]
     check("affine", (0, 4, 6, 2), datagen.PairSet.from_lists([p for p, _ in pairs], [t for _, t in pairs]),
           memory="ultralow")
+
+
+def test_reap_gives_the_rows_back():
+    """wavefront_aligner_reap frees what the tiles hold; the aligner goes on."""
+    rng = np.random.default_rng(9)
+    pairs = [pair(rng, 5000, 0.02) for _ in range(40)]
+    ps = datagen.PairSet.from_lists([p for p, _ in pairs], [t for _, t in pairs])
+    L = wfa_amd.lib()
+    for memory in ("high", "ultralow"):
+        metric, pen = ("affine2p", PEN) if memory == "high" else ("affine", (0, 4, 6, 2))
+        al = wfa_amd.Aligner(metric=metric, penalties=pen, memory=memory)
+        al.upload(ps).free()
+        held = free_device_bytes()
+        results = []
+        for _ in range(2):
+            db = al.upload(ps)
+            assert db.run() == 0
+            results.append(db.download())
+            db.free()
+            taken = held - free_device_bytes()
+            L.wavefront_aligner_reap(al.wf)
+            left = held - free_device_bytes()
+            say("%s: %.0f MB held by a run, %.0f MB after" % (memory, taken / 1e6, left / 1e6))
+            assert taken > 64e6 and left < 32e6
+        want, got = results
+        assert np.array_equal(got.score, want.score)
+        assert all(got.ops(i) == want.ops(i) for i in range(ps.n))

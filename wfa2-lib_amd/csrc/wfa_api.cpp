@@ -202,6 +202,18 @@ Engine::~Engine() {
     if (ev) (void)hipEventDestroy(ev);
 }
 
+void Engine::TileState::release() {
+  for (DevBuf* x : {&d_state, &d_range, &d_dsteps, &d_job_range, &d_dev, &d_ends, &d_flags, &d_dsum, &d_step_state,
+                    &d_step_off, &d_step0, &d_step_act, &d_up, &d_jobs, &d_marks, &d_act, &d_tab})
+    x->release();
+  shape = 0;  // the table goes up again
+}
+
+void Engine::BiTiles::release() {
+  for (DevBuf* x : {&d_hull, &d_dsteps, &d_state, &d_off, &d_marks, &d_act}) x->release();
+  steps = 0;
+}
+
 Engine* engine_of(wavefront_aligner_t* wf) { return static_cast<Engine*>(wf->device); }
 wfa::Counters* counters_of(Engine* e) { return e->counters.as<wfa::Counters>(); }
 
@@ -1399,6 +1411,9 @@ extern "C" void wavefront_aligner_reap(wavefront_aligner_t* const wf) {
   e->scratch = nullptr;
   e->rec.release();
   e->ring.release();
+  e->over.release();
+  e->tile.release();
+  e->bi_tiles.release();
 }
 
 extern "C" void wavefront_aligner_delete(wavefront_aligner_t* const wf) {

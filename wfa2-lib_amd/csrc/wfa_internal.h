@@ -155,6 +155,7 @@ struct Engine {
     DevBuf d_state, d_range, d_dsteps, d_job_range, d_dev, d_ends, d_flags, d_dsum, d_step_state, d_step_off, d_step0, d_step_act, d_up, d_jobs, d_marks, d_act, d_tab;
     HostBuf h_n;                      // jobs left, written by the device
     HostBuf h_up;                     // what goes up for a pass
+    void release();                   // (device buffers)
     hipEvent_t ev[5] = {nullptr, nullptr, nullptr, nullptr, nullptr};
   } tile;
   // BiWFA sub-problems in tiles (wfa_bialign.cpp): range tables and buffers.
@@ -163,6 +164,7 @@ struct Engine {
     std::vector<int> lo, hi;
     DevBuf d_hull, d_dsteps, d_state, d_off, d_marks, d_act;
     HostBuf h_n;
+    void release();  // (device buffers)
     hipEvent_t ev[2] = {nullptr, nullptr};
   } bi_tiles;
   // Set for the duration of a no-allocation run: plan groups take their
