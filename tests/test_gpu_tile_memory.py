@@ -140,3 +140,31 @@ def test_reap_gives_the_rows_back():
         want, got = results
         assert np.array_equal(got.score, want.score)
         assert all(got.ops(i) == want.ops(i) for i in range(ps.n))
+
+
+def test_a_lane_keeps_to_its_memory():
+    """128 requests of 12 kbp, scores only, in a lane of 256 MB: 6 MB of rows
+    each, nearly all of them admitted at once under an error prior of 0.2%.
+    The lane may take its 64 MB arena, 128 MB of rows, what the rows outgrew
+    (kept while the server runs: about their size again), and its sequences."""
+    rng = np.random.default_rng(10)
+    pairs = [pair(rng, 12000, 0.002) for _ in range(128)]
+    ref = O.oracle_align(O.Conf("affine2p", PEN, "high", True), O.Pairs([p for p, _ in pairs], [t for _, t in pairs]))
+    before = free_device_bytes()
+    srv = wfa_amd.Server(metric="affine2p", penalties=PEN, medium_lanes=1, lane_memory_bytes=256 << 20,
+                         error_prior=0.002)
+    wfa_amd.lib().wfa_server_destroy(srv.h)
+    srv.attr.alignment_scope = 0
+    srv.h = wfa_amd.lib().wfa_server_create(ctypes.byref(srv.attr), ctypes.byref(srv.config))
+    ids = [srv.submit(p, t) for p, t in pairs]
+    got, t0 = {}, srv.clock()
+    while len(got) < len(ids):
+        for r in srv.collect(max_results=256, timeout_ms=200):
+            got[r.id] = r
+        assert srv.clock() - t0 < 60, "requests did not finish"
+    taken = before - free_device_bytes()
+    srv.close()
+    say("%.0f MB taken" % (taken / 1e6))
+    for x, i in enumerate(ids):
+        assert (got[i].status, got[i].score) == (ref.status[x], ref.score[x]), x
+    assert taken < (64 + 2 * 128 + 64) * 1.05e6

@@ -125,12 +125,14 @@ void wfa_server_t::lane_main(int cls) {
     ++lane_errors;
     return;
   }
-  // The lane's record arena is its memory budget.  Each lane has a hardware
+  // The lane's record arena is its memory budget, and half of it again bounds
+  // each buffer of wavefront rows (tiles, single steps, BiWFA).  Each lane has a hardware
   // queue of its own: on a shared queue, one lane's kernels (seconds for a
   // long batch, hundreds of milliseconds for a medium one) would hold up the
   // batches of the others (streams sharing a queue run in order).
   if (wfa_host::Engine* e = wfa_host::engine_of(wf)) {
     e->rec_cap = cfg.lane_memory_bytes;
+    e->rows_cap = std::max<size_t>(cfg.lane_memory_bytes / 2, 1);
     e->own_queue = true;
     // CUs from the top: short | medium | long
     const double s = cfg.short_cu_share, m = cfg.medium_cu_share, l = cfg.long_cu_share;
