@@ -156,7 +156,7 @@ struct Engine {
     HostBuf h_n;                      // jobs left, written by the device
     HostBuf h_up;                     // what goes up for a pass
     void release();                   // (device buffers)
-    hipEvent_t ev[5] = {nullptr, nullptr, nullptr, nullptr, nullptr};
+    hipEvent_t ev[3] = {nullptr, nullptr, nullptr};  // two looks at the jobs left; the upload
   } tile;
   // BiWFA sub-problems in tiles (wfa_bialign.cpp): range tables and buffers.
   struct BiTiles {
@@ -280,7 +280,7 @@ bool tile_fits(int plen, int tlen);
 // bytes) would have to grow, a quarter of the memory that is free.
 size_t rows_limit(const Engine* e, size_t want, size_t most, size_t held);
 // Jobs whose rows do not fit are left to the HBM-ring family (`ring`).
-int run_tile_group(Engine* e, const JobSet& js, const PlanGroup& grp, const wfa::Penalties& pen, int records,
+int run_tile_group(Engine* e, const JobSet& js, PlanGroup& grp, const wfa::Penalties& pen, int records,
                    RunTotals* tot, std::vector<int>* ring);
 
 }  // namespace wfa_host

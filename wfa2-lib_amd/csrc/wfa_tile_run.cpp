@@ -17,8 +17,8 @@ constexpr int kTileMaxJobs = 32768;  // grid y
 // Records a long pair is planned with: 1-20 kbp pairs of 1-15% error write
 // 0.25 L^2 bytes on average and up to 0.7 L^2.
 constexpr double kTileRecordShareOfL2 = 0.5;
-// Blocks between two looks at the number of jobs left.
-constexpr int kTileFirstChunk = 4, kTileChunk = 16;
+// Blocks between two looks at the number of jobs left: 1, 2, 4, 4, then 16.
+constexpr int kTileChunk = 16;
 
 bool put(DevBuf& d, const void* from, size_t bytes, hipStream_t st) {
   return d.ensure(bytes) && hip_ok(hipMemcpyAsync(d.p, from, bytes, hipMemcpyHostToDevice, st), "range table") &&
@@ -185,11 +185,11 @@ int run_steps(Engine* e, const JobSet& js, int shape, const wfa::TileGeometry& g
       if (!hip_ok(wfa::launch_tile_compact(act[which], n_act + which, a.done, nullptr, INT_MAX, act[which ^ 1],
                                            n_act + (which ^ 1), nullptr, const_cast<int*>(h_n) + slot, st),
                   "tile compact") ||
-          !hip_ok(hipEventRecord(t.ev[3 + slot], st), "tile event"))
+          !hip_ok(hipEventRecord(t.ev[slot], st), "tile event"))
         return WF_STATUS_OOM;
       which ^= 1;
       if (b > 0) {
-        if (!hip_ok(hipEventSynchronize(t.ev[3 + (slot ^ 1)]), "steps")) return WF_STATUS_OOM;
+        if (!hip_ok(hipEventSynchronize(t.ev[slot ^ 1]), "steps")) return WF_STATUS_OOM;
         known = h_n[slot ^ 1];
       }
     }
@@ -200,8 +200,10 @@ int run_steps(Engine* e, const JobSet& js, int shape, const wfa::TileGeometry& g
 }
 
 // Aligns the jobs of a tile group; statuses, scores and CIGARs stay on the
-// device, and jobs to be re-run are counted in the run counters.
-int run_tile_group(Engine* e, const JobSet& js, const PlanGroup& grp, const wfa::Penalties& pen, int records,
+// device, and jobs to be re-run are counted in the run counters.  The last
+// pass is only queued, with the group's events around its kernels (a single
+// pair of 1,100 bp at 0.5% errors spent more time on waits than on kernels).
+int run_tile_group(Engine* e, const JobSet& js, PlanGroup& grp, const wfa::Penalties& pen, int records,
                    RunTotals* tot, std::vector<int>* ring) {
   Engine::TileState& t = e->tile;
   const int shape = wfa::tile_shape(pen);
@@ -219,6 +221,8 @@ int run_tile_group(Engine* e, const JobSet& js, const PlanGroup& grp, const wfa:
   const int max_blocks = max_steps / T + 2;
   if (!tile_table(e, shape, (max_blocks + 1) * T)) return WF_STATUS_OOM;
   for (auto& ev : t.ev)
+    if (!ev && !hip_ok(hipEventCreateWithFlags(&ev, hipEventDisableTiming), "hipEventCreate")) return WF_STATUS_OOM;
+  for (auto& ev : grp.ev)
     if (!ev && !hip_ok(hipEventCreate(&ev), "hipEventCreate")) return WF_STATUS_OOM;
   if (!t.h_n.ensure(4096)) return WF_STATUS_OOM;
   volatile int* h_n = t.h_n.as<int>();
@@ -243,9 +247,9 @@ int run_tile_group(Engine* e, const JobSet& js, const PlanGroup& grp, const wfa:
   const size_t tab_bytes = (records ? (size_t)max_blocks * 4 : 0) + (size_t)4 * T * 8 + sizeof(wfa::TileJob) +
                            sizeof(wfa::TileSlot) + 4 * sizeof(wfa::TileRange) + 7 * 4;
   size_t want = 0;
-  for (int i : grp.ids) want += rows_of(i) + tab_bytes;
+  for (int i : grp.ids) want += rows_of(i);
   size_t limit = rows_limit(e, want, kTileStateBytes, t.d_state.cap);
-  bool some = false;  // a pass has run
+  bool some = false, timed = false;  // a pass has run; the group's events are its own
 
   for (int first = 0; first < n_all;) {
     // the jobs of one pass: their buffers and planned records fit
@@ -289,10 +293,13 @@ int run_tile_group(Engine* e, const JobSet& js, const PlanGroup& grp, const wfa:
       }
       continue;
     }
-    // block infos and slots go up in one copy
+    // block infos and slots go up in one copy (once the one before is through)
+    (void)hipEventSynchronize(t.ev[2]);
     memcpy(t.h_up.p, info.data(), up_info);
     memcpy(t.h_up.as<char>() + up_info, slots.data(), nn * sizeof(wfa::TileSlot));
-    if (!hip_ok(hipMemcpyAsync(t.d_up.p, t.h_up.p, up, hipMemcpyHostToDevice, st), "tiles")) return WF_STATUS_OOM;
+    if (!hip_ok(hipMemcpyAsync(t.d_up.p, t.h_up.p, up, hipMemcpyHostToDevice, st), "tiles") ||
+        !hip_ok(hipEventRecord(t.ev[2], st), "tile event"))
+      return WF_STATUS_OOM;
     int* marks = t.d_marks.as<int>();
     int* n_act = t.d_act.as<int>();  // counts of the two lists, and of the jobs lost
     int* act[2] = {n_act + 16, n_act + 16 + n};
@@ -316,17 +323,17 @@ int run_tile_group(Engine* e, const JobSet& js, const PlanGroup& grp, const wfa:
     a.rec_tab = t.d_tab.as<uint32_t>();
     a.tab_stride = max_blocks;
     a.lmax_words = lw;
-    (void)hipEventRecord(t.ev[0], st);
+    (void)hipEventRecord(grp.ev[0], st);
     if (!hip_ok(wfa::launch_tile_fill(a.state, ints, st), "tile fill") ||
         !hip_ok(wfa::launch_tile_init(shape, a, n, reinterpret_cast<wfa::TileSlot*>(t.d_up.as<char>() + up_info),
                                       wfa::TileSeqs{js.plen, js.tlen, js.ppos, js.tpos}, act[0], n_act, lost, st),
                 "tile init"))
       return WF_STATUS_OOM;
-    int known = n, which = 0, chunk = 0;
+    int known = n, jobs_lost = 0, which = 0, chunk = 0;
     uint64_t unit = 0;
     bool full = false;
     for (int b = 0; b < max_blocks && known > 0 && !full;) {
-      const int to = std::min(max_blocks, b + (chunk < 4 ? kTileFirstChunk : kTileChunk));
+      const int to = std::min(max_blocks, b + (chunk < 4 ? std::min(1 << chunk, 4) : kTileChunk));
       for (; b < to; ++b) {
         a.act = act[which];
         a.n_act = n_act + which;
@@ -348,16 +355,18 @@ int run_tile_group(Engine* e, const JobSet& js, const PlanGroup& grp, const wfa:
       const int slot = chunk & 1;
       if (!hip_ok(wfa::launch_tile_compact(act[which], n_act + which, a.done, a.irr, b * T, act[which ^ 1],
                                            n_act + (which ^ 1), lost, const_cast<int*>(h_n) + slot, st), "tile compact") ||
-          !hip_ok(hipEventRecord(t.ev[3 + slot], st), "tile event"))
+          !hip_ok(hipEventRecord(t.ev[slot], st), "tile event"))
         return WF_STATUS_OOM;
       which ^= 1;
       if (chunk > 0) {
-        if (!hip_ok(hipEventSynchronize(t.ev[3 + (slot ^ 1)]), "tiles")) return WF_STATUS_OOM;
+        if (!hip_ok(hipEventSynchronize(t.ev[slot ^ 1]), "tiles")) return WF_STATUS_OOM;
         known = h_n[slot ^ 1];
+        jobs_lost = h_n[(slot ^ 1) + wfa::kTileHostLost];
       }
       ++chunk;
     }
-    if (!full) {
+    // (known == 0: the last list that was seen was empty, so every job was done or lost by then)
+    if (!full && (known > 0 || jobs_lost > 0)) {
       const int rc = run_steps(e, js, shape, g, a, slots, n, info, records, rec_units, &unit);
       if (rc != WF_STATUS_OK) return rc;
     }
@@ -385,7 +394,7 @@ int run_tile_group(Engine* e, const JobSet& js, const PlanGroup& grp, const wfa:
     f.dsteps_total = &c->dsteps;
     f.retry_count = &c->retry;
     if (!hip_ok(wfa::launch_tile_finish(shape, f, st), "tile finish")) return WF_STATUS_OOM;
-    (void)hipEventRecord(t.ev[1], st);
+    (void)hipEventRecord(grp.ev[1], st);
     if (records) {
       wfa::TileTraceArgs ta{};
       ta.jobs = a.jobs;
@@ -404,17 +413,23 @@ int run_tile_group(Engine* e, const JobSet& js, const PlanGroup& grp, const wfa:
       ta.lmax_words = lw;
       if (!hip_ok(wfa::launch_tile_backtrace(shape, ta, n, st), "tile backtrace")) return WF_STATUS_OOM;
     }
-    (void)hipEventRecord(t.ev[2], st);
-    if (!hip_ok(hipStreamSynchronize(st), "tiles")) return WF_STATUS_OOM;
-    float fms = 0, bms = 0;
-    (void)hipEventElapsedTime(&fms, t.ev[0], t.ev[1]);
-    (void)hipEventElapsedTime(&bms, t.ev[1], t.ev[2]);
-    tot->forward_ms += fms;
-    tot->backtrace_ms += bms;
+    (void)hipEventRecord(grp.ev[2], st);
     if (some) ++tot->launches;  // a further pass (the caller counts one)
-    some = true;
+    some = timed = true;
     first += taken;
+    if (first < n_all) {
+      // the buffers and events are used again
+      if (!hip_ok(hipStreamSynchronize(st), "tiles")) return WF_STATUS_OOM;
+      float fms = 0, bms = 0;
+      (void)hipEventElapsedTime(&fms, grp.ev[0], grp.ev[1]);
+      (void)hipEventElapsedTime(&bms, grp.ev[1], grp.ev[2]);
+      tot->forward_ms += fms;
+      tot->backtrace_ms += bms;
+      timed = false;
+    }
   }
+  if (!timed)
+    for (auto& ev : grp.ev) (void)hipEventRecord(ev, st);  // (no time, for the caller to read)
   return WF_STATUS_OK;
 }
 
