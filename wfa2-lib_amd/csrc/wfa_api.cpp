@@ -920,6 +920,20 @@ bool wide_follows(const Engine* e, const JobSet& js, const PlanGroup& g, const P
          (pen.ncomp == 5 || js.ef.on);
 }
 
+// As many waves as the arena has room for: each holds a pair's records, or
+// what is left of its chunk, to the end of the launch.  With more of them than
+// that none may get through a pair, and a round without a pair done falls to
+// one workgroup: 20,000 pairs of 1,000 bp at 6% errors in an arena of 64 MB
+// take 52 ms, without the bound 3.2 s, and under gap-affine-2p, where
+// two launches share the arena, they failed.  (An arena of the run's estimate
+// does not come near it.)
+void bound_grid(const Engine* e, const PlanGroup& g, int records, bool shared, LaunchShape* shape) {
+  if (!records || g.family != wfa::kWave) return;
+  const size_t chunks = (wfa::wave_record_units(g.wave, g.wcap) + wfa::kChunkUnits - 1) / wfa::kChunkUnits;
+  const size_t most = e->rec.cap / 16 / wfa::kChunkUnits / chunks / (shared ? 2 : 1);
+  shape->grid = (int)std::max<size_t>(1, std::min<size_t>((size_t)shape->grid, most));
+}
+
 // Enqueues forward + backtrace of one group on the aligner's stream; with
 // fresh, the run counters were just cleared and need no reset of their own.
 int enqueue_group(wavefront_aligner_t* wf, Engine* e, const JobSet& js, PlanGroup& grp, const Penalties& pen,
@@ -928,7 +942,7 @@ int enqueue_group(wavefront_aligner_t* wf, Engine* e, const JobSet& js, PlanGrou
   if (n == 0) return WF_STATUS_OK;
   hipStream_t st = e->stream;
   set_wave(js, grp, pen, records);
-  const LaunchShape shape = shape_of(e, grp, js.bits, pen, js.heur.cut());
+  LaunchShape shape = shape_of(e, grp, js.bits, pen, js.heur.cut());
   bool ident = true;
   for (int i = 0; i < n && ident; ++i) ident = grp.ids[i] == i;
   if (!ident && !grp.ids_on_device) {
@@ -956,6 +970,7 @@ int enqueue_group(wavefront_aligner_t* wf, Engine* e, const JobSet& js, PlanGrou
   ForwardArgs wide;
   LaunchShape wide_shape;
   grp.wave_wide = wide_follows(e, js, grp, pen) && e->over.ensure((size_t)n * 4);
+  bound_grid(e, grp, records, grp.wave_wide, &shape);
   if (grp.wave_wide) {
     PlanGroup g8;
     g8.family = wfa::kWave;
@@ -967,6 +982,7 @@ int enqueue_group(wavefront_aligner_t* wf, Engine* e, const JobSet& js, PlanGrou
     g8.ids.swap(grp.ids);
     wide_shape = shape_of(e, g8, js.bits, pen, 0);
     g8.ids.swap(grp.ids);
+    bound_grid(e, g8, records, true, &wide_shape);
     fa.over_ids = e->over.as<int>();
     fa.over_n = &counters_of(e)->over;
     wide = fa;
@@ -1145,7 +1161,8 @@ int run_jobs(wavefront_aligner_t* wf, Engine* e, const JobSet& js, std::vector<P
         g.est_rec_bytes = w;
         set_wave(js, g, pen, records);
         if (g.family != wfa::kTile)  // and the record chunk of every workgroup
-          g.est_rec_bytes += (double)shape_of(e, g, js.bits, pen, js.heur.cut()).grid * wfa::kChunkUnits * 16;
+          g.est_rec_bytes += (double)shape_of(e, g, js.bits, pen, js.heur.cut()).grid * wfa::kChunkUnits * 16 *
+                             (g.family == wfa::kWave && g.wcap == 8 ? 2 : 1);
         if (wide_follows(e, js, g, pen)) g.est_rec_bytes += kWideRecordBytes;
       }
       want += g.est_rec_bytes;

@@ -14,6 +14,8 @@ bool wave_phases(int shape, int pbf, int tbf, int nmax, WaveArgs* w);
 // the place of its records (segments of steps).
 bool wave_cuts(int shape, const HeurArgs& heur);
 void wave_cut_phases(WaveArgs* w);
+// Most record units (16 bytes) that a wave reserves for one pair.
+uint32_t wave_record_units(const WaveArgs& w, int nmax);
 size_t wave_lds_bytes(int lds_words);
 int wave_max_blocks_per_cu(int shape, int nmax, bool rec, int bits, bool ef, bool cut, size_t lds);
 // nmax: most diagonals per lane (4 or 8; 1 with a cut-off).

@@ -93,23 +93,27 @@ struct WaveRing {
 };
 
 struct WaveChunk {  // record chunk of this wave (16-byte units)
-  uint32_t cur, end;
+  uint32_t cur, end, begin;
+  // The records written since `from` (a copy of this) go back: those of a pair
+  // that does not finish here.  Where the pair took a new chunk, all of that.
+  __device__ __forceinline__ void give_back(const WaveChunk& from) { cur = begin == from.begin ? from.cur : begin; }
 };
 
-// Room for `units` of records in the wave's chunk, or a new chunk.
+// Room for `units` of records in the wave's chunk, or a new chunk (twice as
+// large where the last phase alone may fill one: what is left of a chunk when
+// the next phase does not fit is lost).
+template <int NMAX>
 __device__ __forceinline__ bool reserve_records(WaveChunk& ch, uint32_t units) {
   if (ch.cur + units <= ch.end) return true;
   KernArgs A = args_now();
-  const uint32_t want = units > kChunkUnits ? units : kChunkUnits;
+  constexpr uint32_t chunk = NMAX == 8 ? 2 * kChunkUnits : kChunkUnits;
+  const uint32_t want = units > chunk ? units : chunk;
   unsigned long long b = 0;
   if ((threadIdx.x & 63) == 0) b = atomicAdd(A->rec_top, (unsigned long long)want);
   const unsigned blo = (unsigned)lane_of((int)(unsigned)(b & 0xFFFFFFFFull), 0);
   const unsigned bhi = (unsigned)lane_of((int)(unsigned)(b >> 32), 0);
-  if (bhi != 0 || (unsigned long long)blo + want > A->rec_units) {
-    ch.cur = ch.end = 0;
-    return false;
-  }
-  ch.cur = blo;
+  if (bhi != 0 || (unsigned long long)blo + want > A->rec_units) return false;
+  ch.cur = ch.begin = blo;
   ch.end = blo + want;
   return true;
 }
@@ -130,7 +134,7 @@ __device__ __forceinline__ void wave_phase(WavePair& p, WaveChunk& ch, WaveRows<
   uint32_t* rec = nullptr;
   if constexpr (REC) {
     const uint32_t units = (uint32_t)((last - first + G - 1) / G * (N > 4 ? N / 4 : 1)) * 16u;
-    if (!reserve_records(ch, units)) {
+    if (!reserve_records<NMAX>(ch, units)) {
       p.status = kDevArenaFull;
       return;
     }
@@ -393,7 +397,7 @@ __global__ void __launch_bounds__(64, S::NC == 5 ? (NMAX == 8 ? 2 : 3) : (NMAX =
   __shared__ __align__(16) int16_t ring_lds[S::NC == 5 ? WaveRing<NMAX>::kBytes / 2 : 8];
   const WaveRing<NMAX> ring{ring_lds};
   const int lane = threadIdx.x;
-  WaveChunk ch{0, 0};
+  WaveChunk ch{0, 0, 0};
   unsigned long long wg_dsteps = 0;
   bool q_first = true;
   for (;;) {
@@ -440,9 +444,10 @@ __global__ void __launch_bounds__(64, S::NC == 5 ? (NMAX == 8 ? 2 : 3) : (NMAX =
     }
     wave_sync();
     uint32_t header = kNoBlock;
+    const WaveChunk before = ch;
     if constexpr (REC) {
       // the pair's header: the units of its phases' records
-      if (reserve_records(ch, 1)) header = ch.cur++;
+      if (reserve_records<NMAX>(ch, 1)) header = ch.cur++;
       else p.status = kDevArenaFull;
     }
     // phases: rows of 1, 2, 4 (and 8) diagonals per lane in turn
@@ -476,6 +481,7 @@ __global__ void __launch_bounds__(64, S::NC == 5 ? (NMAX == 8 ? 2 : 3) : (NMAX =
     if (p.status == 1) p.status = kDevRingOverflow;  // wider than the wave holds
     KernArgs B = args_now();
     const bool good = p.status == kDevCompleted;
+    if (REC && !good) ch.give_back(before);
     const int ds = good ? wave_table<typename S::Slots>.dsteps[p.i] + p.dev + (EF ? wave_table<typename S::Slots>.nonnull[p.i] * (B->pbf + B->tbf) : 0) : 0;
     if (lane == 0) {
       B->out_status[id] = p.status;
@@ -648,7 +654,7 @@ __device__ __forceinline__ int cut_pair(const WaveSeqs<2>& q, WaveChunk& ch, uin
       last = B->wave.last[seg];
       if constexpr (REC) {
         const uint32_t units = (uint32_t)((last - first) / G) * 16u;
-        if (!reserve_records(ch, units)) return kDevArenaFull;
+        if (!reserve_records<2>(ch, units)) return kDevArenaFull;
 #pragma unroll
         for (int x = 0; x < kWaveCutSegments; ++x) base[x] = x == seg ? ch.cur : base[x];
         rec = reinterpret_cast<uint32_t*>(B->rec_arena + ch.cur) + lane;
@@ -814,7 +820,7 @@ __global__ void __launch_bounds__(64, 7) wfa_wave_cut_kernel(ForwardArgs a) {
   uint32_t* seqP = reinterpret_cast<uint32_t*>(smem);
   uint32_t* seqT = seqP + a.wave.lds_words;
   const int lane = threadIdx.x;
-  WaveChunk ch{0, 0};
+  WaveChunk ch{0, 0, 0};
   unsigned long long wg_dsteps = 0;
   bool q_first = true;
   for (;;) {
@@ -831,16 +837,20 @@ __global__ void __launch_bounds__(64, 7) wfa_wave_cut_kernel(ForwardArgs a) {
     wave_sync();
     int status = kDevArenaFull, steps = 0, dsteps = 0, wide = 0;
     uint32_t header = kNoBlock, base[kWaveCutSegments] = {0, 0, 0};
-    if (!REC || reserve_records(ch, 1)) {
+    const WaveChunk before = ch;
+    if (!REC || reserve_records<2>(ch, 1)) {
       if constexpr (REC) header = ch.cur++;
+      const WaveChunk narrow = ch;
       status = cut_pair<S, 1, REC>(q, ch, base, steps, dsteps);
       if (status == kDevRingOverflow) {
         wide = 1;
+        if constexpr (REC) ch.give_back(narrow);
         status = cut_pair<S, 2, REC>(q, ch, base, steps, dsteps);
       }
     }
     KernArgs B = args_now();
     const bool good = status == kDevCompleted;
+    if (REC && !good) ch.give_back(before);
     if (lane == 0) {
       B->out_status[id] = status;
       B->out_score[id] = steps * B->pen.g;
@@ -946,6 +956,16 @@ void wave_cut_phases(WaveArgs* w) {
   w->last[1] = 176;
   w->last[2] = w->last[3] = kWaveSteps;
   static_assert(kWaveCutSegments == 3 && kWaveSteps % 4 == 0, "segments");
+}
+
+uint32_t wave_record_units(const WaveArgs& w, int nmax) {
+  if (w.cut) return 1 + (uint32_t)(w.last[kWaveCutSegments - 1] / 2) * 16u;  // two diagonals per lane
+  uint32_t units = 1;
+  for (int ph = 0, first = 0; ph < kWavePhases && (1 << ph) <= nmax; first = w.last[ph++]) {
+    const int n = 1 << ph, g = n < 4 ? 4 / n : 1;
+    units += (uint32_t)((w.last[ph] - first + g - 1) / g * (n > 4 ? n / 4 : 1)) * 16u;
+  }
+  return units;
 }
 
 int wave_max_blocks_per_cu(int shape, int nmax, bool rec, int bits, bool ef, bool cut, size_t lds) {
