@@ -1988,8 +1988,10 @@ namespace wfa_host {
 // swapped back afterwards.
 int device_batch_run_in(wavefront_aligner_t* wf, wfa_device_batch_t* b, char* scratch, size_t bytes) {
   constexpr size_t kRingShare = 64ull << 20;
-  constexpr size_t kMinArena = 32ull << 20;
   constexpr size_t kCounters = (sizeof(wfa::Counters) + 255) & ~(size_t)255;
+  // the counters' queues at the arena's cost: as many pairs per call as with
+  // one queue in 256 bytes (20,970,976 in 256 MB)
+  constexpr size_t kMinArena = (32ull << 20) + 256 - kCounters;
   if (!b) return WF_STATUS_OOM;
   presets_check(wf, b->plen.data(), b->tlen.data(), b->n);
   const int sup = check_supported(wf);
