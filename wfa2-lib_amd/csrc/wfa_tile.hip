@@ -702,7 +702,7 @@ __global__ void __launch_bounds__(256) tile_finish_kernel(TileFinishArgs a) {
 // of once per step.  The replay extends with all 64 lanes (1,024 symbols at a
 // time) from sequences in LDS.  Same two passes over the CIGAR slot as
 // wfa_backtrace_kernel.
-template <class S, bool LDS>
+template <class S>
 __global__ void __launch_bounds__(64) tile_backtrace_kernel(TileTraceArgs a) {
   constexpr int T = TileGeom<S>::T;
   extern __shared__ __align__(16) unsigned char smem[];
@@ -801,11 +801,9 @@ __global__ void __launch_bounds__(64) tile_backtrace_kernel(TileTraceArgs a) {
     const unsigned pbit = 2u * (unsigned)(ppos & 31), tbit = 2u * (unsigned)(tpos & 31);
     uint32_t* sP = reinterpret_cast<uint32_t*>(smem);
     uint32_t* sT = sP + 2 * a.lmax_words;
-    if constexpr (LDS) {
-      const int nwp = (((int)(ppos & 31) + plen) / 32 + 2) * 2, nwt = (((int)(tpos & 31) + tlen) / 32 + 2) * 2;
-      for (int x = lane; x < nwp; x += 64) sP[x] = P[x];
-      for (int x = lane; x < nwt; x += 64) sT[x] = Q[x];
-    }
+    const int nwp = (((int)(ppos & 31) + plen) / 32 + 2) * 2, nwt = (((int)(tpos & 31) + tlen) / 32 + 2) * 2;
+    for (int x = lane; x < nwp; x += 64) sP[x] = P[x];
+    for (int x = lane; x < nwt; x += 64) sT[x] = Q[x];
     __threadfence_block();  // the walk's operations, before other lanes read them
     wave_sync();
     int v = 0, h = 0, w = start;
@@ -813,7 +811,7 @@ __global__ void __launch_bounds__(64) tile_backtrace_kernel(TileTraceArgs a) {
       for (;;) {
         const int rem = min(plen - v, tlen - h);
         const int at = min(16 * lane, rem);
-        const WaveSeqs<2> q{LDS ? sP : P, LDS ? sT : Q, pbit, tbit, plen, tlen};
+        const WaveSeqs<2> q{sP, sT, pbit, tbit, plen, tlen};
         const int m1 = q.run(h + at, v + at, rem - at);
         const unsigned long long stop = __ballot(m1 < 16);
         const int f = stop ? (int)__builtin_ctzll(stop) : 0;
@@ -1143,8 +1141,8 @@ hipError_t launch_tile_finish(int shape, const TileFinishArgs& a, hipStream_t st
 
 hipError_t launch_tile_backtrace(int shape, const TileTraceArgs& a, int n, hipStream_t st) {
   const size_t lds = (size_t)2 * a.lmax_words * sizeof(uint64_t);
-  if (shape == 2) hipLaunchKernelGGL((tile_backtrace_kernel<Shape2p, true>), dim3(n), dim3(64), lds, st, a);
-  else hipLaunchKernelGGL((tile_backtrace_kernel<ShapeAffine, true>), dim3(n), dim3(64), lds, st, a);
+  if (shape == 2) hipLaunchKernelGGL((tile_backtrace_kernel<Shape2p>), dim3(n), dim3(64), lds, st, a);
+  else hipLaunchKernelGGL((tile_backtrace_kernel<ShapeAffine>), dim3(n), dim3(64), lds, st, a);
   return hipGetLastError();
 }
 
