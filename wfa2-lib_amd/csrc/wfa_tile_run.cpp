@@ -17,7 +17,8 @@ constexpr int kTileMaxJobs = 32768;  // grid y
 // Records a long pair is planned with: 1-20 kbp pairs of 1-15% error write
 // 0.25 L^2 bytes on average and up to 0.7 L^2.
 constexpr double kTileRecordShareOfL2 = 0.5;
-// Blocks between two looks at the number of jobs left: 1, 2, 4, 4, then 16.
+// Blocks between two looks at the number of jobs left: 1, 2, 4 at a time up to
+// some 32, then 16.
 constexpr int kTileChunk = 16;
 
 bool put(DevBuf& d, const void* from, size_t bytes, hipStream_t st) {
@@ -333,7 +334,7 @@ int run_tile_group(Engine* e, const JobSet& js, PlanGroup& grp, const wfa::Penal
     uint64_t unit = 0;
     bool full = false;
     for (int b = 0; b < max_blocks && known > 0 && !full;) {
-      const int to = std::min(max_blocks, b + (chunk < 4 ? std::min(1 << chunk, 4) : kTileChunk));
+      const int to = std::min(max_blocks, b + (b < 3 ? 1 + b : b < 2 * kTileChunk ? 4 : kTileChunk));
       for (; b < to; ++b) {
         a.act = act[which];
         a.n_act = n_act + which;
